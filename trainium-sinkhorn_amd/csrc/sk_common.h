@@ -114,6 +114,10 @@ __host__ __device__ inline int last_wg(int g, const Split& s) { return owner_of(
 //     [3] the scale of the second cloud that copy was made against, [4] the copy's unit t (a power of two),
 //     [5] L0, the integer offset of the cloud's log2 weights in the on-device loop (a float; written at loop
 //         init, 0 elsewhere),
+//     [6] an integer, 1 while the on-device loop has moved to a new eps and its next f update is still to make the
+//         copy's tiles (each workgroup its own rows, in registers; sk_lse_partial.hip), with [7] the new c and [8] the
+//         new t; [2] is 0 meanwhile, for every reader but the loop. The control of the iteration that made the tiles
+//         moves [7], [8] to [2], [4] (every workgroup of its launch has read the header by then),
 // then the tiles of the cloud's own pieces (s x), then (kF16x2 only) the tiles of its log2-unit copy: two fp16
 // pieces of t fl(c_b x) / s_2 per coordinate, which the first cloud of a pair carries so that its piece products
 // with the second cloud's own pieces sum to t c_b x.y, the half-step's score in log2 units times t (see
@@ -181,13 +185,15 @@ struct PartialArgs {
     int* group_counters;  // or null: per row group arrival counters (zero on entry, left zero); the partial
                           // kernel's last workgroup to finish a row group merges it (no merge kernel)
     int ngroups;
-    // ... and, in the last merge workgroup of a g update, the loop control (null: none), which also remakes the
-    // log2-unit copy of the first cloud (rebake, the packed first cloud; null: never) when eps changes; the f
-    // update's merge advances the state's iteration counters (tick; null: none).
+    // ... and, in the last merge workgroup of a g update, the loop control (null: none), which also marks the
+    // log2-unit copy of the first cloud (rebake) to be remade when eps changes; the f update's merge advances the
+    // state's iteration counters (tick; null: none).
     sk_state* tick;
     sk_state* state;
     LoopCfg cfg;
-    char* rebake;
+    char* rebake;       // the packed first cloud, in both updates (null: the loop runs without the copy)
+    float next_k2;      // the merge, set inside the kernel: half the next iteration's score scale when the g update
+                        // already knows it differs from this one's (an eps schedule), else 0
 };
 
 // Launch the partial kernel for kp = 16 * nc on P workgroups (nc <= 4: launch_partial_small, else

@@ -114,14 +114,8 @@ __device__ inline BakeParams bake_params(const void* first, const void* second, 
     return b;
 }
 
-// One 16-byte unit (8 coordinates of one tile row half, one K chunk) of the copy.
-__device__ inline void bake_unit(char* first, long long idx, int npad, int nc, const BakeParams& b) {
-    const f16x8* own = reinterpret_cast<const f16x8*>(first + kHeaderBytes);
-    f16x8* cp = reinterpret_cast<f16x8*>(first + kHeaderBytes) + (size_t)(npad / SK_TILE) * nc * 2 * 64;
-    const int lane = (int)(idx % 64);
-    const long long tc = idx / 64;                          // tile * nc + chunk
-    const f16x8 p0 = own[tc * 128 + lane], p1 = own[tc * 128 + 64 + lane];
-    f16x8 q0, q1;
+// Eight coordinates of the copy from the cloud's own pieces.
+__device__ __forceinline__ void bake_pieces(const f16x8& p0, const f16x8& p1, const BakeParams& b, f16x8& q0, f16x8& q1) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const float x = ((float)p0[e] + (float)p1[e]) * b.inv_s1;
@@ -130,6 +124,16 @@ __device__ inline void bake_unit(char* first, long long idx, int npad, int nc, c
         q0[e] = a0;
         q1[e] = (_Float16)(w - (float)a0);
     }
+}
+
+// One 16-byte unit (8 coordinates of one tile row half, one K chunk) of the copy.
+__device__ inline void bake_unit(char* first, long long idx, int npad, int nc, const BakeParams& b) {
+    const f16x8* own = reinterpret_cast<const f16x8*>(first + kHeaderBytes);
+    f16x8* cp = reinterpret_cast<f16x8*>(first + kHeaderBytes) + (size_t)(npad / SK_TILE) * nc * 2 * 64;
+    const int lane = (int)(idx % 64);
+    const long long tc = idx / 64;                          // tile * nc + chunk
+    f16x8 q0, q1;
+    bake_pieces(own[tc * 128 + lane], own[tc * 128 + 64 + lane], b, q0, q1);
     cp[tc * 128 + lane] = q0;
     cp[tc * 128 + 64 + lane] = q1;
 }
@@ -139,6 +143,21 @@ __device__ inline void bake_header(char* first, const void* second, const BakePa
     h[2] = b.valid ? b.c : 0.0f;
     h[3] = packed_scale(second);
     h[4] = b.valid ? b.t : 1.0f;
+    reinterpret_cast<int*>(first)[6] = 0;
+}
+
+// The log2-unit copy a half-step finds on the first cloud (header h1): its score scale (0: none), its second cloud's
+// scale and its unit, and whether its tiles are still to be made by the loop's f update (pending; only the on-device
+// loop, which says so with `loop`, looks at a copy in that state).
+struct CopyTag {
+    float c, s2, t;
+    int pending;
+};
+__device__ __forceinline__ CopyTag copy_tag(const float* h1, bool loop) {
+    const float c = h1[2], s2 = h1[3], t = h1[4], c7 = h1[7], t8 = h1[8];
+    const int w6 = reinterpret_cast<const int*>(h1)[6];
+    const bool p = loop && w6 != 0;
+    return {p ? c7 : c, s2, p ? t8 : t, p ? 1 : 0};
 }
 
 // The on-device loop's log2 weights. In log2 units a column term is R_j + log2(e) log w_j (R_j = (c / 2) gh_j,
@@ -202,7 +221,8 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
     const float sc0 = a.sc[0], sc1 = a.sc[1], sc2 = a.sc[2], sc3 = a.sc[3];   // valid in both modes
     const float* h1 = reinterpret_cast<const float*>(a.rows_role == 0 ? a.xr : a.yc);   // the first cloud
     const float* h2 = reinterpret_cast<const float*>(a.rows_role == 0 ? a.yc : a.xr);
-    const float cb = h1[2], cb_s2 = h1[3], s2 = h2[1], cb_t = h1[4];
+    const CopyTag tag = copy_tag(h1, a.rebake != nullptr);
+    const float cb = tag.c, cb_s2 = tag.s2, s2 = h2[1];
     const float L0 = loop_weight_offset(a.yc);                     // the column cloud's log2 weight offset (loop)
     const int ic = i < a.rows_pad ? i : a.rows_pad - 1;
     const float x2 = a.mode == kHalfStep ? a.xsq[ic] : 0.0f;
@@ -218,7 +238,7 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) v0[k] = p0 + k <= p1 ? ld<COH>(pp + (size_t)k * a.rows_pad) : make_float2(kEmpty, 0.0f);
     const int skip = *skip_p;
-    asm volatile("" ::"s"(sc0), "s"(sc1), "s"(sc2), "s"(sc3), "s"(cb), "s"(cb_s2), "s"(s2), "s"(cb_t), "s"(L0),
+    asm volatile("" ::"s"(sc0), "s"(sc1), "s"(sc2), "s"(sc3), "s"(cb), "s"(cb_s2), "s"(s2), "s"(L0),
                  "v"(x2), "v"(o), "v"(old), "v"(wi), "v"(ll), "v"(skip));
     if (skip != 0) return false;
     const float c_hs = sc0 * kLog2e;
@@ -274,12 +294,17 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
                 const double k2 = 0.5 * (double)c_hs;
                 const double R = kappa * (od * (double)kLog2eD - (Md + l2s)) + (kappa - 1.0) * (x2d * k2);
                 val = (float)(R / k2);
-                if (i < a.n_store) st<COH>(a.out2 + i, (float)(R + (double)ll));
+                // (a schedule's next eps is known here: its log2-unit potential comes from fh, as the control derives
+                // it for a new stage)
+                const double Rn = a.next_k2 != 0.0f ? (double)val * (double)a.next_k2 : R;
+                if (i < a.n_store) st<COH>(a.out2 + i, (float)(Rn + (double)ll));
             } else {
                 // eps lse = 2 M + eps ln(S) in accumulator units (log2-unit slots: M / c), with the caller's eps
                 // (float) as the reference's epilogue multiplies by it (src/trnopt/sinkhorn.py:119)
                 const double eps_lse = 2.0 * (l2 ? Md / (double)c_hs : Md) + (double)sc2 * kLn2D * l2s;
                 val = (float)(kappa * ((double)sc2 * od - eps_lse) + (kappa - 1.0) * x2d);
+                if (a.out2 != nullptr && a.next_k2 != 0.0f && i < a.n_store)
+                    st<COH>(a.out2 + i, (float)((double)val * (double)a.next_k2 + (double)ll));
             }
             if (a.meas != nullptr) {
                 if (i < a.n_real) dmax = fabsf(val - old);
@@ -387,13 +412,15 @@ __device__ inline void control_step(sk_state* st, const float2* meas, int nmeas,
 // The loop's state counters as a g update sees them on entry (before any workgroup can reach the control).
 struct LoopCounters {
     int it, stage, stage_it;
+    int pending;               // the copy was pending in this iteration (its f update has made the tiles)
 };
 __device__ inline LoopCounters loop_counters(const PartialArgs& a) {
-    LoopCounters k = {0, 0, 0};
+    LoopCounters k = {0, 0, 0, 0};
     if (a.state != nullptr) {
         k.it = a.state->it;
         k.stage = a.state->stage;
         k.stage_it = a.state->stage_it;
+        if (a.rebake != nullptr) k.pending = reinterpret_cast<const int*>(a.rebake)[6];
     }
     return k;
 }
@@ -401,7 +428,7 @@ __device__ inline LoopCounters loop_counters(const PartialArgs& a) {
 // After row group g is merged (all threads of the workgroup; the group's results are stored): the f update
 // counts the iteration (once, by group 0's merge); a g update whose counters call for the loop control runs it in
 // the last workgroup to arrive (counter: zero on entry, left zero), which on a new eps also derives the log2-unit
-// potentials again and remakes the first cloud's log2-unit copy for the next f update. COH as in merge_group:
+// potentials again and has the next f update remake the first cloud's log2-unit copy. COH as in merge_group:
 // the other groups' results were stored in this launch by other workgroups. NT: the workgroup's threads.
 template <bool COH, int NT>
 __device__ inline void loop_step(const PartialArgs& a, int g, const LoopCounters& lc, int* counter) {
@@ -412,7 +439,7 @@ __device__ inline void loop_step(const PartialArgs& a, int g, const LoopCounters
         }
         return;
     }
-    if (a.state == nullptr || !needs_control(lc.it, lc.stage, lc.stage_it, a.cfg)) return;
+    if (a.state == nullptr || !(lc.pending != 0 || needs_control(lc.it, lc.stage, lc.stage_it, a.cfg))) return;
     __shared__ int s_last;
     if constexpr (!COH) __threadfence();   // release: this group's outputs and meas[g]
     __syncthreads();                       // (COH: every wave's stores have completed)
@@ -426,7 +453,7 @@ __device__ inline void loop_step(const PartialArgs& a, int g, const LoopCounters
     __shared__ float s_sc0_ran;
     __shared__ int s_done;
     if (tid_x() == 0) s_sc0_ran = a.state->sc_x[0];
-    if (tid_x() < 64) control_step<COH>(a.state, a.meas, a.ngroups, a.cfg);
+    if (tid_x() < 64) control_step<COH>(a.state, a.meas, a.meas != nullptr ? a.ngroups : 0, a.cfg);
     if (tid_x() == 0) {
         st<COH>(counter, 0);
         s_done = a.state->done;
@@ -434,25 +461,49 @@ __device__ inline void loop_step(const PartialArgs& a, int g, const LoopCounters
     }
     if (a.rebake == nullptr) return;
     __syncthreads();
-    if (s_done != 0 || s_sc[0] == s_sc0_ran) return;     // same eps next: the copy and the log2 states stand
-    // A new eps (a schedule or a stage): the log2-unit potentials R = (c / 2) fh of both clouds again from the
-    // accumulator-unit ones (stored as R + Ll, loop_weight_offset), and the first cloud's log2-unit copy for the
-    // new score scale, so that the next f update already finds them. (This is the g update: rows y, columns x.)
-    const double k2 = 0.5 * (double)(s_sc[0] * kLog2e);
-    const int nx = a.s.nt * SK_TILE;
-    for (int i = tid_x(); i < a.rows_pad; i += NT)
-        a.out2[i] = (float)((double)ld<COH>(a.out + i) * k2 + (double)a.rows_l2lo[i]);
-    for (int i = tid_x(); i < nx; i += NT) a.u2[i] = (float)((double)a.u[i] * k2 + (double)a.cols_l2lo[i]);
-    const void* second = a.xr;
-    const BakeParams b = bake_params(a.rebake, second, s_sc);
-    const float* h = reinterpret_cast<const float*>(a.rebake);
-    if (b.valid ? h[2] == b.c && h[3] == packed_scale(second) : h[2] == 0.0f) return;
-    if (b.valid) {
-        const long long total = (long long)(nx / SK_TILE) * a.nc * 64;
-        for (long long idx = tid_x(); idx < total; idx += NT) bake_unit(a.rebake, idx, nx, a.nc, b);
+    float* h = reinterpret_cast<float*>(a.rebake);
+    if (tid_x() == 0 && lc.pending != 0) {                // this iteration's f update made the copy's tiles
+        h[2] = h[7];
+        h[4] = h[8];
+        reinterpret_cast<int*>(h)[6] = 0;
     }
-    __syncthreads();
-    if (tid_x() == 0) bake_header(a.rebake, second, b);
+    if (s_done != 0 || s_sc[0] == s_sc0_ran) return;     // same eps next: the copy and the log2 states stand
+    // A new eps (a schedule or a stage): the header hands the new copy to the next f update, which makes its tiles
+    // (made here, by this one workgroup, they took 165 us at 10,000 x 64, twice the iteration); x's log2-unit
+    // potential is that f update's own result. y's, R = (c / 2) gh, the merges have already written for a schedule
+    // (next_k2); for a new stage, which only this control knows of, it comes from gh here (stored as R + Ll,
+    // loop_weight_offset), eight loads in flight per thread. (This is the g update: rows y, columns x.)
+    if (a.next_k2 == 0.0f) {
+        const double k2 = 0.5 * (double)(s_sc[0] * kLog2e);
+        for (int i0 = tid_x(); i0 < a.rows_pad; i0 += 8 * NT) {
+            float v[8], l[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int i = i0 + k * NT < a.rows_pad ? i0 + k * NT : a.rows_pad - 1;
+                v[k] = ld<COH>(a.out + i);
+                l[k] = a.rows_l2lo[i];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (i0 + k * NT < a.rows_pad) a.out2[i0 + k * NT] = (float)((double)v[k] * k2 + (double)l[k]);
+        }
+    }
+    if (tid_x() == 0) {
+        const BakeParams b = bake_params(a.rebake, a.xr, s_sc);
+        h[2] = 0.0f;
+        h[3] = packed_scale(a.xr);
+        h[7] = b.c;
+        h[8] = b.t;
+        reinterpret_cast<int*>(h)[6] = b.valid ? 1 : 0;
+    }
+}
+
+// Half the score scale of the iteration after the one a g update belongs to, when an eps schedule (no stages) already
+// fixes it and it differs from this one's; 0 otherwise. (sc0: this iteration's 2 / eps.)
+__device__ inline float next_half_scale(const LoopCounters& lc, const LoopCfg& c, float sc0) {
+    if (c.n_stages > 0 || lc.it > c.n_sched || lc.it < 1 || lc.it >= c.max_iters) return 0.0f;
+    const float next = (float)(2.0 / eps_for(c, lc.it, 0));
+    return next == sc0 ? 0.0f : 0.5f * (next * kLog2e);
 }
 
 }  // namespace sk

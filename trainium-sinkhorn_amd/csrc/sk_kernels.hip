@@ -46,7 +46,7 @@
 // update the merges also produce per-group convergence partials, and at a check, a schedule step or the last
 // iteration the last group's merge runs the balanced / unbalanced checks at the reference's cadence, advances
 // the stage, sets `done`, and writes the next iteration's eps and {2/eps, 1/eps, eps, kappa} into the device
-// state (remaking x's log2-unit copy when eps changes). Every loop kernel returns immediately once `done` is
+// state (a new eps also marks x's log2-unit copy, which the next f update remakes). Every loop kernel returns immediately once `done` is
 // set, so the host may enqueue whole batches of iterations.
 
 #include <hip/hip_runtime.h>
@@ -105,6 +105,7 @@ __global__ void pack_header_kernel(unsigned* __restrict__ header) {
         header[3] = 0u;
         header[4] = __float_as_uint(1.0f);  // the copy's unit
         header[5] = 0u;                     // L0, the loop's log2 weight offset (the on-device loop writes it)
+        header[6] = 0u;                     // no copy pending (the on-device loop)
     }
 }
 
@@ -257,7 +258,11 @@ __global__ void fill_mask_kernel(float* __restrict__ mask, int m, int mpad) {
 __global__ __launch_bounds__(kRowsPerGroup) void merge_kernel(PartialArgs a) {
     const LoopCounters lc = loop_counters(a);
     // The loop's convergence partials are read only by a control that checks: skip them otherwise.
-    if (a.state != nullptr && !needs_control(lc.it, lc.stage, lc.stage_it, a.cfg)) a.meas = nullptr;
+    a.next_k2 = 0.0f;
+    if (a.state != nullptr) {
+        if (!needs_control(lc.it, lc.stage, lc.stage_it, a.cfg)) a.meas = nullptr;
+        else if (a.rebake != nullptr) a.next_k2 = next_half_scale(lc, a.cfg, a.sc[0]);
+    }
     if (!merge_group<false, kRowsPerGroup>(a, (int)blockIdx.x)) return;
     loop_step<false, kRowsPerGroup>(a, (int)blockIdx.x, lc, a.counters);
 }
@@ -421,7 +426,7 @@ struct Pass {
     sk_state* tick;   // the loop's state whose iteration counters the merge advances (f update), or null
     sk_state* state;  // loop control after the merge (g update of the loop), or null
     LoopCfg cfg;
-    char* rebake;   // with state: the packed first cloud, whose log2-unit copy the control remakes on a new eps
+    char* rebake;   // in the loop: the packed first cloud, whose log2-unit copy is remade on a new eps (null: no copy)
 };
 
 PartialArgs pass_args(const Pass& ps, const Plan& pl) {
@@ -459,6 +464,7 @@ PartialArgs pass_args(const Pass& ps, const Plan& pl) {
     a.state = ps.state;
     a.cfg = ps.cfg;
     a.rebake = ps.rebake;
+    a.next_k2 = 0.0f;
     return a;
 }
 
@@ -893,6 +899,7 @@ void loop_passes(const sk_loop_f32* L, const LoopLayout& lo, Pass& f, Pass& g) {
     f.cols_l2lo = lo.lyl;
     f.n_store = L->x.npad;
     f.tick = st;
+    f.rebake = log2_enabled() ? (char*)const_cast<void*>(L->x.pk) : nullptr;
     f.part = lo.part;
     f.group_counters = fused_merge(lo.pf) ? lo.counters + 1 : nullptr;
 
@@ -925,7 +932,7 @@ void loop_passes(const sk_loop_f32* L, const LoopLayout& lo, Pass& f, Pass& g) {
     g.counters = lo.counters;
     g.state = st;
     g.cfg = loop_cfg(L);
-    g.rebake = log2_enabled() ? (char*)const_cast<void*>(L->x.pk) : nullptr;
+    g.rebake = f.rebake;
     g.group_counters = fused_merge(lo.pg) ? lo.counters + 1 : nullptr;
 }
 

@@ -523,7 +523,7 @@ struct Streamed {
 
     __device__ __forceinline__ static void run(const PartialArgs& a, int rb0, int tb, int te, int slot, const float* cu,
                                                const float* cv, float alpha, float beta, float beta_lo, float cs,
-                                               float c, float inv_sigma, float* lds_col) {
+                                               float c, float inv_sigma, bool stale, float* lds_col) {
         const int tid = tid_x();
         const int lane = tid & 63;
         const int h = lane >> 5;
@@ -541,6 +541,31 @@ struct Streamed {
 #pragma unroll
                 for (int p = 0; p < kPieces; ++p)
                     xv[b][cc][p] = xt[(size_t)blk * TILE16 + (cc * kPieces + p) * 64 + lane];
+        }
+        // The first f update at a new eps (header word [6]): the copy's tiles are still those of the last one. The
+        // rows come from the cloud's own pieces and are scaled here, in every segment; the segment in slot 0 of its
+        // row group also writes them to the copy, which the g update then reads as columns. (Made by the one
+        // workgroup that ran the loop control, at its own store rate, they held every eps step of a 10,000 x 64 cloud
+        // up by 165 us; spread over this launch's prologues: 10k mixture solve with 29 scheduled eps 13.7 -> 9.6 ms.)
+        if constexpr (L2 && ROLE == 0 && CT == kF16x2) {
+            if (__builtin_expect(stale, 0)) {
+                const BakeParams bp = bake_params(a.xr, a.yc, a.sc);
+                T* own = const_cast<T*>(packed_tiles<T>(a.xr));
+                T* copy = const_cast<T*>(xt);
+#pragma unroll
+                for (int b = 0; b < RB; ++b) {
+                    const int blk = rb0 + b < a.nrb ? rb0 + b : a.nrb - 1;
+#pragma unroll
+                    for (int cc = 0; cc < NC; ++cc) {
+                        const size_t u = (size_t)blk * TILE16 + cc * kPieces * 64 + lane;
+                        bake_pieces(own[u], own[u + 64], bp, xv[b][cc][0], xv[b][cc][1]);
+                        if (slot == 0) {
+                            copy[u] = xv[b][cc][0];
+                            copy[u + 64] = xv[b][cc][1];
+                        }
+                    }
+                }
+            }
         }
         float M[RB], S[RB];
 #pragma unroll
@@ -804,7 +829,11 @@ __device__ inline void arrive(const PartialArgs& a, const PartialArgs* kp, int g
     // The loop's counters as this launch found them: the control runs only after every group is merged, this
     // one included, so nothing has changed them yet.
     const LoopCounters lc = loop_counters(m);
-    if (m.state != nullptr && !needs_control(lc.it, lc.stage, lc.stage_it, m.cfg)) m.meas = nullptr;   // no check
+    m.next_k2 = 0.0f;
+    if (m.state != nullptr) {
+        if (!needs_control(lc.it, lc.stage, lc.stage_it, m.cfg)) m.meas = nullptr;   // no check
+        else if (m.rebake != nullptr) m.next_k2 = next_half_scale(lc, m.cfg, m.sc[0]);
+    }
     if (merge_group<true, kBlockK>(m, g)) loop_step<true, kBlockK>(m, g, lc, m.counters);
     __syncthreads();   // the next segment's column staging reuses LDS the merge does not touch; keep waves together
 }
@@ -815,7 +844,8 @@ __device__ inline void arrive(const PartialArgs& a, const PartialArgs* kp, int g
 template <int NC, int ROLE, int CT, bool L2, bool KARG>
 __device__ __forceinline__ void segments(const PartialArgs& a, const PartialArgs* kp, int p, int wv, const float* cu,
                                          const float* cv, float alpha, float beta, float beta_lo, float cs, float c,
-                                         float inv_sigma, typename Contract<CT>::T* lds_y, float* lds_col) {
+                                         float inv_sigma, bool stale, typename Contract<CT>::T* lds_y,
+                                         float* lds_col) {
     // The segment bounds are 32-bit integer arithmetic (the divisions expand to vector code); their results are
     // the same in every lane, and readfirstlane hands them to the scalar unit, so the tile loop's counters and
     // operand addresses stay in scalar registers.
@@ -830,7 +860,7 @@ __device__ __forceinline__ void segments(const PartialArgs& a, const PartialArgs
         const int rb0 = (g * kWavesK + wv) * kRowBlocksK;
         if constexpr (streamed_form(NC, CT))
             Streamed<NC, ROLE, CT, L2>::run(a, rb0, tb, te, slot, cu, cv, alpha, beta, beta_lo, cs, c, inv_sigma,
-                                            lds_col);
+                                            stale, lds_col);
         else
             Staged<NC, ROLE, CT, L2>::run(a, rb0, tb, te, slot, cu, cv, alpha, beta, beta_lo, cs, c, inv_sigma, lds_y,
                                           lds_col);
@@ -855,7 +885,8 @@ __device__ __forceinline__ void partial_pass(const PartialArgs& a, const Partial
     const float* h1 = reinterpret_cast<const float*>(ROLE == 0 ? a.xr : a.yc);   // the first cloud's header
     const float sc0 = a.sc[0], sc2 = a.sc[2];                         // a.sc is valid in both modes
     const float sx = packed_scale(a.xr), sy = packed_scale(a.yc);   // 1 for kBF16x3
-    const float cb = h1[2], cb_s2 = h1[3], cb_t = h1[4];
+    const CopyTag tag = copy_tag(h1, a.rebake != nullptr);
+    const float cb = tag.c, cb_s2 = tag.s2, cb_t = tag.t;
     const int skip = *skip_p;
     // The argument fields the segments need, requested with the first batch of argument loads rather than
     // after the scalars have arrived.
@@ -863,8 +894,9 @@ __device__ __forceinline__ void partial_pass(const PartialArgs& a, const Partial
                  "s"(a.s.ftot), "s"(a.s.q), "s"(a.s.r), "s"(a.group_counters), "s"(a.s.dP.m), "s"(a.s.dP.k),
                  "s"(a.s.dspan.m), "s"(a.s.dspan.k), "s"(a.s.dnt.m), "s"(a.s.dnt.k), "s"(a.s.dftot.m),
                  "s"(a.s.dftot.k), "s"(a.u), "s"(a.v), "s"(a.u2), "s"(a.v2), "s"(a.part));
-    asm volatile("" ::"s"(sc0), "s"(sc2), "s"(sx), "s"(sy), "s"(cb), "s"(cb_s2), "s"(cb_t), "v"(skip));
+    asm volatile("" ::"s"(sc0), "s"(sc2), "s"(sx), "s"(sy), "s"(cb), "s"(cb_s2), "s"(cb_t), "s"(tag.pending), "v"(skip));
     if (skip != 0) return;
+    const bool stale = ROLE == 0 && tag.pending != 0;    // this f update makes the copy's tiles
     constexpr bool kStream = streamed_form(NC, CT);
     constexpr int kLdsY = kStream ? 1 : 3 * NC * Contract<CT>::pieces * 64;     // staged: three tile buffers
     constexpr int kLdsCol = kStream ? col_floats(CT == kF16x2) : 4 * 32;        // staged: four column buffers
@@ -900,17 +932,17 @@ __device__ __forceinline__ void partial_pass(const PartialArgs& a, const Partial
             // The usual unit t = 1 gets its own inlined copy: with c = 1 a constant, each exponential's argument is
             // the two-operand a - m (v_sub_f32) instead of the three-operand fma.
             if (a.u2 != nullptr && cb_t == 1.0f)
-                segments<NC, ROLE, CT, true, KARG>(a, kp, p, wv, a.u2, a.v2, 1.0f, 1.0f, 0.0f, 1.0f, 1.0f, 1.0f, lds_y, lds_col);
+                segments<NC, ROLE, CT, true, KARG>(a, kp, p, wv, a.u2, a.v2, 1.0f, 1.0f, 0.0f, 1.0f, 1.0f, 1.0f, stale, lds_y, lds_col);
             else if (a.u2 != nullptr)
-                segments<NC, ROLE, CT, true, KARG>(a, kp, p, wv, a.u2, a.v2, 1.0f, 1.0f, 0.0f, cb_t, it, it, lds_y, lds_col);
+                segments<NC, ROLE, CT, true, KARG>(a, kp, p, wv, a.u2, a.v2, 1.0f, 1.0f, 0.0f, cb_t, it, it, stale, lds_y, lds_col);
             else
-                segments<NC, ROLE, CT, true, KARG>(a, kp, p, wv, a.u, a.v, alpha, beta, 0.0f, c * cb_t, it, it, lds_y, lds_col);
+                segments<NC, ROLE, CT, true, KARG>(a, kp, p, wv, a.u, a.v, alpha, beta, 0.0f, c * cb_t, it, it, false, lds_y, lds_col);
             return;
         }
     }
     const float sigma = sx * sy, inv_sigma = (1.0f / sx) * (1.0f / sy);
-    segments<NC, ROLE, CT, false, KARG>(a, kp, p, wv, a.u, a.v, alpha, beta, 0.0f, sigma, c * inv_sigma, inv_sigma, lds_y,
-                                  lds_col);
+    segments<NC, ROLE, CT, false, KARG>(a, kp, p, wv, a.u, a.v, alpha, beta, 0.0f, sigma, c * inv_sigma, inv_sigma, false,
+                                         lds_y, lds_col);
 }
 
 template <int NC, int ROLE, int CT>
