@@ -245,10 +245,11 @@ int sk_loop_run_batch_f32(const void* ws, size_t ws_bytes, int count, const int*
  * over the materialised n x m float64 matrix:
  *     median over i < n, j < m of max((|xc_i|^2 + |yc_j|^2) - 2 xc_i . yc_j, 0)   (float64),
  * np.median's definition (mean of the two middle values when n m is even). xc (n, d), yc (m, d): row-major
- * float64 device arrays, already centred; out: one device double. Six radix-select passes over the cost
- * keys: the first three recompute every cost, the third keeping the keys that can still hold the answer
- * (up to 2^22 of them, 8 bytes each, in ws) for the last three. ws (sk_cost_median_workspace_bytes) also
- * holds zero-padded copies of xc and yc. n m < 2^32, d <= SK_MEDIAN_D_MAX; ws 256-byte aligned.
+ * float64 device arrays, already centred; out: one device double. Two passes over approximate costs (fp16 matrix
+ * cores) bracket the middle ranks and collect the pairs that can hold the answer (up to 2^22 of them, 12 bytes each, in
+ * ws), whose float64 costs are then selected by radix; with more of them (massive ties), six radix-select passes over
+ * every float64 cost. ws (sk_cost_median_workspace_bytes) also holds zero-padded copies and fp16 tiles of xc and yc.
+ * n m < 2^32, d <= SK_MEDIAN_D_MAX; ws 256-byte aligned.
  */
 #define SK_MEDIAN_D_MAX 128
 size_t sk_cost_median_workspace_bytes(int n, int m, int d);

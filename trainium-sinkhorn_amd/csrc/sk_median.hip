@@ -7,16 +7,22 @@
 //
 // (np.median's definition: the middle element for odd N, the mean of the two middle ones for even N.)
 //
-// Radix select on the fused cost stream: non-negative doubles order like their bit patterns, so the k-th
-// smallest cost is found digit by digit from the top (11, 11, 11, 11, 11, 9 bits). A pass recomputes every
-// C_ij tile by tile (256 rows x 32 columns per step: one row per thread, the dot products in registers, the
-// column coordinates from zero-padded copies through the scalar cache), keeps the pairs whose high bits equal
-// the prefix found so far, and histograms their next digit in LDS; a one-workgroup scan then picks the digit
-// holding rank k and narrows the prefix. The two ranks k0 and k1 share one histogram while their prefixes
-// agree. The third pass also collects the keys that still match a rank's prefix (a small fraction: a 22-bit
-// prefix) into the workspace, and the last three passes read only those; when there are more than the
-// workspace holds (massive ties), they recompute every cost instead. Every launch goes on the caller's stream
-// with no host round trip.
+// The float64 costs are only needed near the answer. Two passes over approximate costs A_ij, |A_ij - C_ij| <= E,
+// find out where that is: the dot products come from the fp16 matrix cores (two fp16 pieces per scaled
+// coordinate, three products, as in sk_lse_partial.hip), the rest in float32. An order statistic moves by at most
+// E when every element does, so C_(k) lies within E of A_(k), and every pair whose cost can be C_(k0) or C_(k1)
+// has A within [A_(k0) - 2 E, A_(k1) + 2 E]:
+//   1. histogram of all A (16,384 bins of relative width 2^-10) -> the bins of ranks k0 and k1, widened by 2 E;
+//   2. the pairs below that bracket counted, the pairs inside collected (0.1-0.3 % of them);
+//   3. the float64 costs of the collected pairs, and their order statistics k0 - below and k1 - below by a radix
+//      select (non-negative doubles order like their bit patterns), 11 bits at a time.
+// When the bracket holds more pairs than the workspace (massive ties), six radix-select passes over every float64
+// cost take over (select_pass_kernel). Every launch goes on the caller's stream with no host round trip.
+//
+// From the norms to the answer, all launches back to back: 7,355 x 8,962 d 30 192 us (the histogram pass 37 of them,
+// the collecting pass 50); 10,000 x 10,000 d 64 457 us; 7,000 x 7,000 d 128 276 us; 300 x 257 d 30 96 us. With three
+// radix passes over every float64 cost (254 to 187 us each at 7,355 x 8,962, where their fma floor is 54) it was 704,
+// 1,633, 1,529 and 121 us.
 
 #include <hip/hip_runtime.h>
 
@@ -28,46 +34,81 @@
 
 namespace {
 
+using sk::f16x8;
 using sk::fail;
 using sk::hip_fail;
 
 constexpr int kBins = 2048;                 // 11-bit digits
 constexpr int kRowsPerBlock = 256;          // one row per thread
 constexpr int kColTile = 32;                // column points per LDS tile
-constexpr int kTargetBlocks = 1024;         // workgroups a pass aims for (4 per CU): columns per workgroup follow
+constexpr int kTargetBlocks = 1024;         // blocks a full pass aims for: columns per block follow
 constexpr int kChunk = 8;                   // coordinates per register chunk of the row
 constexpr int kPasses = 6;
-constexpr int kCompactPass = 2;             // this pass also collects the keys matching its prefix ...
-constexpr unsigned long long kCandMax = 1ull << 22;   // ... up to this many; later passes read only those
+constexpr unsigned long long kCandMax = 1ull << 22;   // collected pairs, at most
 constexpr int kShift[kPasses] = {53, 42, 31, 20, 9, 0};
 constexpr int kWidth[kPasses] = {11, 11, 11, 11, 11, 9};
 
 struct SelectState {
     unsigned long long prefix[2];   // bits of the answer known so far (above the current digit)
-    unsigned long long k[2];        // rank still to find among the pairs that match the prefix
+    unsigned long long k[2];        // rank still to find among the keys that match the prefix
     int same;                       // 1 while both ranks have the same prefix (one histogram serves both)
-    int pad;
+    int arrived;                    // workgroups of the current launch that have added their counts
 };
 
-__global__ void norms_kernel(const double* __restrict__ p, int n, int d, double* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double* r = p + (size_t)i * d;
-    double s = 0.0;
-    for (int k = 0; k < d; ++k) s = fma(r[k], r[k], s);
-    out[i] = s;
-}
+// What the launches of one call hand on (device memory, the start of the workspace).
+struct MedianState {
+    SelectState cand;               // the select over the collected pairs
+    SelectState full;               // the select over every pair (only with `fallback`)
+    unsigned long long below;       // pairs below the bracket
+    unsigned long long count;       // pairs inside it
+    unsigned long long base;        // key of the bracket's lower end less E: subtracted from the collected keys
+    int bits;                       // bits of the largest difference to base
+    int fallback;                   // 1: the bracket held more pairs than the workspace, or not the ranks
+    int arrived;
+    float lo, hi;                   // the bracket, in scaled units
+    double scale;                   // power of two: (max |x| + max |y|) scale in [8, 16)
+    double err;                     // E in scaled units
+};
 
-__global__ void select_init_kernel(SelectState* st, unsigned* __restrict__ hist, unsigned long long* count,
-                                   unsigned long long N) {
-    for (int b = threadIdx.x; b < 2 * kBins; b += blockDim.x) hist[b] = 0u;
-    if (threadIdx.x == 0) {
-        *count = 0ull;
-        st->prefix[0] = st->prefix[1] = 0ull;
-        st->k[0] = (N - 1ull) / 2ull;
-        st->k[1] = N / 2ull;
-        st->same = 1;
+// |p|^2 of every point of both clouds (fma in ascending coordinate order) and each workgroup's maximum of them. One
+// point per thread of the workgroup's 32, its rows first copied to LDS with coalesced loads. The first workgroup also
+// writes the initial state and clears the histograms.
+constexpr int kNormRows = 32;
+__global__ __launch_bounds__(256) void norms_kernel(const double* __restrict__ x, int n, const double* __restrict__ y, int m,
+                                                    int d, double* __restrict__ xx, double* __restrict__ yy,
+                                                    double* __restrict__ block_max, int xblocks, MedianState* st,
+                                                    unsigned* __restrict__ hist) {
+    extern __shared__ double rows[];           // kNormRows x (d | 1): an odd row length, so that rows spread over banks
+    const bool is_x = (int)blockIdx.x < xblocks;
+    const double* p = is_x ? x : y;
+    const int np = is_x ? n : m, i0 = (is_x ? (int)blockIdx.x : (int)blockIdx.x - xblocks) * kNormRows;
+    const int nr = np - i0 < kNormRows ? np - i0 : kNormRows, ld = d | 1;
+    if (blockIdx.x == 0) {
+        for (int b = threadIdx.x; b < 2 * kBins; b += blockDim.x) hist[b] = 0u;
+        if (threadIdx.x == 0) {
+            const unsigned long long N = (unsigned long long)n * (unsigned long long)m;
+            SelectState s = {};
+            s.k[0] = (N - 1ull) / 2ull;
+            s.k[1] = N / 2ull;
+            s.same = 1;
+            *st = MedianState{};
+            st->cand = s;
+            st->full = s;
+        }
     }
+    for (int e = threadIdx.x; e < nr * d; e += blockDim.x) {
+        const int r = e / d;
+        rows[r * ld + (e - r * d)] = p[(size_t)i0 * d + e];
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;             // the first wave
+    double s = 0.0;
+    if ((int)threadIdx.x < nr) {
+        for (int k = 0; k < d; ++k) s = fma(rows[threadIdx.x * ld + k], rows[threadIdx.x * ld + k], s);
+        (is_x ? xx : yy)[i0 + threadIdx.x] = s;
+    }
+    for (int o = 32; o > 0; o >>= 1) s = fmax(s, __shfl_xor(s, o));
+    if (threadIdx.x == 0) block_max[blockIdx.x] = s;
 }
 
 __device__ __forceinline__ unsigned long long cost_key(double c) {
@@ -76,52 +117,425 @@ __device__ __forceinline__ unsigned long long cost_key(double c) {
     return b & 0x7fffffffffffffffull;
 }
 
-// Row-major copy of p (n x d) with rows of dp coordinates (zeros after d) and zero rows up to n_pad.
-__global__ void pad_kernel(const double* __restrict__ p, int n, int d, int n_pad, int dp, double* __restrict__ out) {
-    const long long total = (long long)n_pad * dp;
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (long long)gridDim.x * blockDim.x) {
-        const long long i = e / dp;
-        const int k = (int)(e - i * dp);
-        out[e] = i < n && k < d ? p[i * d + k] : 0.0;
+// The pairs' approximate costs A = |x|^2 + |y|^2 - 2 x . y, in units scaled so that (max |x| + max |y|)^2 lies in
+// [64, 256). Histogram bins are the float's top bits: 1,024 per octave over the 16 octaves below 256.
+constexpr int kHistBits = 14, kHistBins = 1 << kHistBits, kHistShift = 13;
+constexpr unsigned kHistBase = (0x43800000u >> kHistShift) - (unsigned)kHistBins;    // 256 = 2^8 is past the last bin
+// E over (max |x| + max |y|)^2 =: R^2. Two fp16 pieces leave a coordinate v within max(2^-23 |v|, 2^-25) and the product
+// x1 y1 out: 2^-22 |x||y| + sqrt(d) 2^-25 (|x| + |y|) in all, below 2^-23 R^2 (R >= 8, d <= 128, |x||y| <= R^2 / 4);
+// 3 d products summed in float32 err by at most 3 d 2^-24 |x||y| <= 2^-17.4 R^2; the cost's own float32 steps by 2^-22 R^2.
+// Twice the dot product's error is below 2^-16 R^2.
+constexpr double kCostErr = 0x1p-16;
+
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ double max_of(const double* __restrict__ v, int n) {
+    double mx = 0.0;
+    for (int e = (int)(threadIdx.x & 63); e < n; e += 64) mx = fmax(mx, v[e]);
+    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    return mx;
+}
+
+// Both clouds laid out for the passes: a float64 copy with rows of dp coordinates (zeros after d; the columns' also to
+// whole tiles), the fp16 pieces of the scaled coordinates in the order of the matrix cores (as sk_pack_cloud_f32's
+// tiles: one thread per tile, K chunk and lane), the scaled |p|^2 in float32 (padding points: 1e38, above every cost).
+__global__ __launch_bounds__(256) void layout_kernel(const double* __restrict__ x, int n, const double* __restrict__ y, int m,
+                                                     int d, int dp, int mp, int nc, const double* __restrict__ xx,
+                                                     const double* __restrict__ yy, const double* __restrict__ block_max,
+                                                     int xblocks, int yblocks, double* __restrict__ xp,
+                                                     double* __restrict__ yp, f16x8* __restrict__ xt,
+                                                     f16x8* __restrict__ yt, float* __restrict__ xf, float* __restrict__ yf,
+                                                     int ntx, int nty, MedianState* st) {
+    const double R = sqrt(max_of(block_max, xblocks)) + sqrt(max_of(block_max + xblocks, yblocks));
+    int e = 0;
+    if (R > 0.0 && R < 1.0e300) frexp(R, &e);            // R in [2^(e - 1), 2^e)
+    const double s = R > 0.0 && R < 1.0e300 ? ldexp(1.0, 4 - e) : 1.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->scale = s;
+        st->err = kCostErr * (R * s) * (R * s);
+    }
+    // one wave per row, and one per tile: no index divisions
+    const int lane = (int)(threadIdx.x & 63), wave = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    const int waves = (int)(gridDim.x * (blockDim.x >> 6));
+    for (int side = 0; side < 2; ++side) {
+        const double* p = side == 0 ? x : y;
+        const int np = side == 0 ? n : m, rows = side == 0 ? n : mp, nt = side == 0 ? ntx : nty;
+        double* out = side == 0 ? xp : yp;
+        f16x8* tiles = side == 0 ? xt : yt;
+        float* f = side == 0 ? xf : yf;
+        for (int i = wave; i < rows; i += waves)
+            for (int k = lane; k < dp; k += 64) out[(size_t)i * dp + k] = i < np && k < d ? p[(size_t)i * d + k] : 0.0;
+        for (int T = wave; T < nt; T += waves) {
+            const int row = T * SK_TILE + (lane & 31);
+            for (int cc = 0; cc < nc; ++cc) {
+                f16x8 p0, p1;
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    const int k = 16 * cc + 8 * (lane >> 5) + c;
+                    const float v = row < np && k < d ? (float)(p[(size_t)row * d + k] * s) : 0.0f;
+                    const _Float16 a = (_Float16)v;
+                    p0[c] = a;
+                    p1[c] = (_Float16)(v - (float)a);
+                }
+                f16x8* o = tiles + ((size_t)T * nc + cc) * 128 + lane;
+                o[0] = p0;
+                o[64] = p1;
+            }
+            if (lane < 32) f[row] = row < np ? (float)((side == 0 ? xx : yy)[row] * s * s) : 1.0e38f;
+        }
     }
 }
 
-// How a full pass relates to the candidate keys.
-enum PassMode { kPlain = 0, kCollect = 1, kIfOverflow = 2 };
+// One pass over the approximate costs, one workgroup of 8 waves per CU. The (64 rows -- 32 above kp 64 --, column tile) units, row by row, are
+// cut into equal contiguous ranges, one per wave: the rows' pieces stay in registers, the column tiles come straight
+// from L2 one tile ahead. COLLECT false: every cost into the workgroup's histogram in LDS, stored whole to its slab (summed by
+// bracket_kernel; no global atomics). COLLECT true: the pairs below the bracket counted, those inside staged in LDS and
+// copied out with one reservation per workgroup. Bound by the LDS atomics of the histogram (one per cost).
+constexpr int kApproxWaves = 8, kApproxThreads = 64 * kApproxWaves;
+constexpr int row_blocks_of(int nc) { return nc <= 4 ? 2 : 1; }   // 32-row blocks per wave (256 registers a lane)
+constexpr unsigned kStage = 8192;               // collected pairs a workgroup stages in LDS
 
-constexpr unsigned kStage = 2048;           // collected keys a workgroup stages in LDS before one reservation
-
-__device__ __forceinline__ unsigned long long readlane64(unsigned long long v, int lane) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), lane);
-    return ((unsigned long long)hi << 32) | lo;
+template <int NC, bool COLLECT>
+__global__ __launch_bounds__(kApproxThreads) void approx_pass_kernel(
+    const f16x8* __restrict__ xt, const f16x8* __restrict__ yt, const float* __restrict__ xf, const float* __restrict__ yf,
+    int n, int m, int ntx, int nty, MedianState* st, unsigned* __restrict__ slabs, unsigned* __restrict__ pairs,
+    unsigned long long cap) {
+    __shared__ unsigned bins[COLLECT ? kStage : kHistBins];
+    __shared__ unsigned fill;
+    __shared__ unsigned long long base;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+    if (tid == 0) fill = 0u;
+    if constexpr (!COLLECT)
+        for (int b = tid; b < kHistBins; b += kApproxThreads) bins[b] = 0u;
+    __syncthreads();
+    float lo = 0.0f;
+    unsigned lo_bits = 0u, span = 0u;
+    if constexpr (COLLECT) {
+        lo = st->lo;
+        lo_bits = __float_as_uint(lo);
+        span = __float_as_uint(st->hi) - lo_bits;
+    }
+    constexpr int RB = row_blocks_of(NC);
+    const int rbs = (ntx + RB - 1) / RB;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned long long below = 0;
+    const unsigned long long units = (unsigned long long)rbs * (unsigned)nty, waves = (unsigned long long)gridDim.x * kApproxWaves;
+    const unsigned long long w = (unsigned long long)blockIdx.x * kApproxWaves + wave;
+    const unsigned u1 = (unsigned)(units * (w + 1) / waves);
+    for (unsigned u = (unsigned)(units * w / waves); u < u1;) {
+        const int rb = (int)(u / (unsigned)nty), t0 = (int)(u - (unsigned)rb * (unsigned)nty);
+        const int t1 = u1 - u < (unsigned)(nty - t0) ? t0 + (int)(u1 - u) : nty;
+        u += (unsigned)(t1 - t0);
+        f16x8 xv[RB][NC][2];
+        float xr[RB];
+        int row[RB];
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            const int blk = RB * rb + b < ntx ? RB * rb + b : ntx - 1;
+            const bool twice = RB * rb + b >= ntx;           // a missing block repeats the last one: kept out by its |x|^2
+            row[b] = blk * SK_TILE + (lane & 31);
+            xr[b] = twice ? 1.0e38f : xf[row[b]];
+#pragma unroll
+            for (int c = 0; c < 2 * NC; ++c) xv[b][c / 2][c % 2] = xt[(size_t)blk * (NC * 128) + c * 64 + lane];
+        }
+        f16x8 ya[NC][2], yb[NC][2];
+        sk::f32x4 qa[4], qb[4];
+        auto load = [&](int t, f16x8 (&yv)[NC][2], sk::f32x4 (&q)[4]) {
+            const int tc = t < t1 ? t : t1 - 1;
+#pragma unroll
+            for (int c = 0; c < 2 * NC; ++c) yv[c / 2][c % 2] = yt[(size_t)tc * (NC * 128) + c * 64 + lane];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = *reinterpret_cast<const sk::f32x4*>(yf + tc * SK_TILE + 8 * k + 4 * h);
+        };
+        unsigned cnt = 0;
+        auto tile = [&](int t, const f16x8 (&yv)[NC][2], const sk::f32x4 (&q)[4]) {
+#pragma unroll
+            for (int b = 0; b < RB; ++b) {
+                sk::f32x16 acc = {};
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(yv[c][0], xv[b][c][0], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(yv[c][1], xv[b][c][0], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(yv[c][0], xv[b][c][1], acc, 0, 0, 0);
+                }
+                unsigned in = 0;                     // COLLECT: the lane's costs inside the bracket
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float a = fmaxf(fmaf(acc[r], -2.0f, q[r / 4][r % 4]) + xr[b], 0.0f);
+                    if constexpr (!COLLECT) {
+                        const unsigned v = __float_as_uint(a) >> kHistShift;
+                        const unsigned c = v < kHistBase ? kHistBase : v;
+                        atomicAdd(&bins[(c < kHistBase + kHistBins ? c : kHistBase + kHistBins - 1) - kHistBase], 1u);
+                    } else {
+                        cnt += a < lo ? 1u : 0u;
+                        // non-negative floats order like their bits: lo <= a <= hi in one comparison
+                        in |= __float_as_uint(a) - lo_bits <= span ? 1u << r : 0u;
+                    }
+                }
+                if constexpr (COLLECT) {
+                    if (in != 0u) {
+                        // (padding points cost 1e38, above every bracket)
+                        unsigned p = atomicAdd(&fill, (unsigned)__popc(in));
+                        do {
+                            const int r = __ffs((int)in) - 1;
+                            in &= in - 1u;
+                            const unsigned col = (unsigned)(t * SK_TILE + 8 * (r >> 2) + 4 * h + (r & 3));
+                            const unsigned idx = (unsigned)row[b] * (unsigned)m + col;
+                            if (p < kStage) {
+                                bins[p] = idx;
+                            } else {
+                                const unsigned long long g = atomicAdd(&st->count, 1ull);
+                                if (g < cap) pairs[g] = idx;
+                            }
+                            ++p;
+                        } while (in != 0u);
+                    }
+                }
+            }
+        };
+        load(t0, ya, qa);
+        for (int t = t0; t < t1; t += 2) {
+            load(t + 1, yb, qb);
+            tile(t, ya, qa);
+            if (t + 1 >= t1) break;
+            load(t + 2, ya, qa);
+            tile(t + 1, yb, qb);
+        }
+        below += cnt;
+    }
+    if constexpr (!COLLECT) {
+        __syncthreads();
+        for (int b = tid; b < kHistBins; b += kApproxThreads) slabs[(size_t)blockIdx.x * kHistBins + b] = bins[b];
+    } else {
+        for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o);
+        if (lane == 0 && below != 0) atomicAdd(&st->below, below);
+        __syncthreads();
+        const unsigned nf = fill < kStage ? fill : kStage;
+        if (tid == 0 && nf != 0u) base = atomicAdd(&st->count, (unsigned long long)nf);
+        __syncthreads();
+        for (unsigned e = tid; e < nf; e += kApproxThreads)
+            if (base + e < cap) pairs[base + e] = bins[e];
+    }
 }
 
-// Collect the wave's lanes with `take`: into the workgroup's LDS stage while it has room (reservations are
-// contiguous from 0, so the filled part is [0, *fill)), else straight into cand with a reservation of the
-// wave's own. Keys past cap are counted, not stored, so that *count > cap tells the later passes to
-// recompute instead.
-__device__ __forceinline__ void collect(bool take, unsigned long long key, unsigned long long* stage,
-                                        unsigned* reserved, unsigned* fill, unsigned long long* cand,
-                                        unsigned long long* count, unsigned long long cap) {
-    const unsigned long long bal = __ballot(take);
-    if (bal == 0ull) return;
-    const int lane = (int)(threadIdx.x & 63);
-    const int leader = __ffsll((long long)bal) - 1;
-    const unsigned cnt = (unsigned)__popcll(bal);
-    const unsigned below = (unsigned)__popcll(bal & ((1ull << lane) - 1ull));
-    unsigned sb = 0u;
-    if (lane == leader) sb = atomicAdd(reserved, cnt);
-    sb = (unsigned)__builtin_amdgcn_readlane((int)sb, leader);
-    if (sb + cnt <= kStage) {
-        if (take) stage[sb + below] = key;
-        if (lane == leader) atomicMax(fill, sb + cnt);
-        return;
+// Hand-over within a launch without fences (as the loop's merges, sk_lse_partial.hip): data goes through device-scope
+// atomics only, every wave waits for its own to complete, and the workgroup's arrival is counted after a barrier. A
+// device-scope fence instead writes back and invalidates the XCD's L2, 5 us a launch here. True in the last workgroup.
+__device__ inline bool last_to_arrive(int* counter, int blocks) {
+    __shared__ int last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == blocks - 1 ? 1 : 0;
+    __syncthreads();
+    return last != 0;
+}
+
+// The slabs summed (64 bins per workgroup, a quarter of the slabs per wave), and by the last workgroup to finish the bins
+// of the two ranks: the bracket.
+constexpr int kSumBlocks = kHistBins / 64;
+static_assert(kSumBlocks == 256, "one workgroup sum per thread of the last workgroup");
+__global__ __launch_bounds__(256) void bracket_kernel(const unsigned* __restrict__ slabs, int nslabs, MedianState* st,
+                                                      unsigned long long* __restrict__ total) {
+    __shared__ unsigned long long part[256];
+    __shared__ int pick[2];
+    const int tid = threadIdx.x, bin = (int)blockIdx.x * 64 + (tid & 63);
+    unsigned long long s = 0;
+    for (int k = tid >> 6; k < nslabs; k += 4 * 16) {
+        unsigned v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = k + 4 * e < nslabs ? slabs[(size_t)(k + 4 * e) * kHistBins + bin] : 0u;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s += v[e];
     }
-    unsigned long long base = 0ull;
-    if (lane == leader) base = atomicAdd(count, (unsigned long long)cnt);
-    const unsigned long long idx = readlane64(base, leader) + below;
-    if (take && idx < cap) cand[idx] = key;
+    part[tid] = s;
+    __syncthreads();
+    if (tid < 64) {
+        const unsigned long long t = part[tid] + part[tid + 64] + part[tid + 128] + part[tid + 192];
+        __hip_atomic_store(total + bin, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned long long sum = t;
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        if (tid == 0) __hip_atomic_store(total + kHistBins + blockIdx.x, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!last_to_arrive(&st->arrived, kSumBlocks)) return;
+    // the workgroups' sums scanned, one per thread: the workgroup whose bins hold a rank; then that one's 64 bins by a wave
+    __shared__ unsigned long long before[2];
+    const unsigned long long mine = __hip_atomic_load(total + kHistBins + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    part[tid] = mine;
+    if (tid < 2) {
+        pick[tid] = 0;
+        before[tid] = 0;
+    }
+    __syncthreads();
+    for (int off = 1; off < 256; off <<= 1) {
+        const unsigned long long v = tid >= off ? part[tid - off] : 0ull;
+        __syncthreads();
+        part[tid] += v;
+        __syncthreads();
+    }
+    for (int r = 0; r < 2; ++r) {
+        const unsigned long long rank = st->full.k[r], b = part[tid] - mine;
+        if (rank >= b && rank < b + mine) {
+            pick[r] = tid;
+            before[r] = b;
+        }
+    }
+    __syncthreads();
+    if (tid < 128) {
+        const int r = tid >> 6, lane = tid & 63, first = pick[r] * 64;
+        unsigned long long c = __hip_atomic_load(total + first + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long v = __shfl_up(c, o);
+            if (lane >= o) c += v;
+        }
+        const unsigned long long hit = __ballot(st->full.k[r] < before[r] + c);
+        if (lane == 0) pick[r] = first + (hit != 0ull ? __ffsll((long long)hit) - 1 : 63);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        const double err = st->err, s2 = st->scale * st->scale;
+        const double l = pick[0] == 0 ? 0.0 : (double)__uint_as_float((kHistBase + (unsigned)pick[0]) << kHistShift);
+        const double u = pick[1] == kHistBins - 1 ? 1.0e30
+                                                  : (double)__uint_as_float((kHistBase + (unsigned)pick[1] + 1u) << kHistShift);
+        // one float step outwards on top of 2 E; then E more for the float64 costs of the pairs inside
+        const double lb = l - 2.0 * err, ub = u + 2.0 * err;
+        st->lo = lb > 0.0 ? (float)(lb * (1.0 - 0x1p-22)) : 0.0f;
+        st->hi = (float)(ub * (1.0 + 0x1p-22));
+        const double c0 = (lb - 2.0 * err) / s2, c1 = (ub + 2.0 * err) / s2;
+        const unsigned long long k0 = c0 > 0.0 ? (unsigned long long)__double_as_longlong(c0) : 0ull;
+        const unsigned long long k1 = (unsigned long long)__double_as_longlong(c1 < 1.7e308 ? c1 : 1.7e308);
+        st->base = k0;
+        st->bits = k1 > k0 ? 64 - __clzll((long long)(k1 - k0)) : 1;
+    }
+}
+
+// The float64 keys of the collected pairs, less the bracket's base; a key outside the bracket's bits (a cost further
+// from its approximation than E, which no finite input gives) sends the call to the full passes, as do too many pairs
+// and ranks that are not inside.
+__global__ __launch_bounds__(256) void exact_kernel(const unsigned* __restrict__ pairs, const double* __restrict__ xp,
+                                                    const double* __restrict__ yp, const double* __restrict__ xx,
+                                                    const double* __restrict__ yy, int m, int dp, MedianState* st,
+                                                    unsigned long long* __restrict__ keys, unsigned long long cap) {
+    const unsigned long long count = st->count, below = st->below, base = st->base;
+    const unsigned long long k0 = st->full.k[0], k1 = st->full.k[1];
+    const bool ok = count <= cap && k0 >= below && k1 - below < count;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (ok) {
+            st->cand.k[0] = k0 - below;
+            st->cand.k[1] = k1 - below;
+        } else {
+            st->fallback = 1;
+        }
+    }
+    if (!ok) return;
+    const int bits = st->bits;
+    for (unsigned long long e = (unsigned long long)blockIdx.x * 256 + threadIdx.x; e < count; e += (unsigned long long)gridDim.x * 256) {
+        const unsigned idx = pairs[e];
+        const unsigned i = idx / (unsigned)m, j = idx - i * (unsigned)m;
+        const double2* xr = reinterpret_cast<const double2*>(xp + (size_t)i * dp);
+        const double2* yr = reinterpret_cast<const double2*>(yp + (size_t)j * dp);
+        double acc = 0.0;
+        for (int k = 0; k < dp / 2; k += 4) {
+            double2 a[4], b[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                a[q] = xr[k + q];
+                b[q] = yr[k + q];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc = fma(a[q].y, b[q].y, fma(a[q].x, b[q].x, acc));
+        }
+        const unsigned long long key = cost_key((xx[i] + yy[j]) - 2.0 * acc);
+        const unsigned long long v = key - base;
+        if (key < base || (bits < 64 && (v >> bits) != 0ull)) st->fallback = 1;
+        keys[e] = v;
+    }
+}
+
+// Pick, for each rank, the digit whose bin holds it; narrow the prefix and the rank; clear the histograms. By the last
+// workgroup (256 threads, eight bins each) of the launch that filled them.
+__device__ inline void select_digit(SelectState* st, unsigned* hist, int shift, int width) {
+    __shared__ unsigned long long part[256];
+    __shared__ int pick[2];
+    __shared__ unsigned long long below[2];
+    const int tid = threadIdx.x;
+    const int bins = 1 << width, per = (bins + 255) / 256;
+    const int same = st->same;
+    for (int s = 0; s < 2; ++s) {
+        const unsigned* hs = hist + (same ? 0 : s) * kBins;
+        unsigned c[kBins / 256];
+        unsigned long long mine = 0;
+        for (int b = 0; b < per; ++b) {
+            c[b] = tid * per + b < bins ? __hip_atomic_load(hs + tid * per + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+            mine += c[b];
+        }
+        part[tid] = mine;
+        if (tid == 0) {
+            pick[s] = 0;
+            below[s] = 0ull;
+        }
+        __syncthreads();
+        for (int off = 1; off < 256; off <<= 1) {
+            const unsigned long long v = tid >= off ? part[tid - off] : 0ull;
+            __syncthreads();
+            part[tid] += v;
+            __syncthreads();
+        }
+        const unsigned long long k = st->k[s];
+        unsigned long long before = part[tid] - mine;
+        if (k >= before && k < before + mine) {
+            int b = 0;
+            while (k >= before + c[b]) before += c[b++];
+            pick[s] = tid * per + b;
+            below[s] = before;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        for (int s = 0; s < 2; ++s) {
+            st->prefix[s] |= (unsigned long long)pick[s] << shift;
+            st->k[s] -= below[s];
+        }
+        st->same = (same && pick[0] == pick[1]) ? 1 : 0;
+        st->arrived = 0;
+    }
+    for (int b = tid; b < 2 * kBins; b += 256) hist[b] = 0u;
+}
+
+// A workgroup's digit counts into the launch's, and the digit picked by the last workgroup to add its own (true there).
+__device__ inline bool add_counts(SelectState* st, const unsigned (&h)[2][kBins], unsigned* hist, int shift, int width, int blocks) {
+    for (int b = threadIdx.x; b < 2 * kBins; b += 256) {
+        const unsigned v = (&h[0][0])[b];
+        if (v != 0u) atomicAdd(&hist[b], v);
+    }
+    if (!last_to_arrive(&st->arrived, blocks)) return false;
+    select_digit(st, hist, shift, width);
+    return true;
+}
+
+// One digit of the select over the collected keys; digit q holds bits [bits - 11 (q + 1), bits - 11 q).
+__global__ __launch_bounds__(256) void select_cand_kernel(const unsigned long long* __restrict__ keys, MedianState* st,
+                                                          unsigned* __restrict__ hist, int q) {
+    __shared__ unsigned h[2][kBins];
+    const int top = st->bits - 11 * q;
+    if (st->fallback != 0 || top <= 0) return;
+    const int shift = top > 11 ? top - 11 : 0, width = top > 11 ? 11 : top;
+    const unsigned long long c = st->count;
+    const int tid = threadIdx.x;
+    const int same = st->cand.same;
+    const unsigned long long high = top >= 64 ? 0ull : ~((1ull << top) - 1ull);
+    const unsigned long long p0 = st->cand.prefix[0] & high, p1 = st->cand.prefix[1] & high;
+    const unsigned dmask = (1u << width) - 1u;
+    for (int b = tid; b < 2 * kBins; b += 256) (&h[0][0])[b] = 0u;
+    __syncthreads();
+    for (unsigned long long e = (unsigned long long)blockIdx.x * 256 + tid; e < c; e += (unsigned long long)gridDim.x * 256) {
+        const unsigned long long key = keys[e];
+        const unsigned digit = (unsigned)(key >> shift) & dmask;
+        if ((key & high) == p0) atomicAdd(&h[0][digit], 1u);
+        if (!same && (key & high) == p1) atomicAdd(&h[1][digit], 1u);
+    }
+    __syncthreads();
+    add_counts(&st->cand, h, hist, shift, width, (int)gridDim.x);
 }
 
 // One digit pass over the workgroup's block of 256 rows x `cols` columns, on the zero-padded copies (rows of
@@ -134,19 +548,21 @@ __device__ __forceinline__ void collect(bool take, unsigned long long key, unsig
 // this keeps them on scalar loads whatever else the kernel stores.
 typedef __attribute__((address_space(4))) const double ConstDouble;
 
-template <int MODE>
 __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
     const double* __restrict__ xp, const double* __restrict__ yp, const double* __restrict__ xx,
-    const double* __restrict__ yy, int n, int m, int dp, int cols, const SelectState* __restrict__ st,
-    unsigned* __restrict__ hist, int shift, int width, unsigned long long* __restrict__ cand,
-    unsigned long long* __restrict__ count, unsigned long long cap) {
+    const double* __restrict__ yy, int n, int m, int dp, int cols, MedianState* ms, unsigned* __restrict__ hist, int shift,
+    int width, double* __restrict__ out) {
     __shared__ unsigned h[2][kBins];
-    __shared__ unsigned long long stage[MODE == kCollect ? kStage : 1];
-    __shared__ unsigned reserved, fill;
-    __shared__ unsigned long long stage_base;
-    if (MODE == kIfOverflow && *count <= cap) return;     // the candidate pass below does this digit
     const int tid = threadIdx.x;
-    if (tid == 0) reserved = fill = 0u;
+    SelectState* st = &ms->full;
+    if (ms->fallback == 0) {                              // the collected pairs hold the answer
+        if (shift == 0 && blockIdx.x == 0 && tid == 0) {
+            const double a = __longlong_as_double((long long)(ms->cand.prefix[0] + ms->base));
+            const double b = __longlong_as_double((long long)(ms->cand.prefix[1] + ms->base));
+            *out = (a + b) * 0.5;
+        }
+        return;
+    }
     const int same = st->same;
     const unsigned long long high = shift + width >= 64 ? 0ull : ~((1ull << (shift + width)) - 1ull);
     const unsigned long long p0 = st->prefix[0] & high, p1 = st->prefix[1] & high;
@@ -154,146 +570,54 @@ __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
     for (int b = tid; b < 2 * kBins; b += kRowsPerBlock) (&h[0][0])[b] = 0u;
     __syncthreads();
 
-    const int i = blockIdx.x * kRowsPerBlock + tid;
-    const bool row_ok = i < n;
-    const double xi2 = row_ok ? xx[i] : 0.0;
-    const double* xr = xp + (size_t)(row_ok ? i : 0) * dp;
-    const int j_begin = blockIdx.y * cols;
-    const long long j_lim = (long long)j_begin + cols;
-    const int j_end = j_lim < m ? (int)j_lim : m;
+    const int rbs = (n + kRowsPerBlock - 1) / kRowsPerBlock, cbs = (m + cols - 1) / cols;
+    for (int blk = blockIdx.x; blk < rbs * cbs; blk += gridDim.x) {
+        const int i = blk % rbs * kRowsPerBlock + tid;
+        const bool row_ok = i < n;
+        const double xi2 = row_ok ? xx[i] : 0.0;
+        const double* xr = xp + (size_t)(row_ok ? i : 0) * dp;
+        const int j_begin = blk / rbs * cols;
+        const long long j_lim = (long long)j_begin + cols;
+        const int j_end = j_lim < m ? (int)j_lim : m;
 
-    for (int j0 = j_begin; j0 < j_end; j0 += kColTile) {
-        const int nj = j_end - j0 < kColTile ? j_end - j0 : kColTile;
-        const ConstDouble* yt = (const ConstDouble*)(yp + (size_t)j0 * dp);
-        double acc[kColTile];
+        for (int j0 = j_begin; j0 < j_end; j0 += kColTile) {
+            const int nj = j_end - j0 < kColTile ? j_end - j0 : kColTile;
+            const ConstDouble* yt = (const ConstDouble*)(yp + (size_t)j0 * dp);
+            double acc[kColTile];
 #pragma unroll
-        for (int jj = 0; jj < kColTile; ++jj) acc[jj] = 0.0;
-        for (int k0 = 0; k0 < dp; k0 += kChunk) {
-            double xv[kChunk];
+            for (int jj = 0; jj < kColTile; ++jj) acc[jj] = 0.0;
+            for (int k0 = 0; k0 < dp; k0 += kChunk) {
+                double xv[kChunk];
 #pragma unroll
-            for (int e = 0; e < kChunk; ++e) xv[e] = xr[k0 + e];
+                for (int e = 0; e < kChunk; ++e) xv[e] = xr[k0 + e];
+#pragma unroll
+                for (int jj = 0; jj < kColTile; ++jj) {
+                    const ConstDouble* yr = yt + (size_t)jj * dp + k0;
+                    double a = acc[jj];
+#pragma unroll
+                    for (int e = 0; e < kChunk; ++e) a = fma(xv[e], yr[e], a);
+                    acc[jj] = a;
+                }
+            }
 #pragma unroll
             for (int jj = 0; jj < kColTile; ++jj) {
-                const ConstDouble* yr = yt + (size_t)jj * dp + k0;
-                double a = acc[jj];
-#pragma unroll
-                for (int e = 0; e < kChunk; ++e) a = fma(xv[e], yr[e], a);
-                acc[jj] = a;
-            }
-        }
-#pragma unroll
-        for (int jj = 0; jj < kColTile; ++jj) {
-            const bool ok = row_ok && jj < nj;
-            const double c = (xi2 + (jj < nj ? yy[j0 + jj] : 0.0)) - 2.0 * acc[jj];
-            const unsigned long long key = cost_key(c);
-            const unsigned digit = (unsigned)(key >> shift) & dmask;
-            const bool m0 = ok && (key & high) == p0;
-            const bool m1 = ok && !same && (key & high) == p1;
-            if (m0) atomicAdd(&h[0][digit], 1u);
-            if (m1) atomicAdd(&h[1][digit], 1u);
-            if (MODE == kCollect) collect(m0 || m1, key, stage, &reserved, &fill, cand, count, cap);
-        }
-    }
-    __syncthreads();
-    for (int b = tid; b < 2 * kBins; b += kRowsPerBlock) {
-        const unsigned v = (&h[0][0])[b];
-        if (v != 0u) atomicAdd(&hist[b], v);
-    }
-    if (MODE == kCollect) {
-        const unsigned nf = fill;                        // the same for every thread (after the barrier)
-        if (nf != 0u) {
-            if (tid == 0) stage_base = atomicAdd(count, (unsigned long long)nf);
-            __syncthreads();
-            for (unsigned e = tid; e < nf; e += kRowsPerBlock) {
-                const unsigned long long idx = stage_base + e;
-                if (idx < cap) cand[idx] = stage[e];
+                const bool ok = row_ok && jj < nj;
+                const double c = (xi2 + (jj < nj ? yy[j0 + jj] : 0.0)) - 2.0 * acc[jj];
+                const unsigned long long key = cost_key(c);
+                const unsigned digit = (unsigned)(key >> shift) & dmask;
+                const bool m0 = ok && (key & high) == p0;
+                const bool m1 = ok && !same && (key & high) == p1;
+                if (m0) atomicAdd(&h[0][digit], 1u);
+                if (m1) atomicAdd(&h[1][digit], 1u);
             }
         }
     }
-}
-
-// One digit pass over the collected keys (every key that can still hold a rank), when they all fit.
-__global__ __launch_bounds__(kRowsPerBlock) void select_cand_kernel(
-    const unsigned long long* __restrict__ cand, const unsigned long long* __restrict__ count,
-    unsigned long long cap, const SelectState* __restrict__ st, unsigned* __restrict__ hist, int shift,
-    int width) {
-    __shared__ unsigned h[2][kBins];
-    const unsigned long long c = *count;
-    if (c > cap) return;                                  // overflowed: the full pass does this digit
-    const int tid = threadIdx.x;
-    const int same = st->same;
-    const unsigned long long high = shift + width >= 64 ? 0ull : ~((1ull << (shift + width)) - 1ull);
-    const unsigned long long p0 = st->prefix[0] & high, p1 = st->prefix[1] & high;
-    const unsigned dmask = (1u << width) - 1u;
-    for (int b = tid; b < 2 * kBins; b += kRowsPerBlock) (&h[0][0])[b] = 0u;
     __syncthreads();
-    for (unsigned long long e = (unsigned long long)blockIdx.x * kRowsPerBlock + tid; e < c;
-         e += (unsigned long long)gridDim.x * kRowsPerBlock) {
-        const unsigned long long key = cand[e];
-        const unsigned digit = (unsigned)(key >> shift) & dmask;
-        if ((key & high) == p0) atomicAdd(&h[0][digit], 1u);
-        if (!same && (key & high) == p1) atomicAdd(&h[1][digit], 1u);
+    if (add_counts(st, h, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0) {
+        const double a = __longlong_as_double((long long)st->prefix[0]);
+        const double b = __longlong_as_double((long long)st->prefix[1]);
+        *out = (a + b) * 0.5;
     }
-    __syncthreads();
-    for (int b = tid; b < 2 * kBins; b += kRowsPerBlock) {
-        const unsigned v = (&h[0][0])[b];
-        if (v != 0u) atomicAdd(&hist[b], v);
-    }
-}
-
-// Pick, for each rank, the digit whose bin holds it; narrow the prefix and the rank; clear the histograms.
-__global__ __launch_bounds__(1024) void select_scan_kernel(SelectState* st, unsigned* __restrict__ hist, int shift,
-                                                           int width) {
-    __shared__ unsigned long long part[1024];
-    __shared__ int pick[2];
-    __shared__ unsigned long long below[2];
-    const int tid = threadIdx.x;
-    const int bins = 1 << width;
-    const int same = st->same;
-    for (int s = 0; s < 2; ++s) {
-        const unsigned* hs = hist + (same ? 0 : s) * kBins;
-        // two bins per thread, then an inclusive scan over the threads (Hillis-Steele)
-        const unsigned long long c0 = 2 * tid < bins ? hs[2 * tid] : 0ull;
-        const unsigned long long c1 = 2 * tid + 1 < bins ? hs[2 * tid + 1] : 0ull;
-        part[tid] = c0 + c1;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            const unsigned long long v = tid >= off ? part[tid - off] : 0ull;
-            __syncthreads();
-            part[tid] += v;
-            __syncthreads();
-        }
-        const unsigned long long k = st->k[s];
-        const unsigned long long before = tid > 0 ? part[tid - 1] : 0ull;
-        if (tid == 0) {
-            pick[s] = 0;
-            below[s] = 0ull;
-        }
-        __syncthreads();
-        if (k >= before && k < before + c0) {
-            pick[s] = 2 * tid;
-            below[s] = before;
-        } else if (k >= before + c0 && k < before + c0 + c1) {
-            pick[s] = 2 * tid + 1;
-            below[s] = before + c0;
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        for (int s = 0; s < 2; ++s) {
-            st->prefix[s] |= (unsigned long long)pick[s] << shift;
-            st->k[s] -= below[s];
-        }
-        st->same = (same && pick[0] == pick[1]) ? 1 : 0;
-    }
-    for (int b = tid; b < 2 * kBins; b += 1024) hist[b] = 0u;
-}
-
-__global__ void select_finish_kernel(const SelectState* st, double* out) {
-    if (threadIdx.x != 0) return;
-    const double a = __longlong_as_double((long long)st->prefix[0]);
-    const double b = __longlong_as_double((long long)st->prefix[1]);
-    *out = (a + b) * 0.5;
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -304,16 +628,72 @@ unsigned long long cand_cap(int n, int m) {
     return N < kCandMax ? N : kCandMax;
 }
 
+// The workspace of one call.
+struct MedianLayout {
+    int dp, mp, nc, ntx, nty, xblocks, yblocks, blocks;
+    unsigned long long cap;
+    size_t state, hist, xx, yy, bmax, xp, yp, xt, yt, xf, yf, total, slabs, keys, bytes;
+};
+
+MedianLayout median_layout(int n, int m, int d) {
+    MedianLayout o;
+    o.dp = padded_dim(d);
+    o.mp = padded_cols(m);
+    o.nc = (d + 15) / 16;
+    o.ntx = (n + SK_TILE - 1) / SK_TILE;
+    o.nty = (m + SK_TILE - 1) / SK_TILE;
+    o.xblocks = (n + kNormRows - 1) / kNormRows;
+    o.yblocks = (m + kNormRows - 1) / kNormRows;
+    o.cap = cand_cap(n, m);
+    const int rbk = row_blocks_of(o.nc);
+    const long long units = (long long)((o.ntx + rbk - 1) / rbk) * o.nty;
+    o.blocks = (int)std::min<long long>(256, (units + kApproxWaves - 1) / kApproxWaves);
+    size_t p = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = p;
+        p += align256(bytes);
+        return at;
+    };
+    o.state = take(sizeof(MedianState));
+    o.hist = take(2 * kBins * sizeof(unsigned));
+    o.xx = take((size_t)n * 8);
+    o.yy = take((size_t)m * 8);
+    o.bmax = take((size_t)(o.xblocks + o.yblocks) * 8);
+    o.xp = take((size_t)n * o.dp * 8);
+    o.yp = take((size_t)o.mp * o.dp * 8);
+    o.xt = take((size_t)o.ntx * o.nc * 2048);
+    o.yt = take((size_t)o.nty * o.nc * 2048);
+    o.xf = take((size_t)o.ntx * SK_TILE * 4);
+    o.yf = take((size_t)o.nty * SK_TILE * 4);
+    o.total = take((size_t)(kHistBins + kSumBlocks) * 8);
+    // the histogram slabs, then (they are done with by then) the collected pairs
+    o.slabs = take(std::max((size_t)o.blocks * kHistBins * 4, (size_t)o.cap * 4));
+    o.keys = take((size_t)o.cap * 8);
+    o.bytes = p;
+    return o;
+}
+
+template <int NC>
+void launch_approx(const MedianLayout& o, char* w, int n, int m, hipStream_t s) {
+    const f16x8 *xt = (const f16x8*)(w + o.xt), *yt = (const f16x8*)(w + o.yt);
+    const float *xf = (const float*)(w + o.xf), *yf = (const float*)(w + o.yf);
+    MedianState* st = (MedianState*)(w + o.state);
+    unsigned* slabs = (unsigned*)(w + o.slabs);
+    hipLaunchKernelGGL((approx_pass_kernel<NC, false>), dim3(o.blocks), dim3(kApproxThreads), 0, s, xt, yt, xf, yf, n, m, o.ntx,
+                       o.nty, st, slabs, slabs, o.cap);
+    hipLaunchKernelGGL(bracket_kernel, dim3(kSumBlocks), dim3(256), 0, s, slabs, o.blocks, st,
+                       (unsigned long long*)(w + o.total));
+    hipLaunchKernelGGL((approx_pass_kernel<NC, true>), dim3(o.blocks), dim3(kApproxThreads), 0, s, xt, yt, xf, yf, n, m, o.ntx,
+                       o.nty, st, slabs, slabs, o.cap);
+}
+
 }  // namespace
 
 extern "C" {
 
 size_t sk_cost_median_workspace_bytes(int n, int m, int d) {
     if (n < 1 || m < 1 || d < 1 || d > SK_MEDIAN_D_MAX) return 0;
-    const size_t dp = (size_t)padded_dim(d);
-    return align256(sizeof(SelectState)) + align256(2 * kBins * sizeof(unsigned)) + align256((size_t)n * 8) +
-           align256((size_t)m * 8) + align256((size_t)n * dp * 8) + align256((size_t)padded_cols(m) * dp * 8) +
-           align256(sizeof(unsigned long long)) + align256((size_t)cand_cap(n, m) * 8);
+    return median_layout(n, m, d).bytes;
 }
 
 int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, double* out, void* ws,
@@ -327,53 +707,46 @@ int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, 
     if (ws_bytes < sk_cost_median_workspace_bytes(n, m, d))
         return fail(SK_E_WORKSPACE, "sk_cost_median_f64: workspace too small");
     if (((uintptr_t)ws & 255) != 0) return fail(SK_E_ARG, "sk_cost_median_f64: workspace must be 256-byte aligned");
-    char* p = (char*)ws;
-    SelectState* st = (SelectState*)p;
-    p += align256(sizeof(SelectState));
-    unsigned* hist = (unsigned*)p;
-    p += align256(2 * kBins * sizeof(unsigned));
-    double* xx = (double*)p;
-    p += align256((size_t)n * 8);
-    double* yy = (double*)p;
-    p += align256((size_t)m * 8);
-    const int dp = padded_dim(d), mp = padded_cols(m);
-    double* xp = (double*)p;
-    p += align256((size_t)n * dp * 8);
-    double* yp = (double*)p;
-    p += align256((size_t)mp * dp * 8);
-    unsigned long long* count = (unsigned long long*)p;
-    p += align256(sizeof(unsigned long long));
-    unsigned long long* cand = (unsigned long long*)p;
-    const unsigned long long cap = cand_cap(n, m);
+    const MedianLayout o = median_layout(n, m, d);
+    char* w = (char*)ws;
+    MedianState* st = (MedianState*)(w + o.state);
+    unsigned* hist = (unsigned*)(w + o.hist);
+    double *xx = (double*)(w + o.xx), *yy = (double*)(w + o.yy), *bmax = (double*)(w + o.bmax);
+    double *xp = (double*)(w + o.xp), *yp = (double*)(w + o.yp);
+    unsigned long long* keys = (unsigned long long*)(w + o.keys);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(norms_kernel, dim3((n + 255) / 256), dim3(256), 0, s, xc, n, d, xx);
-    hipLaunchKernelGGL(norms_kernel, dim3((m + 255) / 256), dim3(256), 0, s, yc, m, d, yy);
-    hipLaunchKernelGGL(pad_kernel, dim3(1024), dim3(256), 0, s, xc, n, d, n, dp, xp);
-    hipLaunchKernelGGL(pad_kernel, dim3(1024), dim3(256), 0, s, yc, m, d, mp, dp, yp);
-    hipLaunchKernelGGL(select_init_kernel, dim3(1), dim3(1024), 0, s, st, hist, count,
-                       (unsigned long long)n * (unsigned long long)m);
-    // 256 rows per workgroup; the columns split into blocks (multiples of a tile) so that a pass has about
-    // kTargetBlocks workgroups, each flushing its nonzero bins once.
+    hipLaunchKernelGGL(norms_kernel, dim3(o.xblocks + o.yblocks), dim3(256), kNormRows * (d | 1) * sizeof(double), s, xc, n, yc,
+                       m, d, xx, yy, bmax, o.xblocks, st, hist);
+    hipLaunchKernelGGL(layout_kernel, dim3(1024), dim3(256), 0, s, xc, n, yc, m, d, o.dp, o.mp, o.nc, xx, yy, bmax, o.xblocks,
+                       o.yblocks, xp, yp, (f16x8*)(w + o.xt), (f16x8*)(w + o.yt), (float*)(w + o.xf), (float*)(w + o.yf),
+                       o.ntx, o.nty, st);
+    switch (o.nc) {
+        case 1: launch_approx<1>(o, w, n, m, s); break;
+        case 2: launch_approx<2>(o, w, n, m, s); break;
+        case 3: launch_approx<3>(o, w, n, m, s); break;
+        case 4: launch_approx<4>(o, w, n, m, s); break;
+        case 5: launch_approx<5>(o, w, n, m, s); break;
+        case 6: launch_approx<6>(o, w, n, m, s); break;
+        case 7: launch_approx<7>(o, w, n, m, s); break;
+        default: launch_approx<8>(o, w, n, m, s); break;
+    }
+    hipLaunchKernelGGL(exact_kernel, dim3(1024), dim3(256), 0, s, (const unsigned*)(w + o.slabs), xp, yp, xx, yy, m, o.dp, st,
+                       keys, o.cap);
+    // Six digits at most; a typical bracket's keys differ in their low 43 bits (four digits, the other launches return).
+    const int cand_blocks = (int)std::min<unsigned long long>(128ull, (o.cap + 255) / 256);
+    for (int q = 0; q < kPasses; ++q)
+        hipLaunchKernelGGL(select_cand_kernel, dim3(cand_blocks), dim3(256), 0, s, keys, st, hist, q);
+    // The passes over every cost, which return at once unless the collected pairs did not hold the answer: blocks of 256
+    // rows by a multiple of a column tile, about kTargetBlocks of them, shared out over the workgroups.
     const int rb = (n + kRowsPerBlock - 1) / kRowsPerBlock;
     const int want = (kTargetBlocks + rb - 1) / rb;
     int cols = (m + want - 1) / want;
     cols = (cols + kColTile - 1) / kColTile * kColTile;
-    const dim3 grid(rb, (m + cols - 1) / cols);
-    // Passes up to kCompactPass recompute every cost; that pass also collects the keys matching its prefix,
-    // and the later passes histogram only those (unless there were more than cap: then they recompute).
-    const int cand_blocks = (int)std::min<unsigned long long>(1024ull, (cap + kRowsPerBlock - 1) / kRowsPerBlock);
-    for (int q = 0; q < kPasses; ++q) {
-        if (q > kCompactPass)
-            hipLaunchKernelGGL(select_cand_kernel, dim3(cand_blocks), dim3(kRowsPerBlock), 0, s, cand, count, cap, st,
-                               hist, kShift[q], kWidth[q]);
-        auto* pass = q < kCompactPass    ? select_pass_kernel<kPlain>
-                     : q == kCompactPass ? select_pass_kernel<kCollect>
-                                         : select_pass_kernel<kIfOverflow>;
-        hipLaunchKernelGGL(pass, grid, dim3(kRowsPerBlock), 0, s, xp, yp, xx, yy, n, m, dp, cols, st, hist, kShift[q],
-                           kWidth[q], cand, count, cap);
-        hipLaunchKernelGGL(select_scan_kernel, dim3(1), dim3(1024), 0, s, st, hist, kShift[q], kWidth[q]);
-    }
-    hipLaunchKernelGGL(select_finish_kernel, dim3(1), dim3(64), 0, s, st, out);
+    const long long blocks = (long long)rb * ((m + cols - 1) / cols);
+    const dim3 grid((unsigned)std::min<long long>(blocks, kTargetBlocks));
+    for (int q = 0; q < kPasses; ++q)
+        hipLaunchKernelGGL(select_pass_kernel, grid, dim3(kRowsPerBlock), 0, s, xp, yp, xx, yy, n, m, o.dp, cols, st, hist,
+                           kShift[q], kWidth[q], out);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? SK_OK : hip_fail(e, "sk_cost_median_f64");
 }
