@@ -240,6 +240,25 @@ int sk_loop_batch_init_f32(const sk_loop_f32* const* loops, int count, void* ws,
 int sk_loop_run_batch_f32(const void* ws, size_t ws_bytes, int count, const int* launch, int iters, void* stream);
 
 /*
+ * A solve's clouds from float64 points (row-major (n, d) device arrays, 1 <= d <= SK_KP_MAX), the normalisation of
+ * src/trnopt/sinkhorn.py:220-238 and the clouds of :131-165 on the GPU. `stat` is a device array of d + 1 doubles: the
+ * centre, then the cost scale; a cloud's normalised points are (p - centre) / sqrt(scale), in float64.
+ * sk_cloud_stats_f64: stat = {mean of all points of x and y, mean squared distance of the `samples` pairs
+ * (x[pairs_x[s]], y[pairs_y[s]]), or 1 if that is 0 or samples is 0}. The indices are the caller's, in range. ws
+ * (sk_cloud_stats_workspace_bytes) must be 256-byte aligned.
+ * sk_centre_f64: out = pts - centre, what sk_cost_median_f64 takes.
+ * sk_prepare_cloud_f64: the packed cloud pk (as sk_pack_cloud_f32 makes it from the points cast to fp32), |p|^2 (float64
+ * sums, cast; sk_pad_points(n) floats, 0 past n) and range, the largest |coordinate| in float64 (infinity if any is
+ * not finite): a caller refuses values above SK_MAX_ABS_COORDINATE, as for sk_pack_cloud_f32.
+ */
+size_t sk_cloud_stats_workspace_bytes(int d);
+int sk_cloud_stats_f64(const double* x, int n, const double* y, int m, int d, const int* pairs_x, const int* pairs_y,
+                       int samples, double* stat, void* ws, size_t ws_bytes, void* stream);
+int sk_centre_f64(const double* pts, int n, int d, const double* centre, double* out, void* stream);
+int sk_prepare_cloud_f64(const double* pts, int n, int d, const double* stat, float* sq, void* pk, double* range,
+                         void* stream);
+
+/*
  * Median of the squared-Euclidean cost over all pairs, the normalisation cost / median(cost) of
  * normalization(how="median") (src/trnopt/sinkhorn.py:229-233), which the reference evaluates on the host
  * over the materialised n x m float64 matrix:

@@ -133,6 +133,19 @@ __host__ __device__ inline const T* packed_log2_tiles(const void* pk, int npad, 
 }
 __device__ inline float packed_scale(const void* pk) { return reinterpret_cast<const float*>(pk)[1]; }
 
+// The power-of-two scale for a max |coordinate| m: m * s in [2^4, 2^5), clamped to [2^-32, 2^40] so that
+// s_x s_y and the scaled column terms stay well inside the fp32 range (m <= 7e13 < 2^46 keeps m s < 2^14).
+// The pieces then hold every coordinate within max(2^-23 |v|, 2^-25) of v = s x: relative to the largest,
+// 2^-23 at worst. The target sits low in the fp16 range so that the first cloud's log2-unit copy against
+// this scale, fl(c x) / s, lands in fp16's full-precision range for the usual score scales (bake_log2).
+__device__ __forceinline__ float pack_scale(float m) {
+    if (!(m > 0.0f)) return 1.0f;
+    int e;
+    frexpf(m, &e);                          // m in [2^(e-1), 2^e)
+    const int k = e > 37 ? -32 : (e < -35 ? 40 : 5 - e);
+    return ldexpf(1.0f, k);
+}
+
 // A half-step takes its scores in log2 units from the matrix cores ("log2_ready") when the first cloud's
 // log2-unit copy was made for its score scale c = (2 / eps) log2(e) and against its second cloud: header word
 // [2] of the first cloud equals c (and is not 0) and word [3] equals the second cloud's scale, word [1]. The

@@ -164,19 +164,6 @@ __global__ __launch_bounds__(256) void absmax_kernel(const float* __restrict__ s
     }
 }
 
-// The power-of-two scale for a max |coordinate| m: m * s in [2^4, 2^5), clamped to [2^-32, 2^40] so that
-// s_x s_y and the scaled column terms stay well inside the fp32 range (m <= 7e13 < 2^46 keeps m s < 2^14).
-// The pieces then hold every coordinate within max(2^-23 |v|, 2^-25) of v = s x: relative to the largest,
-// 2^-23 at worst. The target sits low in the fp16 range so that the first cloud's log2-unit copy against
-// this scale, fl(c x) / s, lands in fp16's full-precision range for the usual score scales (bake_log2).
-__device__ __forceinline__ float pack_scale(float m) {
-    if (!(m > 0.0f)) return 1.0f;
-    int e;
-    frexpf(m, &e);                          // m in [2^(e-1), 2^e)
-    const int k = e > 37 ? -32 : (e < -35 ? 40 : 5 - e);
-    return ldexpf(1.0f, k);
-}
-
 __global__ void pack_cloud_kernel(const float* __restrict__ src, int n, int d, int ld, char* __restrict__ dst,
                                   int npad, int nc) {
     // one thread per (tile, K chunk, lane): 8 coordinates, two pieces each

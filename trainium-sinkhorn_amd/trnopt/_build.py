@@ -42,6 +42,7 @@ UNITS = [   # (source, object name, extra flags)
                                                     "-mllvm", "-amdgpu-mfma-vgpr-form"]),
     ("sk_kernels.hip", "sk_kernels", []),
     ("sk_median.hip", "sk_median", []),
+    ("sk_prepare.hip", "sk_prepare", []),
 ]
 
 

@@ -101,6 +101,14 @@ _SIGS = {
                                               ctypes.c_size_t, ctypes.POINTER(ctypes.c_int), ctypes.c_void_p]),
     "sk_loop_run_batch_f32": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.POINTER(ctypes.c_int),
                                              ctypes.c_int, ctypes.c_void_p]),
+    "sk_cloud_stats_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int]),
+    "sk_cloud_stats_f64": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
+                                          ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p,
+                                          ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "sk_centre_f64": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
+                                     ctypes.c_void_p]),
+    "sk_prepare_cloud_f64": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
+                                            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "sk_cost_median_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "sk_cost_median_f64": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                           ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
@@ -249,21 +257,47 @@ class HipCloud:
 
     def __init__(self, pts: np.ndarray, log_w: np.ndarray, device, off: np.ndarray | None = None, role: int = 0):
         n, d = pts.shape
+        self._check(d, role)
+        pts = np.asarray(pts, dtype=np.float64)
+        _check_range("points", max(float(pts.max()), -float(pts.min())) if pts.size else 0.0)   # no |pts| copy
+        self._vectors(n, d, log_w, device, off, role, np.einsum("ij,ij->i", pts, pts))   # float64 sums, as the reference's
+        # the points unpadded (the packing pads them to npad x kp with zeros), cast to float32 on the host and
+        # copied from pageable memory (a pinned staging buffer for every cloud size bought nothing)
+        self.pk = pack_cloud(torch.from_numpy(pts.astype(np.float32)).to(device))
+
+    @classmethod
+    def prepared(cls, pts: torch.Tensor, stat: torch.Tensor, rng: torch.Tensor, log_w: np.ndarray, off=None,
+                 role: int = 0) -> "HipCloud":
+        """The cloud of float64 points already on the GPU, (n, d), normalised by stat = {centre, cost scale}
+        (cloud_stats): squared norms and packing on the GPU (sk_prepare_cloud_f64). rng (1,) float64 receives the
+        largest |coordinate|, for the caller to check (check_range) before the cloud is used."""
+        c = cls.__new__(cls)
+        n, d = pts.shape
+        cls._check(d, role)
+        c._vectors(n, d, log_w, pts.device, off, role, None)
+        c.pk = torch.empty(packed_bytes(n, d), dtype=torch.uint8, device=pts.device)
+        _check(lib().sk_prepare_cloud_f64(pts.data_ptr(), n, d, stat.data_ptr(), c.sq.data_ptr(), c.pk.data_ptr(),
+                                          rng.data_ptr(), _stream()), "sk_prepare_cloud_f64")
+        return c
+
+    @staticmethod
+    def _check(d: int, role: int) -> None:
         if pad_dim(d) > KP_MAX:
             raise ValueError(f"d = {d} is above the HIP kernels' limit (d <= {KP_MAX})")
         if role not in (0, 1):
             raise ValueError("role must be 0 (first cloud) or 1 (second cloud)")
-        pts = np.asarray(pts, dtype=np.float64)
-        _check_range("points", max(float(pts.max()), -float(pts.min())) if pts.size else 0.0)   # no |pts| copy
+
+    def _vectors(self, n, d, log_w, device, off, role, sq) -> None:
         npad = pad_points(n)
         self.n, self.npad, self.d, self.device, self.role = n, npad, d, device, role
-        # |p|^2 (float64 sums), log w, w, the low part of log w and the offset in one host array and one copy to
+        # |p|^2 (or room for it), log w, w, the low part of log w and the offset in one host array and one copy to
         # the device; padding points have |p|^2 = 0, log weight PAD_LOG_WEIGHT (weight exactly 0) and no offset.
         # log_w_lo = log w - fp32(log w) lets the on-device loop carry the log weights to float64 precision, so
         # that the two marginals' total masses agree (a mismatch of a few 1e-8 from fp32 log weights moves a
         # balanced iteration's potentials by eps times it per iteration).
         vec = np.zeros((4 if off is None else 5, npad), dtype=np.float32)
-        vec[0, :n] = np.einsum("ij,ij->i", pts, pts)   # float64 sums, as the reference's, then cast
+        if sq is not None:
+            vec[0, :n] = sq
         L = np.full(npad, PAD_LOG_WEIGHT)
         L[:n] = log_w
         vec[1] = L
@@ -276,9 +310,6 @@ class HipCloud:
         dv = torch.from_numpy(vec).to(device)
         self.sq, self.log_w, self.w, self.log_w_lo = dv[0], dv[1], dv[2], dv[3]
         self.off = dv[4] if off is not None else None
-        # the points unpadded (the packing pads them to npad x kp with zeros), cast to float32 on the host and
-        # copied from pageable memory (a pinned staging buffer for every cloud size bought nothing)
-        self.pk = pack_cloud(torch.from_numpy(pts.astype(np.float32)).to(device))
 
     def c_struct(self) -> SkCloud:
         return SkCloud(self.pk.data_ptr(), self.sq.data_ptr(), self.log_w.data_ptr(), self.w.data_ptr(),
@@ -335,6 +366,35 @@ def half_step(side: HipCloud, other: HipCloud, other_h: torch.Tensor, sc: torch.
     return out
 
 
+def check_range(max_abs: float) -> None:
+    """Refuses points out of the kernels' range (ValueError), as HipCloud does for points on the host."""
+    _check_range("points", max_abs)
+
+
+def to_device_f64(pts: np.ndarray, device) -> torch.Tensor:
+    return torch.as_tensor(np.ascontiguousarray(pts, dtype=np.float64)).to(device)
+
+
+def cloud_stats(x: torch.Tensor, y: torch.Tensor, stat: torch.Tensor, pairs=None) -> None:
+    """Into stat (d + 1,): the mean of all points of x and y (float64 on the GPU), and the mean squared distance of the
+    sampled pairs (i, j) given as two int arrays (1 if there are none or it is 0)."""
+    lb = lib()
+    (n, d), m = x.shape, y.shape[0]
+    ij = None if pairs is None else torch.from_numpy(np.stack(pairs).astype(np.int32)).to(x.device)
+    ws = _workspace(lb.sk_cloud_stats_workspace_bytes(d), x.device)
+    _check(lb.sk_cloud_stats_f64(x.data_ptr(), n, y.data_ptr(), m, d, None if ij is None else ij[0].data_ptr(),
+                                 None if ij is None else ij[1].data_ptr(), 0 if ij is None else ij.shape[1],
+                                 stat.data_ptr(), ws.data_ptr(), ws.numel(), _stream()), "sk_cloud_stats_f64")
+
+
+def centred(p: torch.Tensor, centre: torch.Tensor) -> torch.Tensor:
+    """p - centre in float64 on the GPU."""
+    out = torch.empty_like(p)
+    _check(lib().sk_centre_f64(p.data_ptr(), p.shape[0], p.shape[1], centre.data_ptr(), out.data_ptr(), _stream()),
+           "sk_centre_f64")
+    return out
+
+
 MEDIAN_D_MAX = 128                        # SK_MEDIAN_D_MAX
 
 
@@ -353,15 +413,18 @@ def cost_median_enqueue(xc: np.ndarray, yc: np.ndarray, device) -> torch.Tensor:
     yc = np.ascontiguousarray(yc, dtype=np.float64)
     if xc.ndim != 2 or yc.ndim != 2 or xc.shape[1] != yc.shape[1]:
         raise ValueError("xc (n, d) and yc (m, d) must share d")
-    (n, d), m = xc.shape, yc.shape[0]
-    lb = lib()
-    X = torch.as_tensor(xc).to(device)
-    Y = torch.as_tensor(yc).to(device)
     out = torch.empty(1, dtype=torch.float64, device=device)
+    cost_median_device(torch.as_tensor(xc).to(device), torch.as_tensor(yc).to(device), out)
+    return out
+
+
+def cost_median_device(X: torch.Tensor, Y: torch.Tensor, out: torch.Tensor) -> None:
+    """cost_median of centred float64 clouds already on the GPU, enqueued, into out (1,)."""
+    (n, d), m, device = X.shape, Y.shape[0], X.device
+    lb = lib()
     ws = _workspace(lb.sk_cost_median_workspace_bytes(n, m, d), device)
     _check(lb.sk_cost_median_f64(X.data_ptr(), Y.data_ptr(), n, m, d, out.data_ptr(), ws.data_ptr(), ws.numel(),
                                  _stream()), "sk_cost_median_f64")
-    return out
 
 
 # ---------------------------------------------------------------------------------------------------------

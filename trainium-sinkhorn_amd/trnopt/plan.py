@@ -55,29 +55,35 @@ def _lse_torch(rows, cols, h_cols, log_w_cols, eps, be, block=2048) -> np.ndarra
     return out
 
 
-def _lse_hip(rows, log_w_rows, cols, h_cols, log_w_cols, eps, opts: SinkhornOptions, role: int) -> np.ndarray:
-    """The same on the fused kernel: one sk_half_step_f32 with |x|^2 = 0, no offset, kappa = 1, so that its
-    output is exactly -eps lse, with the scores in log2 units from the matrix cores (the first cloud's log2-unit
-    copy made for this eps first)."""
-    from . import hip_sinkhorn as hk
-    dev = torch.device(opts.backend.device)
-    if dev.index is None:
-        dev = torch.device("cuda", torch.cuda.current_device())
-    with torch.cuda.device(dev):
-        R = hk.HipCloud(rows, log_w_rows, dev, role=role)
-        C = hk.HipCloud(cols, log_w_cols, dev, role=1 - role)
-        h = torch.zeros(C.npad, dtype=torch.float32, device=dev)
-        h[:C.n] = torch.as_tensor(h_cols, dtype=torch.float32)
-        R.sq = torch.zeros_like(R.sq)
-        out = hk.half_step(R, C, h, hk.scalars(eps, 1.0, dev), use_off=False, log2=True)
-        return (-out[:R.n].to("cpu", torch.float64) / eps).numpy()
+class _HipPlan:
+    """Both clouds on the GPU once, for the log-sum-exps of either side on the fused kernel: each one
+    sk_half_step_f32 with |x|^2 = 0, no offset, kappa = 1, so that its output is exactly -eps lse, with the scores in
+    log2 units from the matrix cores (the first cloud's log2-unit copy made for this eps, by the first of them)."""
 
+    def __init__(self, xs, log_a, ys, log_b, eps, opts):
+        from . import hip_sinkhorn as hk
+        dev = torch.device(opts.backend.device)
+        self.dev = torch.device("cuda", torch.cuda.current_device()) if dev.index is None else dev
+        self.eps, self.hk, self.baked = eps, hk, False
+        with torch.cuda.device(self.dev):
+            self.X = hk.HipCloud(xs, log_a, self.dev, role=0)
+            self.Y = hk.HipCloud(ys, log_b, self.dev, role=1)
+            self.X.sq, self.Y.sq = torch.zeros_like(self.X.sq), torch.zeros_like(self.Y.sq)
+            self.sc = hk.scalars(eps, 1.0, self.dev)
 
-def _side_lse(rows, log_w_rows, cols, g_cols, log_w_cols, eps, opts, role):
-    h = g_cols - (cols * cols).sum(axis=1)          # shifted potential of the column side, float64
-    if _use_hip(opts, rows.shape[1]):
-        return _lse_hip(rows, log_w_rows, cols, h, log_w_cols, eps, opts, role)
-    return _lse_torch(rows, cols, h, log_w_cols, eps, opts.backend)
+    def lse(self, role: int, h_cols) -> torch.Tensor:
+        """Enqueued: -eps lse of x's rows against y's columns (role 0) or the reverse, (n,) on the GPU."""
+        R, C = (self.X, self.Y) if role == 0 else (self.Y, self.X)
+        with torch.cuda.device(self.dev):
+            h = np.zeros(C.npad, dtype=np.float32)
+            h[:C.n] = h_cols
+            out = self.hk.half_step(R, C, torch.from_numpy(h).to(self.dev), self.sc, use_off=False, log2=not self.baked)
+        self.baked = True
+        return out[:R.n]
+
+    def read(self, *outs) -> list:
+        host = torch.cat(outs).to("cpu", torch.float64).numpy()
+        return [-v / self.eps for v in np.split(host, np.cumsum([len(o) for o in outs])[:-1])]
 
 
 def plan_marginals(x, y, res: SinkhornResult, a=None, b=None,
@@ -89,10 +95,15 @@ def plan_marginals(x, y, res: SinkhornResult, a=None, b=None,
     xs, ys = _normalised(x, y, res)
     log_a, log_b = _log_weights(a, len(xs), "a"), _log_weights(b, len(ys), "b")
     f, g, eps = np.asarray(res.f, np.float64), np.asarray(res.g, np.float64), float(res.eps)
-    lse_r = _side_lse(xs, log_a, ys, g, log_b, eps, opts, role=0)
-    lse_c = _side_lse(ys, log_b, xs, f, log_a, eps, opts, role=1)
-    rows = np.exp(log_a + (f - (xs * xs).sum(axis=1)) / eps + lse_r)
-    cols = np.exp(log_b + (g - (ys * ys).sum(axis=1)) / eps + lse_c)
+    xx, yy = np.einsum("ij,ij->i", xs, xs), np.einsum("ij,ij->i", ys, ys)
+    if _use_hip(opts, xs.shape[1]):
+        plan = _HipPlan(xs, log_a, ys, log_b, eps, opts)
+        lse_r, lse_c = plan.read(plan.lse(0, g - yy), plan.lse(1, f - xx))
+    else:
+        lse_r = _lse_torch(xs, ys, g - yy, log_b, eps, opts.backend)
+        lse_c = _lse_torch(ys, xs, f - xx, log_a, eps, opts.backend)
+    rows = np.exp(log_a + (f - xx) / eps + lse_r)
+    cols = np.exp(log_b + (g - yy) / eps + lse_c)
     return rows, cols
 
 
@@ -105,7 +116,12 @@ def pull_back(x, y, res: SinkhornResult, v, a=None, b=None, opts: SinkhornOption
     log_a, log_b = _log_weights(a, len(xs), "a"), _log_weights(b, len(ys), "b")
     log_bv = np.maximum(log_b + _log_vector(v, len(ys)), _NEG)
     f, g, eps = np.asarray(res.f, np.float64), np.asarray(res.g, np.float64), float(res.eps)
-    lse = _side_lse(xs, log_a, ys, g, log_bv, eps, opts, role=0)
-    out = log_a + (f - (xs * xs).sum(axis=1)) / eps + lse
+    xx, yy = np.einsum("ij,ij->i", xs, xs), np.einsum("ij,ij->i", ys, ys)
+    if _use_hip(opts, xs.shape[1]):
+        plan = _HipPlan(xs, log_a, ys, log_bv, eps, opts)
+        (lse,) = plan.read(plan.lse(0, g - yy))
+    else:
+        lse = _lse_torch(xs, ys, g - yy, log_bv, eps, opts.backend)
+    out = log_a + (f - xx) / eps + lse
     mx = out.max()
     return out - (mx + np.log(np.exp(out - mx).sum()))

@@ -191,15 +191,41 @@ def _solve_torch(p, opts: SinkhornOptions):
 # The fused HIP path (kernel="hip")
 
 def _hip_setup(p, opts: SinkhornOptions, dev, state=None):
-    """The device side of one solve on the fused path: both clouds packed, the loop set up (not run)."""
+    """The device side of one solve on the fused path: the points copied to the GPU as they are and normalised there
+    (the centre and the typical cost too, unless the options give them), both clouds packed, the loop set up (not
+    run). Sets p.center and p.scale, and refuses points out of range, with one read-back."""
     from . import hip_sinkhorn as hk
-    X = hk.HipCloud(p.xs, p.log_a, dev, p.off_x, role=0)
-    Y = hk.HipCloud(p.ys, p.log_b, dev, p.off_y, role=1)
+    d = p.x.shape[1]
+    px, py, center, scale = p.x, p.y, p.center, p.scale
+    if p.how is None:
+        if center.size == d or center.size == 1:
+            center = np.broadcast_to(center.reshape(-1), (d,))
+        else:                                # a centre per point, or the like: normalised on the host
+            px, py = (px - center) / np.sqrt(scale), (py - center) / np.sqrt(scale)
+            center, scale = np.zeros(d), 1.0
+    Xd, Yd = hk.to_device_f64(px, dev), hk.to_device_f64(py, dev)
+    stat = torch.empty(d + 3, dtype=torch.float64, device=dev)      # centre, cost scale, the clouds' largest |coordinate|
+    if p.how is None:
+        stat[:d + 1] = torch.from_numpy(np.append(center, scale))
+    elif p.how == "median":
+        hk.cloud_stats(Xd, Yd, stat)
+        med = stat[d:d + 1]
+        hk.cost_median_device(hk.centred(Xd, stat), hk.centred(Yd, stat), med)
+        med.masked_fill_(~(med > 0), 1.0)
+    else:
+        hk.cloud_stats(Xd, Yd, stat, _sample_pairs(len(p.x), len(p.y)))
+    X = hk.HipCloud.prepared(Xd, stat, stat[d + 1:d + 2], p.log_a, p.off_x, role=0)
+    Y = hk.HipCloud.prepared(Yd, stat, stat[d + 2:], p.log_b, p.off_y, role=1)
     loop = hk.DeviceLoop(X, Y, eps=opts.eps, rho_x=p.rho_x, rho_y=p.rho_y, sched=p.sched, stages=p.stages,
                          tol=p.tol, stage_tol=p.stage_tol, max_iters=opts.max_iters,
                          check_every=opts.check_every, stage_max_iters=opts.stage_max_iters,
                          fixed_iters=opts.fixed_iters, balanced=p.balanced, state=state)
     c1 = None if p.balanced else hk.scalars(opts.eps, 1.0, dev)     # requested before the loop's launches
+    host = stat.to("cpu").numpy()
+    hk.check_range(float(host[d + 1]))
+    hk.check_range(float(host[d + 2]))
+    if p.how is not None:
+        p.center, p.scale = host[:d].copy(), float(host[d])
     return SimpleNamespace(X=X, Y=Y, loop=loop, c1=c1)
 
 
@@ -299,38 +325,50 @@ def _log_weights(w, n: int, name: str) -> np.ndarray:
     return np.log(w)
 
 
+def _sample_pairs(n: int, m: int, samples: int = 20_000, seed: int = 0):
+    """The random pairs the typical cost is sampled over (src/trnopt/sinkhorn.py:234-236)."""
+    rng = np.random.default_rng(seed)
+    return rng.integers(n, size=samples), rng.integers(m, size=samples)
+
+
 def normalization(x: np.ndarray, y: np.ndarray, samples: int = 20_000, seed: int = 0,
                   how: str = "mean", device=None) -> tuple[np.ndarray, float]:
     """(center, cost_scale) as the reference computes them (src/trnopt/sinkhorn.py:220-238): center = mean of all
     points; cost_scale = the mean squared x-y distance over `samples` random pairs (rng seed `seed`), or with
     how="median" the median over all pairs when n m <= 1e8 (else over the random pairs). 1 if that is 0.
 
-    device: a ROCm GPU device to take the exact median there (sk_cost_median_f64: radix select over the cost
-    recomputed on the fly, no n x m array); None computes it on the host like the reference."""
+    device: a ROCm GPU device to take the exact median there (sk_cost_median_f64, no n x m array); None computes it
+    on the host like the reference."""
     x = np.asarray(x, dtype=np.float64)
     y = np.asarray(y, dtype=np.float64)
     center = np.concatenate([x, y]).mean(axis=0)
     if how == "median" and len(x) * len(y) <= 100_000_000:
-        xc, yc = x - center, y - center
         if device is not None:
-            from . import hip_sinkhorn as hk
-            scale = hk.cost_median(xc, yc, device)
+            scale = float(_median_enqueue(x, y, center, device).item())
             return center, (scale if scale > 0 else 1.0)
+        xc, yc = x - center, y - center
         C = ((xc * xc).sum(1)[:, None] + (yc * yc).sum(1)[None, :] - 2.0 * (xc @ yc.T)).ravel()
         scale = float(np.median(np.maximum(C, 0.0)))
     else:
-        rng = np.random.default_rng(seed)
-        i, j = rng.integers(len(x), size=samples), rng.integers(len(y), size=samples)
+        i, j = _sample_pairs(len(x), len(y), samples, seed)
         dd = ((x[i] - y[j]) ** 2).sum(axis=1)
         scale = float(np.median(dd) if how == "median" else dd.mean())
     return center, (scale if scale > 0 else 1.0)
+
+
+def _median_enqueue(x, y, center, device) -> torch.Tensor:
+    """The exact median cost on the GPU, enqueued: the points copied as they are, the centre taken off there."""
+    from . import hip_sinkhorn as hk
+    c = hk.to_device_f64(center, device)
+    out = torch.empty(1, dtype=torch.float64, device=c.device)
+    hk.cost_median_device(hk.centred(hk.to_device_f64(x, device), c), hk.centred(hk.to_device_f64(y, device), c), out)
+    return out
 
 
 def median_normalizations(pairs, device, samples: int = 20_000, seed: int = 0) -> list:
     """normalization(x, y, how="median", device=device) for every (x, y) of `pairs`, the exact medians of all of
     them enqueued on the GPU and read back with one synchronisation (a pipeline's pairs, each otherwise a round
     trip of its own). The same (center, cost_scale) as the one-pair call, pair by pair."""
-    from . import hip_sinkhorn as hk
     out, pending = [], []
     for x, y in pairs:
         x = np.asarray(x, dtype=np.float64)
@@ -339,7 +377,7 @@ def median_normalizations(pairs, device, samples: int = 20_000, seed: int = 0) -
             out.append(normalization(x, y, samples=samples, seed=seed, how="median", device=device))
             continue
         center = np.concatenate([x, y]).mean(axis=0)
-        pending.append((len(out), hk.cost_median_enqueue(x - center, y - center, device)))
+        pending.append((len(out), _median_enqueue(x, y, center, device)))
         out.append(center)
     if pending:
         scales = torch.cat([t for _, t in pending]).cpu().numpy()
@@ -355,7 +393,8 @@ def _gpu_device(opts: SinkhornOptions):
 
 def _prepare(x, y, a, b, opts: SinkhornOptions, a_target, b_target, hip: bool = False):
     """Validation, weights, normalisation and the eps schedule (src/trnopt/sinkhorn.py:250-320, 340-344). With
-    the HIP path selected, an exact median normalisation runs on the GPU."""
+    the HIP path selected the normalisation is left to _hip_setup (how: "mean" or "median"), unless the options give
+    it (how None: center and scale as they are) or its median is sampled on the host."""
     be = opts.backend
     x = np.asarray(x, dtype=np.float64)
     y = np.asarray(y, dtype=np.float64)
@@ -374,19 +413,25 @@ def _prepare(x, y, a, b, opts: SinkhornOptions, a_target, b_target, hip: bool = 
         rho_x = rho_y = opts.rho
     off_x = None if a_target is None else _log_weights(a_target, len(x), "a_target") - log_a
     off_y = None if b_target is None else _log_weights(b_target, len(y), "b_target") - log_b
+    how = None
     if isinstance(opts.normalize, tuple):
         center, scale = np.asarray(opts.normalize[0], dtype=np.float64), float(opts.normalize[1])
     elif opts.normalize:
         how = opts.normalize if isinstance(opts.normalize, str) else "mean"
-        center, scale = normalization(x, y, how=how,
-                                      device=_gpu_device(opts) if hip and x.shape[1] <= 128 else None)
+        if hip and not (how == "median" and len(x) * len(y) > 100_000_000):
+            center, scale = None, None
+        else:
+            center, scale = normalization(x, y, how=how)
+            how = None
     else:
         center, scale = np.zeros(x.shape[1]), 1.0
-    root = np.sqrt(scale)
-    if np.any(center != 0.0) or root != 1.0:
-        xs, ys = (x - center) / root, (y - center) / root
-    else:                                   # (x - 0) / 1 is x exactly: no copies
-        xs, ys = x, y
+    xs = ys = None
+    if not hip:
+        root = np.sqrt(scale)
+        if np.any(center != 0.0) or root != 1.0:
+            xs, ys = (x - center) / root, (y - center) / root
+        else:                                   # (x - 0) / 1 is x exactly: no copies
+            xs, ys = x, y
     stages = [e for e in (opts.eps_stages or ()) if e > opts.eps]
     sched = []
     if not stages and opts.eps_start is not None and opts.eps_start > opts.eps:
@@ -398,7 +443,7 @@ def _prepare(x, y, a, b, opts: SinkhornOptions, a_target, b_target, hip: bool = 
     # float32 rounding noise in the potentials' change sits near 1e-6 of eps: floor the thresholds (:340-344)
     stage_tol = max(opts.stage_tol, 1e-5 if f32 else 0.0)
     tol = max(opts.tol, 5e-6) if (f32 and not balanced) else opts.tol
-    return SimpleNamespace(x=x, y=y, xs=xs, ys=ys, log_a=log_a, log_b=log_b, off_x=off_x, off_y=off_y,
+    return SimpleNamespace(x=x, y=y, how=how, xs=xs, ys=ys, log_a=log_a, log_b=log_b, off_x=off_x, off_y=off_y,
                            rho_x=rho_x, rho_y=rho_y, balanced=balanced, center=center, scale=scale,
                            stages=stages, sched=sched, tol=tol, stage_tol=stage_tol)
 
@@ -464,7 +509,7 @@ class _HipBatch:
                 raise ValueError("cores > 1 split rows across NeuronCores in the reference; this build runs on one GPU")
             p = _prepare(q["x"], q["y"], q.get("a"), q.get("b"), opts, q.get("a_target"), q.get("b_target"), True)
             prepared.append((p, opts))
-        if len({str(_gpu_device(o)) for _, o in prepared}) != 1 or len({p.xs.shape[1] for p, _ in prepared}) != 1:
+        if len({str(_gpu_device(o)) for _, o in prepared}) != 1 or len({p.x.shape[1] for p, _ in prepared}) != 1:
             raise ValueError("sinkhorn_batch: every problem must run on one device with one d")
         self.prepared = prepared
         self.dev = dev = _gpu_device(prepared[0][1])
@@ -487,8 +532,8 @@ class _HipBatch:
             for (p, _), (at, bt) in zip(self.prepared, targets):
                 if p.off_x is None or p.off_y is None:
                     raise ValueError("solve(targets): the problem was made without marginal targets")
-                offs.append((_log_weights(at, len(p.xs), "a_target") - p.log_a,
-                             _log_weights(bt, len(p.ys), "b_target") - p.log_b))
+                offs.append((_log_weights(at, len(p.x), "a_target") - p.log_a,
+                             _log_weights(bt, len(p.y), "b_target") - p.log_b))
         with torch.cuda.device(self.dev):
             if offs is not None:
                 for (p, _), su, (ox, oy) in zip(self.prepared, self.setups, offs):
