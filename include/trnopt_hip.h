@@ -93,7 +93,13 @@ int sk_bake_log2_f32(void* first_pk, const void* second_pk, int n_first, int d, 
  * the NKI kernel there is no constraint on rows or m and K may be up to SK_KP_MAX.
  */
 /* ws: sk_row_lse_workspace_bytes() bytes, 256-byte aligned. */
+/* sk_row_lse_range_f32: the same, and into block_max (SK_ROW_LSE_BLOCKS device floats, or NULL) the largest |value| of
+ * xa and ya by blocks, infinity where one is not finite: the call expects finite values up to 7e13 in
+ * magnitude and gives meaningless sums otherwise, and a caller can refuse them by reading the entries. */
+#define SK_ROW_LSE_BLOCKS 512
 size_t sk_row_lse_workspace_bytes(int rows, int m, int K);
+int sk_row_lse_range_f32(const float* xa, const float* ya, float* lse, int rows, int m, int K, float* block_max, void* ws,
+                         size_t ws_bytes, void* stream);
 int sk_row_lse_f32(const float* xa, const float* ya, float* lse, int rows, int m, int K,
                    void* ws, size_t ws_bytes, void* stream);
 
@@ -249,7 +255,7 @@ int sk_loop_run_batch_f32(const void* ws, size_t ws_bytes, int count, const int*
  * sk_centre_f64: out = pts - centre, what sk_cost_median_f64 takes.
  * sk_prepare_cloud_f64: the packed cloud pk (as sk_pack_cloud_f32 makes it from the points cast to fp32), |p|^2 (float64
  * sums, cast; sk_pad_points(n) floats, 0 past n) and range, the largest |coordinate| in float64 (infinity if any is
- * not finite): a caller refuses values above SK_MAX_ABS_COORDINATE, as for sk_pack_cloud_f32.
+ * * not finite): a caller refuses values above 7e13, as for sk_pack_cloud_f32.
  */
 size_t sk_cloud_stats_workspace_bytes(int d);
 int sk_cloud_stats_f64(const double* x, int n, const double* y, int m, int d, const int* pairs_x, const int* pairs_y,

@@ -201,44 +201,67 @@ __global__ __launch_bounds__(256) void bake_log2_kernel(char* __restrict__ first
     if (idx == 0) bake_header(first, second, b);
 }
 
-// The general row log-sum-exp's packing: three bf16 pieces per coordinate (exact), no scale (the header
-// keeps the scale 1 written by pack_header_kernel).
-__global__ void pack_cloud_bf3_kernel(const float* __restrict__ src, int n, int d, int ld, char* __restrict__ dst,
-                                      int npad, int nc) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)(npad / SK_TILE) * nc * 64;
-    if (idx >= total) return;
-    const int lane = (int)(idx % 64);
-    const int cc = (int)((idx / 64) % nc);
-    const long long T = idx / (64 * nc);
-    const int r = lane & 31, h = lane >> 5;
-    const long long row = T * SK_TILE + r;
-    bf16x8 p0, p1, p2;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int k = 16 * cc + 8 * h + e;
-        const float v = (row < n && k < d) ? src[row * ld + k] : 0.0f;
-        const __bf16 a0 = (__bf16)v;
-        const float r1 = v - (float)a0;          // exact: v and a0 share the leading bits
-        const __bf16 a1 = (__bf16)r1;
-        p0[e] = a0;
-        p1[e] = a1;
-        p2[e] = (__bf16)(r1 - (float)a1);        // exact: at most 8 significant bits remain
+// The general row log-sum-exp's operands, in one launch (five, each a few us at these sizes, before): both clouds as
+// three bf16 pieces per coordinate (exact), no scale (header: scale 1, no copy), the column mask (0, or kMaskOut past m),
+// and with block_max (null: not wanted) each workgroup's largest |coordinate|, infinity for one that is not finite,
+// which spares a caller who refuses such input two passes of its own. One thread per unit of 8 coordinates at a time.
+struct Bf3Side {
+    const float* src;
+    int n, npad;
+    char* dst;
+};
+constexpr int kRowLseBlocks = SK_ROW_LSE_BLOCKS;
+__global__ __launch_bounds__(256) void row_lse_operands_kernel(Bf3Side x, Bf3Side y, int d, int nc, float* __restrict__ mask,
+                                                               int m, float* __restrict__ block_max) {
+    const long long ux = (long long)(x.npad / SK_TILE) * nc * 64, uy = (long long)(y.npad / SK_TILE) * nc * 64;
+    const long long step = (long long)gridDim.x * 256, first = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x < 32) {
+        unsigned* h = reinterpret_cast<unsigned*>(threadIdx.x < 16 ? x.dst : y.dst);
+        const int w = threadIdx.x & 15;
+        h[w] = w == 1 || w == 4 ? __float_as_uint(1.0f) : 0u;
     }
-    bf16x8* o = reinterpret_cast<bf16x8*>(dst + kHeaderBytes) + (T * nc + cc) * (3 * 64) + lane;
-    o[0] = p0;
-    o[64] = p1;
-    o[128] = p2;
+    for (long long j = first; j < y.npad; j += step) mask[j] = j < m ? 0.0f : kMaskOut;
+    float mx = 0.0f;
+    for (long long u = first; u < ux + uy; u += step) {
+        const Bf3Side& s = u < ux ? x : y;
+        const long long idx = u < ux ? u : u - ux;
+        const int lane = (int)(idx % 64);
+        const int cc = (int)((idx / 64) % nc);
+        const long long T = idx / (64 * nc);
+        const long long row = T * SK_TILE + (lane & 31);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int k = 16 * cc + 8 * (lane >> 5) + e;
+            v[e] = row < s.n && k < d ? s.src[row * d + k] : 0.0f;
+        }
+        bf16x8 p0, p1, p2;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            mx = fabsf(v[e]) <= 3.0e38f ? fmaxf(mx, fabsf(v[e])) : __builtin_inff();
+            const __bf16 a0 = (__bf16)v[e];
+            const float r1 = v[e] - (float)a0;       // exact: v and a0 share the leading bits
+            const __bf16 a1 = (__bf16)r1;
+            p0[e] = a0;
+            p1[e] = a1;
+            p2[e] = (__bf16)(r1 - (float)a1);        // exact: at most 8 significant bits remain
+        }
+        bf16x8* o = reinterpret_cast<bf16x8*>(s.dst + kHeaderBytes) + (T * nc + cc) * (3 * 64) + lane;
+        o[0] = p0;
+        o[64] = p1;
+        o[128] = p2;
+    }
+    if (block_max == nullptr) return;
+    __shared__ float red[4];
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) block_max[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
 size_t packed_bf3_bytes(int n, int d) {
     return (size_t)kHeaderBytes + (size_t)((n + SK_TILE - 1) / SK_TILE * SK_TILE) *
                                       ((d + SK_KP_ALIGN - 1) / SK_KP_ALIGN * SK_KP_ALIGN) * 6;
-}
-
-__global__ void fill_mask_kernel(float* __restrict__ mask, int m, int mpad) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < mpad) mask[j] = j < m ? 0.0f : kMaskOut;
 }
 
 // The merge pass: one workgroup per row group, then the loop step (sk_epilogue.h).
@@ -592,6 +615,11 @@ size_t sk_row_lse_workspace_bytes(int rows, int m, int K) {
 
 int sk_row_lse_f32(const float* xa, const float* ya, float* lse, int rows, int m, int K, void* ws, size_t ws_bytes,
                    void* stream) {
+    return sk_row_lse_range_f32(xa, ya, lse, rows, m, K, nullptr, ws, ws_bytes, stream);
+}
+
+int sk_row_lse_range_f32(const float* xa, const float* ya, float* lse, int rows, int m, int K, float* block_max, void* ws,
+                         size_t ws_bytes, void* stream) {
     if (xa == nullptr || ya == nullptr || lse == nullptr || ws == nullptr)
         return fail(SK_E_ARG, "sk_row_lse_f32: null pointer");
     if (rows < 1 || m < 1) return fail(SK_E_SHAPE, "sk_row_lse_f32: rows %d, m %d", rows, m);
@@ -611,17 +639,11 @@ int sk_row_lse_f32(const float* xa, const float* ya, float* lse, int rows, int m
     p += align_up((size_t)mp * 4);
     float2* part = (float2*)p;
     hipStream_t st = (hipStream_t)stream;
-    {
-        const int nc = kp / 16;
-        const long long ux = (long long)(rp / SK_TILE) * nc * 64, uy = (long long)(mp / SK_TILE) * nc * 64;
-        hipLaunchKernelGGL(pack_header_kernel, dim3(1), dim3(64), 0, st, (unsigned*)xpk);
-        hipLaunchKernelGGL(pack_header_kernel, dim3(1), dim3(64), 0, st, (unsigned*)ypk);
-        hipLaunchKernelGGL(pack_cloud_bf3_kernel, dim3((unsigned)((ux + 255) / 256)), dim3(256), 0, st, xa, rows, K, K,
-                           (char*)xpk, rp, nc);
-        hipLaunchKernelGGL(pack_cloud_bf3_kernel, dim3((unsigned)((uy + 255) / 256)), dim3(256), 0, st, ya, m, K, K,
-                           (char*)ypk, mp, nc);
-    }
-    hipLaunchKernelGGL(fill_mask_kernel, dim3((mp + 255) / 256), dim3(256), 0, st, mask, m, mp);
+    const Bf3Side sx = {xa, rows, rp, (char*)xpk}, sy = {ya, m, mp, (char*)ypk};
+    // every workgroup writes its block_max entry: the whole grid with it, else as many as there is work for
+    const long long units = ((long long)rp + mp) / SK_TILE * (kp / 16) * 64;
+    const int blocks = block_max != nullptr ? kRowLseBlocks : (int)std::min<long long>(kRowLseBlocks, (units + 255) / 256);
+    hipLaunchKernelGGL(row_lse_operands_kernel, dim3(blocks), dim3(256), 0, st, sx, sy, K, kp / 16, mask, m, block_max);
     Pass ps = {};
     ps.xr = xpk;
     ps.rows_pad = rp;
