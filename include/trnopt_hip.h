@@ -79,7 +79,7 @@ int sk_pack_cloud_f32(const float* pts, int n, int d, int ld, void* out, void* s
  * multiply less per score, same accuracy, the two directions still bit-identical); with any other sc[0],
  * or a copy made against another second cloud, they scale on the VALU as before. The copy is not made
  * (and the pair keeps scaling on the VALU) when max |fl(c x)| / s2 falls outside [2^-1, 2^15). One launch.
- * sk_loop_init_f32 makes it for the loop's first eps and the loop remakes it when eps changes; a caller of
+ * sk_loop_init_f32 makes it for the loop's first eps, and the f update after a change of eps remakes it; a caller of
  * sk_half_step_f32 may make it once per eps. No counterpart in the reference (an fp32-MFMA-free way to
  * apply its 1/eps scaling, src/trnopt/nki_sinkhorn.py:197-210).
  */
@@ -220,6 +220,14 @@ int sk_loop_init_f32(const sk_loop_f32* L, void* stream);
  * below that);
  * iterations after `done` do nothing. ws (sk_loop_workspace_bytes) must be 256-byte aligned. */
 int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream);
+/* The same iterations, bit for bit; where the problem is small (sk_kernels.hip, loop_persists) as one cooperative launch
+ * whose workgroups stay for all of them and pass the potentials to one another directly, else (and while the stream
+ * captures) as sk_loop_run_f32. Cooperative launches of one device run one after another: for a caller whose loops share
+ * the GPU on several streams sk_loop_run_f32 is the better form. If the workgroups should not all get to run, the loop
+ * gives up after about a second: state done with checks = -1, for the caller to start again with sk_loop_run_f32.
+ * sk_loop_resident: 1 where it would be the one launch, else 0. */
+int sk_loop_resident(const sk_loop_f32* L);
+int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream);
 
 /*
  * Several loops at once: `count` independent solves of the same d (each set up and initialised as above, on its

@@ -216,6 +216,12 @@ struct PartialArgs {
 int fail(int code, const char* fmt, ...);
 int hip_fail(hipError_t e, const char* where);
 
+// Several iterations of the loop with passes f and g in one launch (sk_loop.hip): both clouds of at most kLoopMaxBlocks
+// row blocks (one workgroup each, all resident) and kLoopMaxTiles tiles. exchange: loop_exchange_words 8-byte words, zero at
+// loop init.
+constexpr int kLoopMaxTiles = 192, kLoopMaxBlocks = 256;
+inline size_t loop_exchange_words(int nx_pad, int ny_pad) { return (size_t)nx_pad + ny_pad + 3 * (size_t)(ny_pad / 32); }
+hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int polls, hipStream_t stream);
 hipError_t launch_partial_small(const PartialArgs& a, int nc, hipStream_t stream);
 hipError_t launch_partial_large(const PartialArgs& a, int nc, hipStream_t stream);
 inline hipError_t launch_partial(const PartialArgs& a, int nc, hipStream_t stream) {

@@ -199,6 +199,30 @@ __device__ inline void set_scalars(sk_state* st, double e, double rho_x, double 
     st->sc_y[3] = (float)ky;
 }
 
+// A row's new potential from its merged maximum Md (the columns' log2 weight offset back on) and log2 S, see
+// merge_group: val = fh, and with l2 R = (c / 2) fh as well.
+struct RowTerms {
+    float sc2, kappa;      // eps, kappa
+    float c;               // score scale (2 / eps) log2(e)
+    float x2, off;         // |x|^2, log(target / weight)
+};
+__device__ __forceinline__ float row_value(const RowTerms& r, bool l2, bool log2_state, double Md, double l2s, double& R) {
+    const double kappa = r.kappa, x2d = r.x2, od = r.off;
+    if (l2 && log2_state) {
+        // In log2 units, R = (c / 2) fh (the loop's state): (c / 2) eps lse = M + log2 S exactly in the
+        // mathematics, so R = kappa (O - (M + log2 S)) + (kappa - 1) X2 with X2 = (c / 2) |x|^2 and
+        // O = log2(e) off, and fh = R / (c / 2), each rounded once from the double; the state stored for
+        // the other half-step's column terms is R + Ll (loop_weight_offset).
+        const double k2 = 0.5 * (double)r.c;
+        R = kappa * (od * (double)kLog2eD - (Md + l2s)) + (kappa - 1.0) * (x2d * k2);
+        return (float)(R / k2);
+    }
+    // eps lse = 2 M + eps ln(S) in accumulator units (log2-unit slots: M / c), with the caller's eps
+    // (float) as the reference's epilogue multiplies by it (src/trnopt/sinkhorn.py:119)
+    const double eps_lse = 2.0 * (l2 ? Md / (double)r.c : Md) + (double)r.sc2 * kLn2D * l2s;
+    return (float)(kappa * ((double)r.sc2 * od - eps_lse) + (kappa - 1.0) * x2d);
+}
+
 // Merge the slots of row i = 256 g + t (thread t of the workgroup, one row per thread) and apply the epilogue:
 //     lse = (2 / eps) M + ln S  (half-step, accumulator units) or M + ln S  (plain row-LSE)
 // When the partial kernel took its scores in log2 units (log2_ready, tested on the same header words), the
@@ -275,8 +299,6 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
         const Log2Split ls = lse_log2(S);
         const double l2s = (double)ls.e + (double)ls.lm;
         if (a.mode == kHalfStep) {
-            const double kappa = sc3, x2d = x2, od = o;
-            float val;
             // fh = kappa (|x|^2 + eps off - eps lse) - |x|^2 (src/trnopt/sinkhorn.py:119) is evaluated as
             //     fh = kappa (eps off - eps lse) + (kappa - 1) |x|^2,
             // the same number in the mathematics (kappa - 1 is exact), rounded at fh's own magnitude. Rounded the
@@ -286,25 +308,15 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
             // iteration (2e-8 on the 10k x 10k d 64 mixture clouds at eps 0.05, whose f is near 0.4; the
             // reference's float32 sequence drifts the same way, less), which shows as a floor of the balanced
             // error (4.5e-7 there) and an offset of the cost. For kappa = 1 and no offset it is -eps lse, exact.
+            double R = 0.0;
+            const float val = row_value({sc2, sc3, c_hs, x2, o}, l2, a.out2 != nullptr, Md, l2s, R);
             if (l2 && a.out2 != nullptr) {
-                // In log2 units, R = (c / 2) fh (the loop's state): (c / 2) eps lse = M + log2 S exactly in the
-                // mathematics, so R = kappa (O - (M + log2 S)) + (kappa - 1) X2 with X2 = (c / 2) |x|^2 and
-                // O = log2(e) off, and fh = R / (c / 2), each rounded once from the double; the state stored for
-                // the other half-step's column terms is R + Ll (loop_weight_offset).
-                const double k2 = 0.5 * (double)c_hs;
-                const double R = kappa * (od * (double)kLog2eD - (Md + l2s)) + (kappa - 1.0) * (x2d * k2);
-                val = (float)(R / k2);
                 // (a schedule's next eps is known here: its log2-unit potential comes from fh, as the control derives
                 // it for a new stage)
                 const double Rn = a.next_k2 != 0.0f ? (double)val * (double)a.next_k2 : R;
                 if (i < a.n_store) st<COH>(a.out2 + i, (float)(Rn + (double)ll));
-            } else {
-                // eps lse = 2 M + eps ln(S) in accumulator units (log2-unit slots: M / c), with the caller's eps
-                // (float) as the reference's epilogue multiplies by it (src/trnopt/sinkhorn.py:119)
-                const double eps_lse = 2.0 * (l2 ? Md / (double)c_hs : Md) + (double)sc2 * kLn2D * l2s;
-                val = (float)(kappa * ((double)sc2 * od - eps_lse) + (kappa - 1.0) * x2d);
-                if (a.out2 != nullptr && a.next_k2 != 0.0f && i < a.n_store)
-                    st<COH>(a.out2 + i, (float)((double)val * (double)a.next_k2 + (double)ll));
+            } else if (a.out2 != nullptr && a.next_k2 != 0.0f && i < a.n_store) {
+                st<COH>(a.out2 + i, (float)((double)val * (double)a.next_k2 + (double)ll));
             }
             if (a.meas != nullptr) {
                 if (i < a.n_real) dmax = fabsf(val - old);
@@ -359,6 +371,30 @@ __device__ inline bool needs_control(int it, int stage, int stage_it, const Loop
     return c.fixed_iters == 0 && stage_it % c.check_every == 0;
 }
 
+// The decisions of sinkhorn.py:356-378 after iteration `it` from its convergence measures (mx, sm over all rows; inv_eps
+// of the iteration that ran): advances (stage, stage_it), sets conv; true when a check ran, with its measure in err.
+__device__ inline bool control_decide(const LoopCfg& c, int it, float inv_eps, float mx, double sm, int& stage, int& stage_it,
+                                      int& conv, double& err) {
+    if (c.n_stages > 0 && stage < c.n_stages) {
+        // An intermediate stage: advance once the potentials settle or after stage_max_iters.
+        if (stage_it % c.check_every == 0) {
+            const double ch = (double)(mx * inv_eps);
+            if (ch < c.stage_tol || stage_it >= c.stage_max_iters) {
+                stage += 1;
+                stage_it = 0;
+            }
+        }
+        return false;
+    }
+    const bool check = c.fixed_iters == 0 && (c.n_stages > 0 || it > c.n_sched) &&
+                       (stage_it % c.check_every == 0 || it == c.max_iters);
+    if (check) {
+        err = c.balanced != 0 ? sm : (double)(mx * inv_eps);
+        if (err < c.tol) conv = 1;
+    }
+    return check;
+}
+
 // After the g update of one iteration, by one wave: the body of sinkhorn.py:356-378. With (it, stage_it)
 // already advanced by the f update's merge, runs the balanced / unbalanced check at the reference's cadence,
 // advances the stage, sets `done`, and writes the next iteration's eps and {2/eps, 1/eps, eps, kappa}.
@@ -377,30 +413,14 @@ __device__ inline void control_step(sk_state* st, const float2* meas, int nmeas,
         sm += __shfl_xor(sm, o);
     }
     if (tid_x() != 0) return;
-    const float inv_eps = st->sc_x[1];          // 1/eps of the iteration that just ran
-    const int it = st->it;
-    int stage = st->stage;
-    int stage_it = st->stage_it;
-    int conv = 0;
-    if (c.n_stages > 0 && stage < c.n_stages) {
-        // An intermediate stage: advance once the potentials settle or after stage_max_iters.
-        if (stage_it % c.check_every == 0) {
-            const double ch = (double)(mx * inv_eps);
-            if (ch < c.stage_tol || stage_it >= c.stage_max_iters) {
-                stage += 1;
-                stage_it = 0;
-            }
-        }
-    } else {
-        const bool check = c.fixed_iters == 0 && (c.n_stages > 0 || it > c.n_sched) &&
-                           (stage_it % c.check_every == 0 || it == c.max_iters);
-        if (check) {
-            const double err = c.balanced != 0 ? sm : (double)(mx * inv_eps);
-            st->err = err;
-            st->checks += 1;
-            if (err < c.tol) conv = 1;
-        }
+    int stage = st->stage, stage_it = st->stage_it, conv = 0;
+    double err;
+    const bool check = control_decide(c, st->it, st->sc_x[1], mx, sm, stage, stage_it, conv, err);
+    if (check) {
+        st->err = err;
+        st->checks += 1;
     }
+    const int it = st->it;
     const int done = (conv != 0 || it >= c.max_iters) ? 1 : 0;
     st->stage = stage;
     st->stage_it = stage_it;

@@ -311,7 +311,10 @@ __global__ __launch_bounds__(256) void loop_log2_kernel(Log2Side x, Log2Side y, 
 // ---------------------------------------------------------------------------------------------------
 // On-device loop control.
 
-__global__ void loop_init_kernel(sk_state* st, LoopCfg c, int* __restrict__ counters, int ncounters) {
+__global__ void loop_init_kernel(sk_state* st, LoopCfg c, int* __restrict__ counters, int ncounters,
+                                 unsigned long long* __restrict__ exchange, int nexchange) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nexchange; k += gridDim.x * blockDim.x) exchange[k] = 0ull;
+    if (blockIdx.x != 0) return;
     for (int k = threadIdx.x; k < ncounters; k += blockDim.x) counters[k] = 0;
     if (threadIdx.x != 0) return;
     st->it = 0;
@@ -538,6 +541,27 @@ constexpr int kFuseMinGroups = 40;
 bool fused_merge(const Plan& pl) {
     const int v = env_int("TRNOPT_HIP_FUSED_MERGE", -1);
     return v < 0 ? pl.ngroups >= kFuseMinGroups : v != 0;
+}
+
+// Whether the loop's one-launch form (sk_loop.hip) can take a problem, and whether it is the faster one. Its update costs
+// 5 us plus the tiles of one row block on one CU, 16 waves and fewer in the wider kernels; the launches' 7-8 us plus the
+// tiles spread over every CU. Measured (us an iteration, launches against one launch of 10 iterations): 100 x 90 d 5
+// 14.5 / 10.0, 700 x 500 d 16 17.0 / 12.1, 1,500 x 1,400 d 16 20.4 / 16.2, d 30 20.9 / 18.5, 3,000 x 3,100 d 16 21.3 / 18.5;
+// 700 x 500 d 64 18.8 / 16.5, 300 x 280 d 128 19.7 / 17.9; past the line 2,048 x 2,048 d 30 19.1 / 19.8, 1,500 x 1,400 d 64
+// 22.5 / 23.2, 700 x 500 d 128 21.1 / 22.1, 4,500 x 4,600 d 5 23.7 / 23.9. TRNOPT_HIP_LOOP=0 turns it off, =1 takes it
+// wherever it fits.
+constexpr int kLoopMaxChunkTiles = 96;
+bool loop_fits(const Plan& pf, const Plan& pg) {
+    return pf.ok && pg.ok && pf.nt <= kLoopMaxTiles && pg.nt <= kLoopMaxTiles &&
+           std::max(pf.nrb, pg.nrb) <= std::min(kLoopMaxBlocks, cu_count());
+}
+bool loop_persists(const Plan& pf, const Plan& pg) {
+    const int v = env_int("TRNOPT_HIP_LOOP", -1);
+    return v < 0 ? pf.nc * std::max(pf.nt, pg.nt) <= kLoopMaxChunkTiles : v != 0;
+}
+bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
 }
 
 void launch_bake(void* first, const void* second, int npad, int nc, const float* sc, hipStream_t st) {
@@ -801,7 +825,8 @@ size_t sk_loop_workspace_bytes(int nx_pad, int ny_pad, int d) {
     return std::max(partial_bytes(pf, nx_pad), partial_bytes(pg, ny_pad)) +
            align_up((size_t)meas_count(ny_pad) * sizeof(float2)) +
            align_up((size_t)(1 + std::max(pf.ngroups, pg.ngroups)) * sizeof(int)) +
-           3 * (align_up((size_t)nx_pad * sizeof(float)) + align_up((size_t)ny_pad * sizeof(float)));
+           3 * (align_up((size_t)nx_pad * sizeof(float)) + align_up((size_t)ny_pad * sizeof(float))) +
+           (loop_fits(pf, pg) ? align_up(loop_exchange_words(nx_pad, ny_pad) * 8) : 0);
 }
 
 namespace {
@@ -819,6 +844,8 @@ struct LoopLayout {
     float* rf;
     float* rg;
     float *lxh, *lxl, *lyh, *lyl;
+    unsigned long long* exchange;     // of the one-launch form, where it fits, else null
+    int nexchange;
 };
 
 LoopLayout loop_layout(const sk_loop_f32* L) {
@@ -838,6 +865,9 @@ LoopLayout loop_layout(const sk_loop_f32* L) {
     o.lxl = (float*)((char*)o.lxh + bx);
     o.lyh = (float*)((char*)o.lxl + bx);
     o.lyl = (float*)((char*)o.lyh + by);
+    const bool fits = loop_fits(o.pf, o.pg);
+    o.exchange = fits ? (unsigned long long*)((char*)o.lyl + by) : nullptr;
+    o.nexchange = fits ? (int)loop_exchange_words(L->x.npad, L->y.npad) : 0;
     return o;
 }
 }  // namespace
@@ -856,15 +886,15 @@ int sk_loop_init_f32(const sk_loop_f32* L, void* stream) {
     if (L->ws_bytes < need) return fail(SK_E_WORKSPACE, "sk_loop_init_f32: workspace %zu < %zu bytes", L->ws_bytes, need);
     if (((uintptr_t)L->ws & 255) != 0) return fail(SK_E_ARG, "sk_loop_init_f32: workspace must be 256-byte aligned");
     const LoopLayout lo = loop_layout(L);
-    hipLaunchKernelGGL(loop_init_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, L->state, loop_cfg(L),
-                       lo.counters, lo.ncounters);
+    hipLaunchKernelGGL(loop_init_kernel, dim3(lo.exchange != nullptr ? 16 : 1), dim3(256), 0, (hipStream_t)stream, L->state,
+                       loop_cfg(L), lo.counters, lo.ncounters, lo.exchange, lo.nexchange);
     // both clouds' log2 weight offsets into their headers (each is the column cloud of one half-step)
     hipLaunchKernelGGL(weight_offset_kernel, dim3(1), dim3(kWeightMaxThreads), 0, (hipStream_t)stream, L->x.log_w,
                        L->x.n, (unsigned*)const_cast<void*>(L->x.pk));
     hipLaunchKernelGGL(weight_offset_kernel, dim3(1), dim3(kWeightMaxThreads), 0, (hipStream_t)stream, L->y.log_w,
                        L->y.n, (unsigned*)const_cast<void*>(L->y.pk));
     // x's log2-unit copy for the first iteration's eps, both clouds' log2 weights and both log2-unit potentials
-    // (from fh and the caller's gh); the loop control remakes the copy and the potentials when eps changes
+    // (from fh and the caller's gh); when eps changes the next f update remakes the copy and the g update's merge the potentials
     launch_bake(const_cast<void*>(L->x.pk), L->y.pk, L->x.npad, sk_pad_dim(L->d) / 16, L->state->sc_x,
                 (hipStream_t)stream);
     const int nmax = std::max(L->x.npad, L->y.npad);
@@ -975,6 +1005,24 @@ int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream) {
         if (e != hipSuccess) return hip_fail(e, "sk_loop_run_f32");
     }
     return SK_OK;
+}
+
+int sk_loop_resident(const sk_loop_f32* L) {
+    if (check_loop(L, "sk_loop_resident") != SK_OK || !log2_enabled()) return 0;
+    const LoopLayout lo = loop_layout(L);
+    return lo.exchange != nullptr && loop_persists(lo.pf, lo.pg) ? 1 : 0;
+}
+
+int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream) {
+    if (int r = check_loop(L, "sk_loop_run_resident_f32")) return r;
+    if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_resident_f32: iters %d < 0", iters);
+    if (iters < 2 || sk_loop_resident(L) == 0 || capturing((hipStream_t)stream)) return sk_loop_run_f32(L, iters, stream);
+    const LoopLayout lo = loop_layout(L);
+    Pass f, g;
+    loop_passes(L, lo, f, g);
+    const hipError_t e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc,
+                                    env_int("TRNOPT_HIP_LOOP_POLLS", 0), (hipStream_t)stream);
+    return e == hipSuccess ? SK_OK : hip_fail(e, "sk_loop_run_resident_f32");
 }
 
 }  // extern "C"

@@ -1,0 +1,483 @@
+// The on-device loop of small problems as one launch for many iterations (both clouds at most one 32-row block per CU
+// and kLoopMaxTiles column tiles; taken by the rule of loop_persists, sk_kernels.hip).
+//
+// What bounds the launch-by-launch loop there: a half-step at 2,048 x 2,048 d 64 is about 1.5 us of tiles, but its two
+// launches take 11 us: each starts up, fetches its arguments and then the scalars they point to, and the slots, the
+// potentials and the arguments pass between them through memory. Here one workgroup per 32-row block of x and of y
+// stays for all the iterations; all that passes between workgroups is the new potentials, each as one 8-byte word
+// {value, iteration tag} that its readers poll: the data is its own flag, so an exchange costs one store and one load
+// across the XCDs and no barrier, fence or counter. 700 x 500 d 16: 17.0 -> 12.1 us an iteration, 100 x 90 d 5 14.5 -> 10.0
+// (launches of 10 iterations; loop_persists has more sizes and both sides of its line).
+//
+// Bit for bit the launch-by-launch loop: a row block's columns are summed in the same segments as the split of the
+// partial kernel gives its row group (Split), each segment by one wave with the same instructions (sk_tile.h), and a
+// row's segments are merged in the same order (merge_group); the control takes the same decisions from the same measures
+// (control_decide), each workgroup for itself.
+//
+// Every wait ends: the launch is cooperative (all its workgroups are resident), and a poll that has not seen its word after
+// `polls` rounds gives up: its workgroup ends without publishing, so that every other one's polls end the same way, and the
+// state says so (checks = -1, done); the host then runs the loop again in launches.
+//
+// A potential's word is overwritten only after every reader has it: the next iteration's value is published by a
+// workgroup that has read all of the other cloud's values, each published by a workgroup that had read all of this one's.
+
+#include "sk_common.h"
+#include "sk_epilogue.h"
+#include "sk_tile.h"
+
+namespace sk {
+namespace {
+
+constexpr int kMaxPolls = 1 << 20;                  // of a word before a workgroup gives up: about a second
+constexpr int kRowsOfBlock = 32;
+// Waves of a workgroup: as many as hide each other's latencies with the operands in registers (128, 168, 256 a lane).
+constexpr int loop_waves(int nc) { return nc <= 2 ? 16 : nc <= 4 ? 12 : 8; }
+
+typedef unsigned long long u64;
+
+__device__ __forceinline__ void publish(u64* p, unsigned bits, unsigned tag) {
+    __hip_atomic_store(p, (u64)bits | ((u64)tag << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 peek(const u64* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// What every workgroup knows of the loop, in LDS; changed by thread 0 between barriers.
+struct Ctl {
+    sk_state st;          // this workgroup's copy
+    float c, t, s2;       // the log2-unit copy: its score scale (0: none), unit, and the second cloud's scale
+    int pending;          // its tiles are to be made by this iteration's f update
+    int polls;            // rounds before a poll gives up,
+    int abort;            // and whether one has
+};
+
+// The tile loop of one segment, the rows' operands in xv, the first tile's in yv (load_y(t) requests tile t's): (M, S) per
+// lane. A tile's operands are requested as soon as the last MFMA of the one before has read the registers.
+template <int NC, int ROLE, bool L2, class LoadY>
+__device__ __forceinline__ void segment(const f16x8 (&xv)[NC][2], f16x8 (&yv)[NC][2], LoadY&& load_y, const bf16x8* cols,
+                                        const bf16x8& ones, int lane, int tb, int te, float c, float& M, float& S) {
+    using C = Contract<kF16x2>;
+    float Ms[1] = {kEmpty}, Ss[1] = {0.0f};
+    auto none = [](int) { return f32x4{}; };
+    for (int t = tb; t < te; ++t) {
+        const bf16x8 colA = cols[t * 32 + (lane & 31)];
+        f32x16 acc[1] = {f32x16{}};
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc)
+#pragma unroll
+            for (int p = 0; p < C::products; ++p) {
+                const int rp = ROLE == 0 ? C::first[p] : C::second[p], cp = ROLE == 0 ? C::second[p] : C::first[p];
+                acc[0] = C::mfma(yv[cc][cp], xv[cc][rp], acc[0]);
+            }
+        if (t + 1 < te) load_y(t + 1);
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(colA, ones, acc[0], 0, 0, 0);
+        Online<1, L2, true> on;
+        static_for<0, kOps>([&](auto K) { on.template step<decltype(K)::value>(acc, none, Ms, Ss, c); });
+    }
+    M = Ms[0];
+    S = Ss[0];
+}
+
+// One update: rows of block rb (ROLE 0: x, 1: y) against the other cloud. Fills the merged maximum and sum of row tid for
+// tid < 32. expect: the tag of the column potentials (0: the launch's first f update, which takes them from memory).
+template <int NC, int ROLE>
+__device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsigned expect, int rb, Ctl& ctl, bf16x8* cols,
+                                       float2* slots, float& Mr, float& Sr) {
+    constexpr int W = loop_waves(NC), NT = 64 * W, TILE16 = NC * 2 * 64;
+    const int tid = tid_x(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float* sc = ROLE == 0 ? ctl.st.sc_x : ctl.st.sc_y;
+    const float chs = sc[0] * kLog2e;
+    const bool l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(ROLE == 0 ? a.yc : a.xr);
+    const float t = ctl.t;
+    const f16x8* xt = l2 && ROLE == 0 ? packed_log2_tiles<f16x8>(a.xr, a.nrb * 32, NC) : packed_tiles<f16x8>(a.xr);
+    const f16x8* yt = l2 && ROLE == 1 ? packed_log2_tiles<f16x8>(a.yc, a.s.nt * 32, NC) : packed_tiles<f16x8>(a.yc);
+    f16x8 xv[NC][2];
+#pragma unroll
+    for (int k = 0; k < NC * 2; ++k) xv[k / 2][k % 2] = xt[(size_t)rb * TILE16 + k * 64 + lane];
+    const bool remake = l2 && ctl.pending != 0;          // this iteration's f update makes x's log2-unit copy
+    if (ROLE == 0 && remake) {
+        const BakeParams bp = bake_params(a.xr, a.yc, sc);
+        const f16x8* own = packed_tiles<f16x8>(a.xr);
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc) {
+            const size_t u = (size_t)rb * TILE16 + cc * 128 + lane;
+            bake_pieces(own[u], own[u + 64], bp, xv[cc][0], xv[cc][1]);
+        }
+    }
+    // The wave's first segment, its first tile requested before the wait for the potentials (unless that is in the making)
+    const int g = rb / (kRowsPerGroup / kRowsOfBlock), p0 = first_wg(g, a.s), ns = last_wg(g, a.s) - p0 + 1;
+    const int lo = g * a.s.nt, hi = lo + a.s.nt;
+    auto bounds = [&](int s, int& tb, int& te) {
+        const int q0 = __builtin_amdgcn_readfirstlane(unit_at(cost_start(p0 + s, a.s), a.s));
+        const int q1 = __builtin_amdgcn_readfirstlane(unit_at(cost_start(p0 + s + 1, a.s), a.s));
+        tb = (q0 > lo ? q0 : lo) - lo;
+        te = (q1 < hi ? q1 : hi) - lo;
+    };
+    int tb = 0, te = 0;
+    if (wave < ns) bounds(wave, tb, te);
+    f16x8 yv[NC][2];
+    auto load_y = [&](int q) {
+        const f16x8* b0 = yt + (size_t)q * TILE16;
+#pragma unroll
+        for (int k = 0; k < NC * 2; ++k) yv[k / 2][k % 2] = b0[k * 64 + lane];
+    };
+    if (!(ROLE == 1 && remake)) load_y(tb);
+    // Column terms, as partial_pass takes them
+    const float sigma = packed_scale(a.xr) * packed_scale(a.yc);
+    const float inv_sigma = l2 ? 1.0f / t : (1.0f / packed_scale(a.xr)) * (1.0f / packed_scale(a.yc));
+    const float alpha = l2 ? 1.0f : 0.5f, beta = l2 ? 1.0f : 0.5f * sc[2], cs = l2 ? t : sigma;
+    const float c = l2 ? inv_sigma : chs * inv_sigma;
+    const float* u0 = l2 ? a.u2 : a.u;
+    const float* v0 = l2 ? a.v2 : a.v;
+    const int n = a.s.nt * 32;
+    for (int j0 = 0; j0 < n; j0 += 4 * NT) {
+        float u[4], v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = j0 + q * NT + tid < n ? j0 + q * NT + tid : n - 1;
+            v[q] = v0[j];
+            u[q] = expect == 0u ? u0[j] : 0.0f;
+        }
+        if (expect != 0u) {
+            bool all = false;
+            for (int r = 0; !all && r < ctl.polls; ++r) {
+                u64 w[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) w[q] = peek(ex + (j0 + q * NT + tid < n ? j0 + q * NT + tid : n - 1));
+                all = true;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    all = all && (unsigned)(w[q] >> 32) == expect;
+                    u[q] = __uint_as_float((unsigned)w[q]);
+                }
+            }
+            if (!all) ctl.abort = 1;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = j0 + q * NT + tid;
+            const float term = fmaxf(cs * fmaf(beta, v[q], fmaf(0.0f, v[q], alpha * u[q])), kPadScore);
+            if (j < n) cols[j] = column_operand(term);
+        }
+    }
+    __syncthreads();
+    if (remake) {
+        if (ROLE == 0) {
+            // The copy's tiles of this row block, now that every y workgroup has published, i.e. is done with the old copy;
+            // out of this XCD's L2 before the rows' potentials are published (by the same wave).
+            if (wave == 0) {
+                f16x8* copy = const_cast<f16x8*>(xt) + (size_t)rb * TILE16;
+#pragma unroll
+                for (int k = 0; k < NC * 2; ++k) copy[k * 64 + lane] = xv[k / 2][k % 2];
+                __threadfence();
+            }
+        } else {
+            __threadfence();      // the copy that the other workgroups have made, not this L2's old lines
+            load_y(tb);
+        }
+    }
+    const bf16x8 ones = column_ones(lane >> 5);
+    for (int s = wave; s < ns; s += W) {
+        float M, S;
+        if (l2)
+            segment<NC, ROLE, true>(xv, yv, load_y, cols, ones, lane, tb, te, c, M, S);
+        else
+            segment<NC, ROLE, false>(xv, yv, load_y, cols, ones, lane, tb, te, c, M, S);
+        if (s + W < ns) {
+            bounds(s + W, tb, te);
+            load_y(tb);
+        }
+        // as store_rows
+        const float Mo = __shfl_xor(M, 32), So = __shfl_xor(S, 32);
+        const float Mn = fmaxf(M, Mo);
+        const float Sn = S * ex2(c * (M - Mn)) + So * ex2(c * (Mo - Mn));
+        if (lane < 32) slots[s * kRowsOfBlock + lane] = make_float2(fmaxf(Mn * inv_sigma, kEmpty), Sn);
+    }
+    __syncthreads();
+    if (tid < kRowsOfBlock) {
+        // as merge_group
+        const float cm = l2 ? 1.0f : chs;
+        float M = kEmpty, S = 0.0f;
+        for (int q = 0; q < ns; q += kMergeBatch) {
+            float2 v[kMergeBatch];
+#pragma unroll
+            for (int k = 0; k < kMergeBatch; ++k) v[k] = q + k < ns ? slots[(q + k) * kRowsOfBlock + tid] : make_float2(kEmpty, 0.0f);
+            float Mn = M;
+#pragma unroll
+            for (int k = 0; k < kMergeBatch; ++k) Mn = fmaxf(Mn, v[k].x);
+            float Sn = S * ep_ex2(cm * (M - Mn));
+#pragma unroll
+            for (int k = 0; k < kMergeBatch; ++k) Sn += v[k].y * ep_ex2(cm * (v[k].x - Mn));
+            M = Mn;
+            S = Sn;
+        }
+        Mr = M;
+        Sr = S;
+    }
+}
+
+// The control of one iteration (every workgroup for itself, from the same measures): advances ctl, true when the loop is
+// done. ny: row blocks of y; msr their published measures {max change}, {low}, {high half of the error sum}.
+template <int NT>
+__device__ inline bool control(const PartialArgs& g, const u64* msr, unsigned tag, int ny, bool measured, Ctl& ctl, float* lds_mx,
+                               double* lds_sm) {
+    const int tid = tid_x();
+    if (measured) {
+        for (int b = tid; b < ny; b += NT) {
+            u64 w[3];
+            bool all = false;
+            for (int r = 0; !all && r < ctl.polls; ++r) {
+                all = true;
+                for (int q = 0; q < 3; ++q) {
+                    w[q] = peek(msr + 3 * b + q);
+                    all = all && (unsigned)(w[q] >> 32) == tag;
+                }
+            }
+            if (!all) ctl.abort = 1;
+            lds_mx[b] = __uint_as_float((unsigned)w[0]);
+            lds_sm[b] = __longlong_as_double((long long)((w[1] & 0xffffffffull) | (w[2] << 32)));
+        }
+        __syncthreads();
+    }
+    if (tid < 64) {
+        float mx = 0.0f;
+        double sm = 0.0;
+        constexpr int kPer = kRowsPerGroup / kRowsOfBlock;
+        if (measured && tid * kPer < ny) {        // one row group per lane, its sum as merge_group stores it
+            double wsum[kPer / 2];
+#pragma unroll
+            for (int b = 0; b < kPer; ++b) {
+                const int k = tid * kPer + b;
+                const double v = k < ny ? lds_sm[k] : 0.0;
+                wsum[b / 2] = b % 2 == 0 ? v : wsum[b / 2] + v;
+                if (k < ny) mx = fmaxf(mx, lds_mx[k]);
+            }
+            double s = wsum[0];
+#pragma unroll
+            for (int b = 1; b < kPer / 2; ++b) s += wsum[b];
+            sm = (double)(float)s;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            mx = fmaxf(mx, __shfl_xor(mx, o));
+            sm += __shfl_xor(sm, o);
+        }
+        if (tid == 0) {
+            sk_state& st = ctl.st;
+            const LoopCfg& cfg = g.cfg;
+            int stage = st.stage, stage_it = st.stage_it, conv = 0;
+            double err;
+            if (control_decide(cfg, st.it, st.sc_x[1], mx, sm, stage, stage_it, conv, err)) {
+                st.err = err;
+                st.checks += 1;
+            }
+            st.stage = stage;
+            st.stage_it = stage_it;
+            st.converged = conv;
+            st.done = conv != 0 || st.it >= cfg.max_iters ? 1 : 0;
+            if (st.done == 0) {
+                const float ran = st.sc_x[0];
+                set_scalars(&st, eps_for(cfg, st.it, stage), cfg.rho_x, cfg.rho_y);
+                if (st.sc_x[0] != ran) {          // a new eps: the copy for it, made by the next f update
+                    const BakeParams b = bake_params(g.yc, g.xr, st.sc_x);
+                    ctl.c = b.valid ? b.c : 0.0f;
+                    ctl.t = b.valid ? b.t : 1.0f;
+                    ctl.s2 = packed_scale(g.xr);
+                    ctl.pending = b.valid ? 1 : 0;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    return ctl.st.done != 0;
+}
+
+struct LoopArgs {
+    PartialArgs f, g;
+    u64 *ex, *ey, *msr;      // the potentials of x and y and the measures of y's row blocks, tagged words
+    int iters, polls;
+};
+
+template <int NC>
+__global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
+    constexpr int NT = 64 * loop_waves(NC);
+    __shared__ __attribute__((aligned(16))) bf16x8 cols[kLoopMaxTiles * 32];
+    __shared__ float2 slots[kLoopMaxTiles * kRowsOfBlock];      // a segment has a tile at least
+    __shared__ float lds_mx[kLoopMaxBlocks];
+    __shared__ double lds_sm[kLoopMaxBlocks];
+    __shared__ Ctl ctl;
+    const int w = wg_x(), tid = tid_x();
+    sk_state* gst = a.g.state;
+    if (gst->done != 0) return;
+    if (tid == 0) {
+        ctl.st = *gst;
+        const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
+        ctl.c = tag.c;
+        ctl.t = tag.t;
+        ctl.s2 = tag.s2;
+        ctl.pending = tag.pending;
+        ctl.polls = a.polls;
+        ctl.abort = 0;
+    }
+    const bool has_x = w < a.f.nrb, has_y = w < a.g.nrb;
+    const int i = w * kRowsOfBlock + tid;
+    const bool rx = has_x && tid < kRowsOfBlock, ry = has_y && tid < kRowsOfBlock;
+    const LoopCfg& cfg = a.g.cfg;
+    const float x2 = rx ? a.f.xsq[i] : 0.0f, xo = rx && a.f.off != nullptr ? a.f.off[i] : 0.0f, xl = rx ? a.f.rows_l2lo[i] : 0.0f;
+    const float y2 = ry ? a.g.xsq[i] : 0.0f, yo = ry && a.g.off != nullptr ? a.g.off[i] : 0.0f, yl = ry ? a.g.rows_l2lo[i] : 0.0f;
+    const float yw = ry ? a.g.w[i] : 0.0f;
+    float fh = rx ? a.f.out[i] : 0.0f, fr = rx ? a.f.out2[i] : 0.0f, gh = ry ? a.g.out[i] : 0.0f, gr = ry ? a.g.out2[i] : 0.0f;
+    __syncthreads();
+    unsigned ytag = 0u;                    // the tag of y's latest potentials (0: in memory)
+    bool done = false;
+    for (int k = 0; k < a.iters && !done; ++k) {
+        const unsigned tag = 2u * (unsigned)ctl.st.it + 1u;
+        float M = 0.0f, S = 1.0f;
+        // the f update
+        if (has_x) {
+            update<NC, 0>(a.f, a.ey, ytag, w, ctl, cols, slots, M, S);
+            if (rx && ctl.abort == 0) {
+                const float chs = ctl.st.sc_x[0] * kLog2e;
+                const bool l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.f.yc);
+                const Log2Split ls = lse_log2(S);
+                double R = 0.0;
+                fh = row_value({ctl.st.sc_x[2], ctl.st.sc_x[3], chs, x2, xo}, l2, true,
+                               (double)M + (l2 ? (double)loop_weight_offset(a.f.yc) : 0.0), (double)ls.e + (double)ls.lm, R);
+                if (l2) fr = (float)(R + (double)xl);
+                publish(a.ex + i, __float_as_uint(l2 ? fr : fh), tag);
+            }
+        }
+        __syncthreads();
+        if (ctl.abort != 0) break;
+        if (tid == 0) {
+            ctl.st.it += 1;
+            ctl.st.stage_it += 1;
+        }
+        __syncthreads();
+        // the g update
+        const bool need = needs_control(ctl.st.it, ctl.st.stage, ctl.st.stage_it, cfg);
+        const bool measured = need && (cfg.n_stages > 0 || (cfg.fixed_iters == 0 && ctl.st.it > cfg.n_sched));
+        float R32 = 0.0f;
+        bool l2 = false;
+        if (has_y) {
+            update<NC, 1>(a.g, a.ex, tag, w, ctl, cols, slots, M, S);
+            if (ry && ctl.abort == 0) {
+                const float chs = ctl.st.sc_y[0] * kLog2e;
+                l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.g.xr);
+                const Log2Split ls = lse_log2(S);
+                double R = 0.0;
+                const float old = gh;
+                gh = row_value({ctl.st.sc_y[2], ctl.st.sc_y[3], chs, y2, yo}, l2, true,
+                               (double)M + (l2 ? (double)loop_weight_offset(a.g.yc) : 0.0), (double)ls.e + (double)ls.lm, R);
+                R32 = (float)(R + (double)yl);
+                if (measured) {
+                    float dmax = i < a.g.n_real ? fabsf(gh - old) : 0.0f;
+                    const float delta = fminf((old - gh) * ctl.st.sc_y[1], kDeltaCap);
+                    double derr = (double)fabsf(yw * (expf(delta) - 1.0f));
+#pragma unroll
+                    for (int o = 16; o > 0; o >>= 1) {
+                        dmax = fmaxf(dmax, __shfl_xor(dmax, o));
+                        derr += __shfl_xor(derr, o);
+                    }
+                    if (tid == 0) {
+                        const u64 e = (u64)__double_as_longlong(derr);
+                        publish(a.msr + 3 * w, __float_as_uint(dmax), tag + 1u);
+                        publish(a.msr + 3 * w + 1, (unsigned)e, tag + 1u);
+                        publish(a.msr + 3 * w + 2, (unsigned)(e >> 32), tag + 1u);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (ctl.abort != 0) break;
+        if (tid == 0) ctl.pending = 0;                 // this iteration's f update has made the copy
+        const float ran = ctl.st.sc_x[0];
+        if (need) {
+            __syncthreads();
+            done = control<NT>(a.g, a.msr, tag + 1u, a.g.nrb, measured, ctl, lds_mx, lds_sm);
+            if (ctl.abort != 0) break;
+        }
+        if (ry) {
+            // y's potentials in the units of the next f update: at a new eps derived from gh, as the control does
+            if (!done && ctl.st.sc_x[0] != ran)
+                gr = (float)((double)gh * (0.5 * (double)(ctl.st.sc_x[0] * kLog2e)) + (double)yl);
+            else if (l2)
+                gr = R32;
+            const bool next_l2 = ctl.c != 0.0f && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(a.g.xr);
+            publish(a.ey + i, __float_as_uint(next_l2 ? gr : gh), tag + 1u);
+        }
+        ytag = tag + 1u;
+        __syncthreads();
+    }
+    if (rx) {
+        a.f.out[i] = fh;
+        a.f.out2[i] = fr;
+    }
+    if (ry) {
+        a.g.out[i] = gh;
+        a.g.out2[i] = gr;
+    }
+    // The state and the copy's header, once every workgroup has read them (they all have published y's last values, or
+    // x's that those rest on).
+    if (w == 0 && ctl.abort == 0) {
+        bool all = true;
+        for (int j = tid; j < a.g.nrb; j += NT) {
+            bool seen = false;
+            for (int r = 0; !seen && r < ctl.polls; ++r) seen = (unsigned)(peek(a.ey + j * kRowsOfBlock) >> 32) == ytag;
+            all = all && seen;
+        }
+        if (!all) ctl.abort = 1;
+    }
+    __syncthreads();
+    if (ctl.abort != 0) {
+        if (tid == 0) {
+            gst->checks = -1;
+            gst->converged = 0;
+            gst->done = 1;
+        }
+        return;
+    }
+    if (w == 0 && tid == 0) {
+        *gst = ctl.st;
+        float* h = reinterpret_cast<float*>(a.f.rebake);
+        const bool p = ctl.pending != 0;
+        h[2] = p ? 0.0f : ctl.c;
+        h[3] = ctl.s2;
+        if (!p) h[4] = ctl.t;
+        h[7] = ctl.c;
+        h[8] = ctl.t;
+        reinterpret_cast<int*>(h)[6] = p ? 1 : 0;
+    }
+}
+
+template <int NC>
+hipError_t launch_nc(const LoopArgs& a, int workgroups, hipStream_t st) {
+    LoopArgs args = a;
+    void* params[] = {&args};
+    return hipLaunchCooperativeKernel(loop_kernel<NC>, dim3(workgroups), dim3(64 * loop_waves(NC)), params, 0, st);
+}
+
+}  // namespace
+
+hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int polls, hipStream_t st) {
+    LoopArgs a;
+    a.f = f;
+    a.g = g;
+    a.ex = (u64*)exchange;
+    a.ey = a.ex + f.rows_pad;
+    a.msr = a.ey + g.rows_pad;
+    a.iters = iters;
+    a.polls = polls > 0 ? polls : kMaxPolls;
+    const int wgs = f.nrb > g.nrb ? f.nrb : g.nrb;
+    switch (nc) {
+        case 1: return launch_nc<1>(a, wgs, st);
+        case 2: return launch_nc<2>(a, wgs, st);
+        case 3: return launch_nc<3>(a, wgs, st);
+        case 4: return launch_nc<4>(a, wgs, st);
+        case 5: return launch_nc<5>(a, wgs, st);
+        case 6: return launch_nc<6>(a, wgs, st);
+        case 7: return launch_nc<7>(a, wgs, st);
+        case 8: return launch_nc<8>(a, wgs, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace sk

@@ -40,6 +40,7 @@ UNITS = [   # (source, object name, extra flags)
                                                     "-mllvm", "-amdgpu-mfma-vgpr-form"]),
     ("sk_lse_partial.hip", "sk_lse_partial_large", ["-fno-honor-nans", "-mno-amdgpu-ieee", "-DSK_PARTIAL_LARGE=1",
                                                     "-mllvm", "-amdgpu-mfma-vgpr-form"]),
+    ("sk_loop.hip", "sk_loop", ["-fno-honor-nans", "-mno-amdgpu-ieee", "-mllvm", "-amdgpu-mfma-vgpr-form"]),
     ("sk_kernels.hip", "sk_kernels", []),
     ("sk_median.hip", "sk_median", []),
     ("sk_prepare.hip", "sk_prepare", []),
