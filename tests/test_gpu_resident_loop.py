@@ -1,7 +1,7 @@
 """The loop of small problems as one resident launch (sk_loop_run_resident_f32 wherever it fits, TRNOPT_HIP_LOOP=1) against
 the launch-by-launch loop: potentials, iteration counts, errors and convergence bit for bit, over the forms the loop has
 (fixed, to convergence, eps schedule, stages, unbalanced with targets, weights), sizes at the edges of the 32-row blocks,
-256-row groups and its largest (192 tiles), every width of kernel, calls of several lengths, and clouds without a
+256-row groups and its largest (192 tiles), every width of kernel, one to four workgroups per row block, calls of several lengths, and clouds without a
 log2-unit copy; and from several streams and threads."""
 
 import numpy as np
@@ -49,14 +49,15 @@ def _same(p, q):
 
 
 @pytest.mark.parametrize("form", list(FORMS))
-@pytest.mark.parametrize("n,m,d", [(137, 91, 5), (700, 900, 30), (257, 31, 64)])
+@pytest.mark.parametrize("n,m,d", [(137, 91, 5), (700, 900, 30), (257, 31, 64), (1300, 400, 40)])
 def test_every_form_bit_for_bit(hip, monkeypatch, form, n, m, d):
     print(f"resident {form} {n} x {m} d {d}", flush=True)
     _same(*_both(monkeypatch, n, m, d, FORMS[form]))
 
 
 @pytest.mark.parametrize("n,m,d", [(1, 1, 1), (31, 33, 16), (32, 32, 17), (33, 1, 40), (255, 256, 48), (256, 257, 80),
-                                   (513, 100, 96), (64, 6144, 8), (6144, 64, 112), (6144, 6100, 33), (2000, 1900, 128)])
+                                   (513, 100, 96), (64, 6144, 8), (6144, 64, 112), (6144, 6100, 33), (2000, 1900, 128),
+                                   (2700, 2600, 40), (4000, 3900, 20), (280, 4096, 64)])
 def test_sizes_bit_for_bit(hip, monkeypatch, n, m, d):
     print(f"resident {n} x {m} d {d}", flush=True)
     _same(*_both(monkeypatch, n, m, d, dict(eps=0.3, max_iters=5, fixed_iters=True)))

@@ -220,8 +220,14 @@ int hip_fail(hipError_t e, const char* where);
 // row blocks (one workgroup each, all resident) and kLoopMaxTiles tiles. exchange: loop_exchange_words 8-byte words, zero at
 // loop init.
 constexpr int kLoopMaxTiles = 192, kLoopMaxBlocks = 256;
-inline size_t loop_exchange_words(int nx_pad, int ny_pad) { return (size_t)nx_pad + ny_pad + 3 * (size_t)(ny_pad / 32); }
-hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int polls, hipStream_t stream);
+inline size_t loop_exchange_words(int nx_pad, int ny_pad, int slots_x, int slots_y) {
+    return (size_t)nx_pad * (1 + 2 * slots_x) + (size_t)ny_pad * (1 + 2 * slots_y) + 6 * (size_t)(ny_pad / 32);
+}
+// Waves of a workgroup: as many as hide each other's latencies with the operands in registers (128, 168, 256 a lane).
+constexpr int loop_waves(int nc) { return nc <= 2 ? 16 : nc <= 4 ? 12 : 8; }
+// ranks: workgroups that share a row block; slots_x, slots_y: the most segments of one, for ranks > 1 (else 0).
+hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int ranks, int slots_x,
+                       int slots_y, int polls, hipStream_t stream);
 hipError_t launch_partial_small(const PartialArgs& a, int nc, hipStream_t stream);
 hipError_t launch_partial_large(const PartialArgs& a, int nc, hipStream_t stream);
 inline hipError_t launch_partial(const PartialArgs& a, int nc, hipStream_t stream) {

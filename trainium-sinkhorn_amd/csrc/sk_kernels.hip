@@ -543,22 +543,39 @@ bool fused_merge(const Plan& pl) {
     return v < 0 ? pl.ngroups >= kFuseMinGroups : v != 0;
 }
 
-// Whether the loop's one-launch form (sk_loop.hip) can take a problem, and whether it is the faster one. Its update costs
-// 5 us plus the tiles of one row block on one CU, 16 waves and fewer in the wider kernels; the launches' 7-8 us plus the
-// tiles spread over every CU. Measured (us an iteration, launches against one launch of 10 iterations): 100 x 90 d 5
-// 14.5 / 10.0, 700 x 500 d 16 17.0 / 12.1, 1,500 x 1,400 d 16 20.4 / 16.2, d 30 20.9 / 18.5, 3,000 x 3,100 d 16 21.3 / 18.5;
-// 700 x 500 d 64 18.8 / 16.5, 300 x 280 d 128 19.7 / 17.9; past the line 2,048 x 2,048 d 30 19.1 / 19.8, 1,500 x 1,400 d 64
-// 22.5 / 23.2, 700 x 500 d 128 21.1 / 22.1, 4,500 x 4,600 d 5 23.7 / 23.9. TRNOPT_HIP_LOOP=0 turns it off, =1 takes it
-// wherever it fits.
-constexpr int kLoopMaxChunkTiles = 96;
+// Whether the loop's one-launch form (sk_loop.hip) can take a problem.
 bool loop_fits(const Plan& pf, const Plan& pg) {
     return pf.ok && pg.ok && pf.nt <= kLoopMaxTiles && pg.nt <= kLoopMaxTiles &&
            std::max(pf.nrb, pg.nrb) <= std::min(kLoopMaxBlocks, cu_count());
 }
+
+// Its workgroups per row block: up to 4 where they have CUs; one for up to kLoopLoneTiles tiles, which the waves of one take
+// at once. us an iteration by ranks 1 / 2 / 4 / 8: 100 x 90 d 30 11.5 / 12.7 / 12.5 / 12.3, 300 x 280 13.0 / 13.3 / 12.7 / 12.6,
+// 700 x 500 14.6 / 14.0 / 13.6 / 13.4, 1,000 x 1,000 d 64 19.7 / 18.1 / 17.4 / 17.4, 2,048 x 2,048 d 64 27.1 / 22.6 / 19.3.
+constexpr int kLoopMaxRanks = 4, kLoopLoneTiles = 8;
+int loop_ranks(const Plan& pf, const Plan& pg) {
+    if (std::max(pf.nt, pg.nt) <= kLoopLoneTiles) return 1;
+    return std::max(1, std::min(kLoopMaxRanks, std::min(cu_count(), kLoopMaxBlocks) / std::max(pf.nrb, pg.nrb)));
+}
+
+size_t loop_words(const Plan& pf, const Plan& pg) {
+    const bool shared = loop_ranks(pf, pg) > 1;
+    return loop_exchange_words(pf.nrb * SK_TILE, pg.nrb * SK_TILE, shared ? pf.slots : 0, shared ? pg.slots : 0);
+}
+
+// And whether it is the faster one: an update costs it 5 to 7 us plus the tiles of a row block on `ranks` CUs, the launches
+// 7-8 us plus the tiles spread over every CU. The line is tiles x 16-wide chunks per wave of a row block's workgroups. Measured
+// (us an iteration, launches against one launch of 10 iterations): 100 x 90 d 5 13.6 / 9.8, 700 x 500 d 16 17.0 / 11.7, d 64
+// 18.9 / 15.6, d 128 21.2 / 18.5, 2,048 x 2,048 d 16 18.3 / 13.9, d 30 19.0 / 16.0, d 64 21.1 / 19.1, 4,096 x 4,096 d 30 23.4 /
+// 21.1, 300 x 4,096 24.1 / 21.7; at the line 2,300 x 2,300 d 64 21.4 / 21.4; past it 3,000 x 3,000 d 64 24.0 / 25.5,
+// 4,300 x 4,300 d 30 24.2 / 26.7, 1,300 x 1,300 d 128 25.0 / 25.3. TRNOPT_HIP_LOOP=0 turns it off, =1 takes it wherever it fits.
+constexpr int kLoopMaxWaveChunks = 8;
 bool loop_persists(const Plan& pf, const Plan& pg) {
     const int v = env_int("TRNOPT_HIP_LOOP", -1);
-    return v < 0 ? pf.nc * std::max(pf.nt, pg.nt) <= kLoopMaxChunkTiles : v != 0;
+    if (v >= 0) return v != 0;
+    return pf.nc * std::max(pf.nt, pg.nt) <= kLoopMaxWaveChunks * loop_ranks(pf, pg) * loop_waves(pf.nc);
 }
+
 bool capturing(hipStream_t st) {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
@@ -826,7 +843,7 @@ size_t sk_loop_workspace_bytes(int nx_pad, int ny_pad, int d) {
            align_up((size_t)meas_count(ny_pad) * sizeof(float2)) +
            align_up((size_t)(1 + std::max(pf.ngroups, pg.ngroups)) * sizeof(int)) +
            3 * (align_up((size_t)nx_pad * sizeof(float)) + align_up((size_t)ny_pad * sizeof(float))) +
-           (loop_fits(pf, pg) ? align_up(loop_exchange_words(nx_pad, ny_pad) * 8) : 0);
+           (loop_fits(pf, pg) ? align_up(loop_words(pf, pg) * 8) : 0);
 }
 
 namespace {
@@ -867,7 +884,7 @@ LoopLayout loop_layout(const sk_loop_f32* L) {
     o.lyl = (float*)((char*)o.lyh + by);
     const bool fits = loop_fits(o.pf, o.pg);
     o.exchange = fits ? (unsigned long long*)((char*)o.lyl + by) : nullptr;
-    o.nexchange = fits ? (int)loop_exchange_words(L->x.npad, L->y.npad) : 0;
+    o.nexchange = fits ? (int)loop_words(o.pf, o.pg) : 0;
     return o;
 }
 }  // namespace
@@ -886,7 +903,7 @@ int sk_loop_init_f32(const sk_loop_f32* L, void* stream) {
     if (L->ws_bytes < need) return fail(SK_E_WORKSPACE, "sk_loop_init_f32: workspace %zu < %zu bytes", L->ws_bytes, need);
     if (((uintptr_t)L->ws & 255) != 0) return fail(SK_E_ARG, "sk_loop_init_f32: workspace must be 256-byte aligned");
     const LoopLayout lo = loop_layout(L);
-    hipLaunchKernelGGL(loop_init_kernel, dim3(lo.exchange != nullptr ? 16 : 1), dim3(256), 0, (hipStream_t)stream, L->state,
+    hipLaunchKernelGGL(loop_init_kernel, dim3(std::min(std::max(1, lo.nexchange / 1024), 256)), dim3(256), 0, (hipStream_t)stream, L->state,
                        loop_cfg(L), lo.counters, lo.ncounters, lo.exchange, lo.nexchange);
     // both clouds' log2 weight offsets into their headers (each is the column cloud of one half-step)
     hipLaunchKernelGGL(weight_offset_kernel, dim3(1), dim3(kWeightMaxThreads), 0, (hipStream_t)stream, L->x.log_w,
@@ -1018,10 +1035,11 @@ int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream) {
     if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_resident_f32: iters %d < 0", iters);
     if (iters < 2 || sk_loop_resident(L) == 0 || capturing((hipStream_t)stream)) return sk_loop_run_f32(L, iters, stream);
     const LoopLayout lo = loop_layout(L);
+    const int ranks = loop_ranks(lo.pf, lo.pg);
     Pass f, g;
     loop_passes(L, lo, f, g);
-    const hipError_t e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc,
-                                    env_int("TRNOPT_HIP_LOOP_POLLS", 0), (hipStream_t)stream);
+    const hipError_t e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc, ranks, ranks > 1 ? lo.pf.slots : 0,
+                                    ranks > 1 ? lo.pg.slots : 0, env_int("TRNOPT_HIP_LOOP_POLLS", 0), (hipStream_t)stream);
     return e == hipSuccess ? SK_OK : hip_fail(e, "sk_loop_run_resident_f32");
 }
 

@@ -6,8 +6,8 @@
 // potentials and the arguments pass between them through memory. Here one workgroup per 32-row block of x and of y
 // stays for all the iterations; all that passes between workgroups is the new potentials, each as one 8-byte word
 // {value, iteration tag} that its readers poll: the data is its own flag, so an exchange costs one store and one load
-// across the XCDs and no barrier, fence or counter. 700 x 500 d 16: 17.0 -> 12.1 us an iteration, 100 x 90 d 5 14.5 -> 10.0
-// (launches of 10 iterations; loop_persists has more sizes and both sides of its line).
+// across the XCDs and no barrier, fence or counter. 700 x 500 d 5: 16.9 -> 11.6 us an iteration, 100 x 90 14.5 -> 10.0,
+// 2,048 x 2,048 d 64 21.0 -> 19.3 (launches of 10 iterations; loop_persists has more sizes and both sides of its line).
 //
 // Bit for bit the launch-by-launch loop: a row block's columns are summed in the same segments as the split of the
 // partial kernel gives its row group (Split), each segment by one wave with the same instructions (sk_tile.h), and a
@@ -17,6 +17,9 @@
 // Every wait ends: the launch is cooperative (all its workgroups are resident), and a poll that has not seen its word after
 // `polls` rounds gives up: its workgroup ends without publishing, so that every other one's polls end the same way, and the
 // state says so (checks = -1, done); the host then runs the loop again in launches.
+//
+// Where CUs would be idle, `ranks` workgroups share a row block: each takes every ranks-th segment, and rank 0 merges them all,
+// one exchange more and a ranks-th of the tiles (2,048 x 2,048 d 64, us an iteration: one rank 27.1, two 22.6, four 19.3).
 //
 // A potential's word is overwritten only after every reader has it: the next iteration's value is published by a
 // workgroup that has read all of the other cloud's values, each published by a workgroup that had read all of this one's.
@@ -30,8 +33,6 @@ namespace {
 
 constexpr int kMaxPolls = 1 << 20;                  // of a word before a workgroup gives up: about a second
 constexpr int kRowsOfBlock = 32;
-// Waves of a workgroup: as many as hide each other's latencies with the operands in registers (128, 168, 256 a lane).
-constexpr int loop_waves(int nc) { return nc <= 2 ? 16 : nc <= 4 ? 12 : 8; }
 
 typedef unsigned long long u64;
 
@@ -45,8 +46,17 @@ struct Ctl {
     sk_state st;          // this workgroup's copy
     float c, t, s2;       // the log2-unit copy: its score scale (0: none), unit, and the second cloud's scale
     int pending;          // its tiles are to be made by this iteration's f update
+    int unseen;           // this launch has remade them without this workgroup waiting for it: it makes its rows itself
     int polls;            // rounds before a poll gives up,
     int abort;            // and whether one has
+};
+
+// This workgroup's place among the `of` workgroups that share a row block: segment s of the block is rank s % of's. The
+// others' (M, S) reach rank 0, which merges and publishes the block, as two tagged words per row and segment.
+struct Rank {
+    int rank, of;
+    u64* slots;           // of this row block: (segment, row, {M, S})
+    unsigned tag;
 };
 
 // The tile loop of one segment, the rows' operands in xv, the first tile's in yv (load_y(t) requests tile t's): (M, S) per
@@ -79,7 +89,7 @@ __device__ __forceinline__ void segment(const f16x8 (&xv)[NC][2], f16x8 (&yv)[NC
 // One update: rows of block rb (ROLE 0: x, 1: y) against the other cloud. Fills the merged maximum and sum of row tid for
 // tid < 32. expect: the tag of the column potentials (0: the launch's first f update, which takes them from memory).
 template <int NC, int ROLE>
-__device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsigned expect, int rb, Ctl& ctl, bf16x8* cols,
+__device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsigned expect, int rb, const Rank& rk, Ctl& ctl, bf16x8* cols,
                                        float2* slots, float& Mr, float& Sr) {
     constexpr int W = loop_waves(NC), NT = 64 * W, TILE16 = NC * 2 * 64;
     const int tid = tid_x(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -93,7 +103,7 @@ __device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsi
 #pragma unroll
     for (int k = 0; k < NC * 2; ++k) xv[k / 2][k % 2] = xt[(size_t)rb * TILE16 + k * 64 + lane];
     const bool remake = l2 && ctl.pending != 0;          // this iteration's f update makes x's log2-unit copy
-    if (ROLE == 0 && remake) {
+    if (ROLE == 0 && (remake || (l2 && ctl.unseen != 0))) {
         const BakeParams bp = bake_params(a.xr, a.yc, sc);
         const f16x8* own = packed_tiles<f16x8>(a.xr);
 #pragma unroll
@@ -112,7 +122,8 @@ __device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsi
         te = (q1 < hi ? q1 : hi) - lo;
     };
     int tb = 0, te = 0;
-    if (wave < ns) bounds(wave, tb, te);
+    const int s0 = wave * rk.of + rk.rank, step = W * rk.of;
+    if (s0 < ns) bounds(s0, tb, te);
     f16x8 yv[NC][2];
     auto load_y = [&](int q) {
         const f16x8* b0 = yt + (size_t)q * TILE16;
@@ -159,11 +170,12 @@ __device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsi
         }
     }
     __syncthreads();
+    if (rk.rank != 0 && ctl.abort != 0) return;          // publish nothing (rank 0's caller looks)
     if (remake) {
         if (ROLE == 0) {
             // The copy's tiles of this row block, now that every y workgroup has published, i.e. is done with the old copy;
             // out of this XCD's L2 before the rows' potentials are published (by the same wave).
-            if (wave == 0) {
+            if (wave == 0 && rk.rank == 0) {
                 f16x8* copy = const_cast<f16x8*>(xt) + (size_t)rb * TILE16;
 #pragma unroll
                 for (int k = 0; k < NC * 2; ++k) copy[k * 64 + lane] = xv[k / 2][k % 2];
@@ -175,24 +187,46 @@ __device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsi
         }
     }
     const bf16x8 ones = column_ones(lane >> 5);
-    for (int s = wave; s < ns; s += W) {
+    for (int s = s0; s < ns; s += step) {
         float M, S;
         if (l2)
             segment<NC, ROLE, true>(xv, yv, load_y, cols, ones, lane, tb, te, c, M, S);
         else
             segment<NC, ROLE, false>(xv, yv, load_y, cols, ones, lane, tb, te, c, M, S);
-        if (s + W < ns) {
-            bounds(s + W, tb, te);
+        if (s + step < ns) {
+            bounds(s + step, tb, te);
             load_y(tb);
         }
         // as store_rows
         const float Mo = __shfl_xor(M, 32), So = __shfl_xor(S, 32);
         const float Mn = fmaxf(M, Mo);
         const float Sn = S * ex2(c * (M - Mn)) + So * ex2(c * (Mo - Mn));
-        if (lane < 32) slots[s * kRowsOfBlock + lane] = make_float2(fmaxf(Mn * inv_sigma, kEmpty), Sn);
+        const float2 v = make_float2(fmaxf(Mn * inv_sigma, kEmpty), Sn);
+        if (lane < 32) {
+            if (rk.rank == 0) {
+                slots[s * kRowsOfBlock + lane] = v;
+            } else {
+                u64* dst = rk.slots + 2 * (size_t)(s * kRowsOfBlock + lane);
+                publish(dst, __float_as_uint(v.x), rk.tag);
+                publish(dst + 1, __float_as_uint(v.y), rk.tag);
+            }
+        }
     }
+    if (rk.rank == 0 && rk.of > 1)
+        for (int k = tid; k < ns * kRowsOfBlock; k += NT) {
+            if (k / kRowsOfBlock % rk.of == 0) continue;
+            u64 m = 0, q = 0;
+            bool all = false;
+            for (int r = 0; !all && r < ctl.polls; ++r) {
+                m = peek(rk.slots + 2 * (size_t)k);
+                q = peek(rk.slots + 2 * (size_t)k + 1);
+                all = (unsigned)(m >> 32) == rk.tag && (unsigned)(q >> 32) == rk.tag;
+            }
+            if (!all) ctl.abort = 1;
+            slots[k] = make_float2(__uint_as_float((unsigned)m), __uint_as_float((unsigned)q));
+        }
     __syncthreads();
-    if (tid < kRowsOfBlock) {
+    if (rk.rank == 0 && tid < kRowsOfBlock) {
         // as merge_group
         const float cm = l2 ? 1.0f : chs;
         float M = kEmpty, S = 0.0f;
@@ -292,8 +326,10 @@ __device__ inline bool control(const PartialArgs& g, const u64* msr, unsigned ta
 
 struct LoopArgs {
     PartialArgs f, g;
-    u64 *ex, *ey, *msr;      // the potentials of x and y and the measures of y's row blocks, tagged words
-    int iters, polls;
+    u64 *ex, *ey, *msr;      // the potentials of x and y and (two turns of) the measures of y's row blocks, tagged words
+    u64 *sx, *sy;            // the segments' (M, S) of the ranks above 0 (Rank)
+    int iters, polls, ranks;
+    int slots_x, slots_y;    // segments of a row block, at most
 };
 
 template <int NC>
@@ -304,7 +340,16 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     __shared__ float lds_mx[kLoopMaxBlocks];
     __shared__ double lds_sm[kLoopMaxBlocks];
     __shared__ Ctl ctl;
-    const int w = wg_x(), tid = tid_x();
+    const int tid = tid_x(), rank = wg_x() % a.ranks, w = wg_x() / a.ranks;
+    // Row blocks this workgroup has segments of: without any in a pass it takes no part in it.
+    auto segments = [&](const PartialArgs& p) {
+        if (w >= p.nrb) return 0;
+        const int g = w / (kRowsPerGroup / kRowsOfBlock);
+        return last_wg(g, p.s) - first_wg(g, p.s) + 1;
+    };
+    const int nsx = segments(a.f), nsy = segments(a.g);
+    const bool has_x = rank < nsx, has_y = rank < nsy;
+    if (!has_x && !has_y) return;
     sk_state* gst = a.g.state;
     if (gst->done != 0) return;
     if (tid == 0) {
@@ -314,12 +359,14 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         ctl.t = tag.t;
         ctl.s2 = tag.s2;
         ctl.pending = tag.pending;
+        ctl.unseen = 0;
         ctl.polls = a.polls;
         ctl.abort = 0;
     }
-    const bool has_x = w < a.f.nrb, has_y = w < a.g.nrb;
     const int i = w * kRowsOfBlock + tid;
-    const bool rx = has_x && tid < kRowsOfBlock, ry = has_y && tid < kRowsOfBlock;
+    const bool rx = has_x && rank == 0 && tid < kRowsOfBlock, ry = has_y && rank == 0 && tid < kRowsOfBlock;
+    u64* const sx = a.sx + (size_t)w * a.slots_x * kRowsOfBlock * 2;
+    u64* const sy = a.sy + (size_t)w * a.slots_y * kRowsOfBlock * 2;
     const LoopCfg& cfg = a.g.cfg;
     const float x2 = rx ? a.f.xsq[i] : 0.0f, xo = rx && a.f.off != nullptr ? a.f.off[i] : 0.0f, xl = rx ? a.f.rows_l2lo[i] : 0.0f;
     const float y2 = ry ? a.g.xsq[i] : 0.0f, yo = ry && a.g.off != nullptr ? a.g.off[i] : 0.0f, yl = ry ? a.g.rows_l2lo[i] : 0.0f;
@@ -333,7 +380,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         float M = 0.0f, S = 1.0f;
         // the f update
         if (has_x) {
-            update<NC, 0>(a.f, a.ey, ytag, w, ctl, cols, slots, M, S);
+            update<NC, 0>(a.f, a.ey, ytag, w, {rank, a.ranks, sx, tag}, ctl, cols, slots, M, S);
             if (rx && ctl.abort == 0) {
                 const float chs = ctl.st.sc_x[0] * kLog2e;
                 const bool l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.f.yc);
@@ -354,11 +401,12 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         __syncthreads();
         // the g update
         const bool need = needs_control(ctl.st.it, ctl.st.stage, ctl.st.stage_it, cfg);
+        u64* const msr = a.msr + 3 * (size_t)a.g.nrb * (ctl.st.it & 1);
         const bool measured = need && (cfg.n_stages > 0 || (cfg.fixed_iters == 0 && ctl.st.it > cfg.n_sched));
         float R32 = 0.0f;
         bool l2 = false;
         if (has_y) {
-            update<NC, 1>(a.g, a.ex, tag, w, ctl, cols, slots, M, S);
+            update<NC, 1>(a.g, a.ex, tag, w, {rank, a.ranks, sy, tag}, ctl, cols, slots, M, S);
             if (ry && ctl.abort == 0) {
                 const float chs = ctl.st.sc_y[0] * kLog2e;
                 l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.g.xr);
@@ -379,20 +427,24 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
                     }
                     if (tid == 0) {
                         const u64 e = (u64)__double_as_longlong(derr);
-                        publish(a.msr + 3 * w, __float_as_uint(dmax), tag + 1u);
-                        publish(a.msr + 3 * w + 1, (unsigned)e, tag + 1u);
-                        publish(a.msr + 3 * w + 2, (unsigned)(e >> 32), tag + 1u);
+                        publish(msr + 3 * w, __float_as_uint(dmax), tag + 1u);
+                        publish(msr + 3 * w + 1, (unsigned)e, tag + 1u);
+                        publish(msr + 3 * w + 2, (unsigned)(e >> 32), tag + 1u);
                     }
                 }
             }
         }
         __syncthreads();
         if (ctl.abort != 0) break;
-        if (tid == 0) ctl.pending = 0;                 // this iteration's f update has made the copy
+        if (tid == 0) {
+            // This iteration's f update has made the copy: rank 0 its block's tiles itself, and a g update waits for all of them.
+            if (ctl.pending != 0 && rank != 0 && !has_y) ctl.unseen = 1;
+            ctl.pending = 0;
+        }
         const float ran = ctl.st.sc_x[0];
         if (need) {
             __syncthreads();
-            done = control<NT>(a.g, a.msr, tag + 1u, a.g.nrb, measured, ctl, lds_mx, lds_sm);
+            done = control<NT>(a.g, msr, tag + 1u, a.g.nrb, measured, ctl, lds_mx, lds_sm);
             if (ctl.abort != 0) break;
         }
         if (ry) {
@@ -417,7 +469,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     }
     // The state and the copy's header, once every workgroup has read them (they all have published y's last values, or
     // x's that those rest on).
-    if (w == 0 && ctl.abort == 0) {
+    if (w == 0 && rank == 0 && ctl.abort == 0) {
         bool all = true;
         for (int j = tid; j < a.g.nrb; j += NT) {
             bool seen = false;
@@ -435,7 +487,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         }
         return;
     }
-    if (w == 0 && tid == 0) {
+    if (w == 0 && rank == 0 && tid == 0) {
         *gst = ctl.st;
         float* h = reinterpret_cast<float*>(a.f.rebake);
         const bool p = ctl.pending != 0;
@@ -457,16 +509,22 @@ hipError_t launch_nc(const LoopArgs& a, int workgroups, hipStream_t st) {
 
 }  // namespace
 
-hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int polls, hipStream_t st) {
+hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int ranks, int slots_x,
+                       int slots_y, int polls, hipStream_t st) {
     LoopArgs a;
     a.f = f;
     a.g = g;
     a.ex = (u64*)exchange;
     a.ey = a.ex + f.rows_pad;
     a.msr = a.ey + g.rows_pad;
+    a.sx = a.msr + 6 * (size_t)g.nrb;
+    a.sy = a.sx + (size_t)f.nrb * slots_x * kRowsOfBlock * 2;
+    a.slots_x = slots_x;
+    a.slots_y = slots_y;
+    a.ranks = ranks;
     a.iters = iters;
     a.polls = polls > 0 ? polls : kMaxPolls;
-    const int wgs = f.nrb > g.nrb ? f.nrb : g.nrb;
+    const int wgs = (f.nrb > g.nrb ? f.nrb : g.nrb) * ranks;
     switch (nc) {
         case 1: return launch_nc<1>(a, wgs, st);
         case 2: return launch_nc<2>(a, wgs, st);
