@@ -220,12 +220,12 @@ int sk_loop_init_f32(const sk_loop_f32* L, void* stream);
  * below that);
  * iterations after `done` do nothing. ws (sk_loop_workspace_bytes) must be 256-byte aligned. */
 int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream);
-/* The same iterations, bit for bit; where the problem is small (sk_kernels.hip, loop_persists) as one cooperative launch
- * whose workgroups stay for all of them and pass the potentials to one another directly, else (and while the stream
- * captures) as sk_loop_run_f32. Cooperative launches of one device run one after another: for a caller whose loops share
- * the GPU on several streams sk_loop_run_f32 is the better form. If the workgroups should not all get to run, the loop
- * gives up after about a second: state done with checks = -1, for the caller to start again with sk_loop_run_f32.
- * sk_loop_resident: 1 where it would be the one launch, else 0. */
+/* The same iterations, bit for bit; where the problem is small (sk_loop_resident returns 1; else 0) as one cooperative
+ * launch whose workgroups stay for all of them and pass the potentials to one another directly, else (and while the stream
+ * captures, and for a single iteration) as sk_loop_run_f32. Cooperative launches of one device run one after another: for
+ * a caller whose loops share the GPU on several streams sk_loop_run_f32 is the better form. If the workgroups should not
+ * all get to run, the loop gives up after about a second: state done with checks = -1, for the caller to start again with
+ * sk_loop_init_f32 and sk_loop_run_f32. */
 int sk_loop_resident(const sk_loop_f32* L);
 int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream);
 

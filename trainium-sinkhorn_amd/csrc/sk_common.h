@@ -189,7 +189,6 @@ struct PartialArgs {
     float* out;         // merged result (fh, or the plain row-LSE)
     float* out2;        // or null: with log2-unit scores, also the result in log2 units, (c / 2) fh + Ll
     const float* rows_l2lo;   // with out2: the rows' Ll (the low part of their log2 weights)
-    const float* cols_l2lo;   // with out2 and rebake: the columns' Ll
     int n_store;        // rows of out written
     float2* meas;       // per-group convergence partials (g update of the loop), or null
     const float* w;     // row weights, with meas

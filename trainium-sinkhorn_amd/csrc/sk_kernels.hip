@@ -428,7 +428,6 @@ struct Pass {
     float* out;
     float* out2;    // the rows' log2-unit potential + Ll (on-device loop), or null
     const float* rows_l2lo;   // with out2: the rows' Ll
-    const float* cols_l2lo;   // with out2: the columns' Ll
     int n_store;
     float2* meas;
     const float* w;
@@ -465,7 +464,6 @@ PartialArgs pass_args(const Pass& ps, const Plan& pl) {
     a.out = ps.out;
     a.out2 = ps.out2;
     a.rows_l2lo = ps.rows_l2lo;
-    a.cols_l2lo = ps.cols_l2lo;
     a.n_store = ps.n_store;
     a.meas = ps.meas;
     a.w = ps.w;
@@ -952,7 +950,6 @@ void loop_passes(const sk_loop_f32* L, const LoopLayout& lo, Pass& f, Pass& g) {
     f.out = L->fh;
     f.out2 = lo.rf;
     f.rows_l2lo = lo.lxl;
-    f.cols_l2lo = lo.lyl;
     f.n_store = L->x.npad;
     f.tick = st;
     f.rebake = log2_enabled() ? (char*)const_cast<void*>(L->x.pk) : nullptr;
@@ -979,7 +976,6 @@ void loop_passes(const sk_loop_f32* L, const LoopLayout& lo, Pass& f, Pass& g) {
     g.out = L->gh;
     g.out2 = lo.rg;
     g.rows_l2lo = lo.lyl;
-    g.cols_l2lo = lo.lxl;
     g.n_store = L->y.npad;
     g.meas = lo.meas;
     g.w = L->y.w;

@@ -444,6 +444,10 @@ class DeviceLoop:
     `done` return at once, so the host enqueues batches and reads the 72-byte state once per batch, with the
     next batch already queued behind it (no per-iteration synchronisation).
 
+    On the default stream a small loop (sk_loop_resident) runs each call's iterations as one resident launch instead, bit
+    for bit the same; on any other stream the caller may have more loops in flight, which resident launches would run one
+    after another.
+
     With TRNOPT_HIP_GRAPH=1, whole batches of GRAPH_BATCH iterations are replayed from one captured HIP graph
     (20 to 40 kernels, no memset nodes): fewer host calls, for callers whose host enqueue is the bottleneck. Graph
     and eager launches run the same kernels with the same arguments, so the results are bit-identical. The
@@ -490,8 +494,6 @@ class DeviceLoop:
         self._graph = None
 
     def init(self) -> None:
-        # On the default stream small loops run as resident launches (bit for bit the same iterations); on any other
-        # the caller may have more loops in flight, which resident launches would run one after another.
         self._queued, self._g0 = 0, None
         if _stream() == 0 and lib().sk_loop_resident(ctypes.byref(self._L)):
             self._g0 = self.gh.clone()        # to start again from, should a resident launch give up
