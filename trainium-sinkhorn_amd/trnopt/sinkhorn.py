@@ -357,8 +357,11 @@ def normalization(x: np.ndarray, y: np.ndarray, samples: int = 20_000, seed: int
 
 
 def _median_enqueue(x, y, center, device) -> torch.Tensor:
-    """The exact median cost on the GPU, enqueued: the points copied as they are, the centre taken off there."""
+    """The exact median cost on the GPU, enqueued: the points copied as they are, the centre taken off there. Points of up to
+    a quarter megabyte are centred here: that takes less than the centre's copy and the two launches (about 25 us)."""
     from . import hip_sinkhorn as hk
+    if x.size + y.size <= 32_768:
+        return hk.cost_median_enqueue(x - center, y - center, device)
     c = hk.to_device_f64(center, device)
     out = torch.empty(1, dtype=torch.float64, device=c.device)
     hk.cost_median_device(hk.centred(hk.to_device_f64(x, device), c), hk.centred(hk.to_device_f64(y, device), c), out)
