@@ -195,18 +195,14 @@ def _hip_setup(p, opts: SinkhornOptions, dev, state=None):
     (the centre and the typical cost too, unless the options give them), both clouds packed, the loop set up (not
     run). Sets p.center and p.scale, and refuses points out of range, with one read-back."""
     from . import hip_sinkhorn as hk
-    d = p.x.shape[1]
     px, py, center, scale = p.x, p.y, p.center, p.scale
-    if p.how is None:
-        if center.size == d or center.size == 1:
-            center = np.broadcast_to(center.reshape(-1), (d,))
-        else:                                # a centre per point, or the like: normalised on the host
-            px, py = (px - center) / np.sqrt(scale), (py - center) / np.sqrt(scale)
-            center, scale = np.zeros(d), 1.0
+    if p.xs is not None:                     # normalised on the host (_prepare)
+        px, py, center, scale = p.xs, p.ys, np.zeros(()), 1.0
+    d = px.shape[1]
     Xd, Yd = hk.to_device_f64(px, dev), hk.to_device_f64(py, dev)
     stat = torch.empty(d + 3, dtype=torch.float64, device=dev)      # centre, cost scale, the clouds' largest |coordinate|
     if p.how is None:
-        stat[:d + 1] = torch.from_numpy(np.append(center, scale))
+        stat[:d + 1] = torch.from_numpy(np.append(np.broadcast_to(center.reshape(-1), (d,)), scale))
     elif p.how == "median":
         hk.cloud_stats(Xd, Yd, stat)
         med = stat[d:d + 1]
@@ -397,7 +393,9 @@ def _gpu_device(opts: SinkhornOptions):
 def _prepare(x, y, a, b, opts: SinkhornOptions, a_target, b_target, hip: bool = False):
     """Validation, weights, normalisation and the eps schedule (src/trnopt/sinkhorn.py:250-320, 340-344). With
     the HIP path selected the normalisation is left to _hip_setup (how: "mean" or "median"), unless the options give
-    it (how None: center and scale as they are) or its median is sampled on the host."""
+    it (how None: center and scale as they are) or its median is sampled on the host; a given centre that is not one
+    number or one per coordinate (by its shape: an (n, 1) column is one per point, also where n = d) is taken off here,
+    as numpy broadcasts it."""
     be = opts.backend
     x = np.asarray(x, dtype=np.float64)
     y = np.asarray(y, dtype=np.float64)
@@ -429,7 +427,8 @@ def _prepare(x, y, a, b, opts: SinkhornOptions, a_target, b_target, hip: bool = 
     else:
         center, scale = np.zeros(x.shape[1]), 1.0
     xs = ys = None
-    if not hip:
+    d = x.shape[1]
+    if not hip or (center is not None and center.shape not in ((), (1,), (d,), (1, 1), (1, d))):
         root = np.sqrt(scale)
         if np.any(center != 0.0) or root != 1.0:
             xs, ys = (x - center) / root, (y - center) / root
@@ -512,7 +511,7 @@ class _HipBatch:
                 raise ValueError("cores > 1 split rows across NeuronCores in the reference; this build runs on one GPU")
             p = _prepare(q["x"], q["y"], q.get("a"), q.get("b"), opts, q.get("a_target"), q.get("b_target"), True)
             prepared.append((p, opts))
-        if len({str(_gpu_device(o)) for _, o in prepared}) != 1 or len({p.x.shape[1] for p, _ in prepared}) != 1:
+        if len({str(_gpu_device(o)) for _, o in prepared}) != 1 or len({(p.x if p.xs is None else p.xs).shape[1] for p, _ in prepared}) != 1:
             raise ValueError("sinkhorn_batch: every problem must run on one device with one d")
         self.prepared = prepared
         self.dev = dev = _gpu_device(prepared[0][1])
