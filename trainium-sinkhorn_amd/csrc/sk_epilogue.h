@@ -432,7 +432,8 @@ __device__ inline void control_step(sk_state* st, const float2* meas, int nmeas,
 // The loop's state counters as a g update sees them on entry (before any workgroup can reach the control).
 struct LoopCounters {
     int it, stage, stage_it;
-    int pending;               // the copy was pending in this iteration (its f update has made the tiles)
+    int pending;               // this iteration's f update has made the pending copy's tiles: it was for this eps. (A copy
+                               // that another loop on the same clouds has still to make stays that loop's.)
 };
 __device__ inline LoopCounters loop_counters(const PartialArgs& a) {
     LoopCounters k = {0, 0, 0, 0};
@@ -440,7 +441,10 @@ __device__ inline LoopCounters loop_counters(const PartialArgs& a) {
         k.it = a.state->it;
         k.stage = a.state->stage;
         k.stage_it = a.state->stage_it;
-        if (a.rebake != nullptr) k.pending = reinterpret_cast<const int*>(a.rebake)[6];
+        if (a.rebake != nullptr) {
+            const CopyTag t = copy_tag(reinterpret_cast<const float*>(a.rebake), true);
+            k.pending = t.pending != 0 && t.c == a.sc[0] * kLog2e && t.s2 == packed_scale(a.xr) ? 1 : 0;
+        }
     }
     return k;
 }

@@ -437,9 +437,12 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         __syncthreads();
         if (ctl.abort != 0) break;
         if (tid == 0) {
-            // This iteration's f update has made the copy: rank 0 its block's tiles itself, and a g update waits for all of them.
-            if (ctl.pending != 0 && rank != 0 && !has_y) ctl.unseen = 1;
-            ctl.pending = 0;
+            // This iteration's f update has made a pending copy for its eps: rank 0 its block's tiles itself, and a g update
+            // waits for all of them. (Another eps: the copy of another loop on the same clouds, still pending.)
+            if (ctl.pending != 0 && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(a.f.yc)) {
+                if (rank != 0 && !has_y) ctl.unseen = 1;
+                ctl.pending = 0;
+            }
         }
         const float ran = ctl.st.sc_x[0];
         if (need) {
