@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 import torch
 
+from conftest import inf_rel
+
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
 KW = dict(rho_x=None, rho_y=None, tol=0.0, stage_tol=1e9, max_iters=40, check_every=1, stage_max_iters=1000, fixed_iters=True,
@@ -62,3 +64,31 @@ def test_the_header_says_what_the_tiles_are(hip, monkeypatch, n, m, d, form, ste
         for l in loops:
             l.enqueue(step)
             _header_is_true(hip, X, n, m, d, known)
+
+
+def _step_in_turn(hip, X, Y, forms, step):
+    loops = [_loop(hip, X, Y, f) for f in forms]
+    for l in loops:
+        l.init()
+    for _ in range(8 // step):
+        for l in loops:
+            l.enqueue(step)
+    return loops
+
+
+@pytest.mark.parametrize("step", [1, 2])
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("n,m,d", [(300, 200, 20), (1300, 900, 64), (10_273, 300, 30)])
+def test_each_loop_gets_the_potentials_it_has_alone(hip, monkeypatch, n, m, d, form, step):
+    """Alone, the scores come from the copy in every iteration, here from the general path in some: float32 rounding of the
+    scores apart (1e-5 relative, as in the solver tests). A loop whose copy comes back carries on from the potentials of
+    the iterations without it."""
+    print(f"two loops in turn: {form}, {n} x {m}, d {d}, {step} at a time", flush=True)
+    monkeypatch.setenv("TRNOPT_HIP_LOOP", "1")
+    for l, f in zip(_step_in_turn(hip, *_clouds(hip, n, m, d), FORMS[form], step), FORMS[form]):
+        alone = _loop(hip, *_clouds(hip, n, m, d), f)
+        alone.init()
+        alone.enqueue(8)
+        assert (l.read_state().it, l.read_state().eps) == (alone.read_state().it, alone.read_state().eps)
+        for got, want, k in ((l.fh, alone.fh, n), (l.gh, alone.gh, m)):
+            assert inf_rel(got[:k].cpu(), want[:k].cpu()) <= 1e-5

@@ -187,7 +187,7 @@ struct PartialArgs {
     const float* xsq;   // |x|^2 (half-step epilogue)
     const float* off;   // log(target / weight) or null
     float* out;         // merged result (fh, or the plain row-LSE)
-    float* out2;        // or null: with log2-unit scores, also the result in log2 units, (c / 2) fh + Ll
+    float* out2;        // or null: also the result in log2 units, (c / 2) fh + Ll (on-device loop)
     const float* rows_l2lo;   // with out2: the rows' Ll (the low part of their log2 weights)
     int n_store;        // rows of out written
     float2* meas;       // per-group convergence partials (g update of the loop), or null

@@ -200,7 +200,8 @@ __device__ inline void set_scalars(sk_state* st, double e, double rho_x, double 
 }
 
 // A row's new potential from its merged maximum Md (the columns' log2 weight offset back on) and log2 S, see
-// merge_group: val = fh, and with l2 R = (c / 2) fh as well.
+// merge_group: fh, and R = (c / 2) fh, its log2-unit potential. (Also without l2: the copy belongs to the cloud, two loops
+// on one cloud hand it to and fro, and the update that finds it again reads this one's R.)
 struct RowTerms {
     float sc2, kappa;      // eps, kappa
     float c;               // score scale (2 / eps) log2(e)
@@ -220,7 +221,9 @@ __device__ __forceinline__ float row_value(const RowTerms& r, bool l2, bool log2
     // eps lse = 2 M + eps ln(S) in accumulator units (log2-unit slots: M / c), with the caller's eps
     // (float) as the reference's epilogue multiplies by it (src/trnopt/sinkhorn.py:119)
     const double eps_lse = 2.0 * (l2 ? Md / (double)r.c : Md) + (double)r.sc2 * kLn2D * l2s;
-    return (float)(kappa * ((double)r.sc2 * od - eps_lse) + (kappa - 1.0) * x2d);
+    const float fh = (float)(kappa * ((double)r.sc2 * od - eps_lse) + (kappa - 1.0) * x2d);
+    R = (double)fh * (0.5 * (double)r.c);
+    return fh;
 }
 
 // Merge the slots of row i = 256 g + t (thread t of the workgroup, one row per thread) and apply the epilogue:
@@ -310,13 +313,11 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
             // error (4.5e-7 there) and an offset of the cost. For kappa = 1 and no offset it is -eps lse, exact.
             double R = 0.0;
             const float val = row_value({sc2, sc3, c_hs, x2, o}, l2, a.out2 != nullptr, Md, l2s, R);
-            if (l2 && a.out2 != nullptr) {
+            if (a.out2 != nullptr && i < a.n_store) {
                 // (a schedule's next eps is known here: its log2-unit potential comes from fh, as the control derives
                 // it for a new stage)
                 const double Rn = a.next_k2 != 0.0f ? (double)val * (double)a.next_k2 : R;
-                if (i < a.n_store) st<COH>(a.out2 + i, (float)(Rn + (double)ll));
-            } else if (a.out2 != nullptr && a.next_k2 != 0.0f && i < a.n_store) {
-                st<COH>(a.out2 + i, (float)((double)val * (double)a.next_k2 + (double)ll));
+                st<COH>(a.out2 + i, (float)(Rn + (double)ll));
             }
             if (a.meas != nullptr) {
                 if (i < a.n_real) dmax = fabsf(val - old);

@@ -388,7 +388,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
                 double R = 0.0;
                 fh = row_value({ctl.st.sc_x[2], ctl.st.sc_x[3], chs, x2, xo}, l2, true,
                                (double)M + (l2 ? (double)loop_weight_offset(a.f.yc) : 0.0), (double)ls.e + (double)ls.lm, R);
-                if (l2) fr = (float)(R + (double)xl);
+                fr = (float)(R + (double)xl);
                 publish(a.ex + i, __float_as_uint(l2 ? fr : fh), tag);
             }
         }
@@ -404,12 +404,11 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         u64* const msr = a.msr + 3 * (size_t)a.g.nrb * (ctl.st.it & 1);
         const bool measured = need && (cfg.n_stages > 0 || (cfg.fixed_iters == 0 && ctl.st.it > cfg.n_sched));
         float R32 = 0.0f;
-        bool l2 = false;
         if (has_y) {
             update<NC, 1>(a.g, a.ex, tag, w, {rank, a.ranks, sy, tag}, ctl, cols, slots, M, S);
             if (ry && ctl.abort == 0) {
                 const float chs = ctl.st.sc_y[0] * kLog2e;
-                l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.g.xr);
+                const bool l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.g.xr);
                 const Log2Split ls = lse_log2(S);
                 double R = 0.0;
                 const float old = gh;
@@ -454,7 +453,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
             // y's potentials in the units of the next f update: at a new eps derived from gh, as the control does
             if (!done && ctl.st.sc_x[0] != ran)
                 gr = (float)((double)gh * (0.5 * (double)(ctl.st.sc_x[0] * kLog2e)) + (double)yl);
-            else if (l2)
+            else
                 gr = R32;
             const bool next_l2 = ctl.c != 0.0f && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(a.g.xr);
             publish(a.ey + i, __float_as_uint(next_l2 ? gr : gh), tag + 1u);
