@@ -351,9 +351,8 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     const bool has_x = rank < nsx, has_y = rank < nsy;
     if (!has_x && !has_y) return;
     sk_state* gst = a.g.state;
-    if (gst->done != 0) return;
     if (tid == 0) {
-        ctl.st = *gst;
+        ctl.st = *gst;                     // by one thread: a workgroup that gives up may be setting done
         const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
         ctl.c = tag.c;
         ctl.t = tag.t;
@@ -373,6 +372,9 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     const float yw = ry ? a.g.w[i] : 0.0f;
     float fh = rx ? a.f.out[i] : 0.0f, fr = rx ? a.f.out2[i] : 0.0f, gh = ry ? a.g.out[i] : 0.0f, gr = ry ? a.g.out2[i] : 0.0f;
     __syncthreads();
+    const bool idle = ctl.st.done != 0;
+    __syncthreads();                       // every wave has the same answer before one may set abort
+    if (idle) return;
     unsigned ytag = 0u;                    // the tag of y's latest potentials (0: in memory)
     bool done = false;
     for (int k = 0; k < a.iters && !done; ++k) {
