@@ -224,9 +224,11 @@ int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream);
  * launch whose workgroups stay for all of them and pass the potentials to one another directly, else (and while the stream
  * captures, and for a single iteration) as sk_loop_run_f32. Cooperative launches of one device run one after another: for
  * a caller whose loops share the GPU on several streams sk_loop_run_f32 is the better form. If the workgroups should not
- * all get to run, the loop gives up after about a second: state done with checks = -1, for the caller to start again with
- * sk_loop_init_f32 and sk_loop_run_f32. */
+ * all get to run, the launch gives up after about a second, and a launch of one workgroup queued behind it runs the same
+ * iterations again; how often that was since sk_loop_init_f32 is an int at byte sk_loop_repairs_offset of L->ws (0: the
+ * problem has no such form). */
 int sk_loop_resident(const sk_loop_f32* L);
+size_t sk_loop_repairs_offset(const sk_loop_f32* L);
 int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream);
 
 /*

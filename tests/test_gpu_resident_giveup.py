@@ -49,7 +49,16 @@ def test_enqueued_iterations_are_done(hip, monkeypatch, n, m, d, form):
             loop.enqueue(k)
             seen += [fh.clone(), gh.clone()]
         got.append((seen, _state(loop.read_state()), loop.X.pk[:36].cpu()))
+        assert (loop.repairs() > 0) == (polls is not None)
     for p, q in zip(got[0][0], got[1][0]):
         assert torch.equal(p, q)
-    assert got[0][1] == got[1][1] or np.isnan(got[0][1]).any()
+    np.testing.assert_array_equal(got[0][1], got[1][1])
     assert torch.equal(got[0][2][:28], got[1][2][:28])
+
+
+def test_no_launch_gives_up_by_itself(hip, monkeypatch):
+    monkeypatch.setenv("TRNOPT_HIP_LOOP", "1")
+    loop = _loop(hip, 1300, 1000, 64, "fixed")
+    loop.init()
+    loop.enqueue(40)
+    assert (loop.read_state().it, loop.repairs()) == (40, 0)

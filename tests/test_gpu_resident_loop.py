@@ -90,9 +90,12 @@ def test_mixed_calls_continue_one_loop(hip, monkeypatch):
 
 @pytest.mark.parametrize("form", ["fixed", "converged", "stages"])
 def test_a_launch_that_gives_up_is_run_again_as_launches(hip, monkeypatch, form):
-    """With a single poll allowed, any wait gives up: the solve falls back to launches with the same result."""
+    """With a single poll allowed, any wait gives up: the iterations are run again with the result of launches."""
     monkeypatch.setenv("TRNOPT_HIP_LOOP_POLLS", "1")
+    loops, init = [], hip.DeviceLoop.init
+    monkeypatch.setattr(hip.DeviceLoop, "init", lambda loop: (loops.append(loop), init(loop))[1])
     _same(*_both(monkeypatch, 400, 900, 30, FORMS[form]))
+    assert [l.repairs() > 0 for l in loops] == [False, True]
 
 
 def test_threads_and_streams_side_by_side(hip, monkeypatch):

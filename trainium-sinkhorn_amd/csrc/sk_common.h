@@ -218,10 +218,12 @@ int hip_fail(hipError_t e, const char* where);
 // Several iterations of the loop with passes f and g in one launch (sk_loop.hip): both clouds of at most kLoopMaxBlocks
 // row blocks (one workgroup each, all resident) and kLoopMaxTiles tiles. exchange: loop_exchange_words 8-byte words, zero at
 // loop init.
-constexpr int kLoopMaxTiles = 192, kLoopMaxBlocks = 256;
+constexpr int kLoopMaxTiles = 192, kLoopMaxBlocks = 256, kLoopSavedWords = 34;
 inline size_t loop_exchange_words(int nx_pad, int ny_pad, int slots_x, int slots_y) {
-    return (size_t)nx_pad * (1 + 2 * slots_x) + (size_t)ny_pad * (1 + 2 * slots_y) + 6 * (size_t)(ny_pad / 32);
+    return (size_t)nx_pad * (1 + 2 * slots_x) + (size_t)ny_pad * (2 + 2 * slots_y) + 6 * (size_t)(ny_pad / 32) + kLoopSavedWords;
 }
+// Byte offset in the exchange of the 4-byte count of launches that gave up and were run again.
+size_t loop_repairs_at(int nx_pad, int ny_pad, int slots_x, int slots_y);
 // Waves of a workgroup: as many as hide each other's latencies with the operands in registers (128, 168, 256 a lane).
 constexpr int loop_waves(int nc) { return nc <= 2 ? 16 : nc <= 4 ? 12 : 8; }
 // ranks: workgroups that share a row block; slots_x, slots_y: the most segments of one, for ranks > 1 (else 0).

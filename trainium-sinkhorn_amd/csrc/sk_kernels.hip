@@ -1026,6 +1026,15 @@ int sk_loop_resident(const sk_loop_f32* L) {
     return lo.exchange != nullptr && loop_persists(lo.pf, lo.pg) ? 1 : 0;
 }
 
+size_t sk_loop_repairs_offset(const sk_loop_f32* L) {
+    if (check_loop(L, "sk_loop_repairs_offset") != SK_OK) return 0;
+    const LoopLayout lo = loop_layout(L);
+    if (lo.exchange == nullptr) return 0;
+    const bool shared = loop_ranks(lo.pf, lo.pg) > 1;
+    return (size_t)((char*)lo.exchange - (char*)L->ws) +
+           loop_repairs_at(lo.pf.nrb * SK_TILE, lo.pg.nrb * SK_TILE, shared ? lo.pf.slots : 0, shared ? lo.pg.slots : 0);
+}
+
 int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream) {
     if (int r = check_loop(L, "sk_loop_run_resident_f32")) return r;
     if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_resident_f32: iters %d < 0", iters);

@@ -15,14 +15,18 @@
 // (control_decide), each workgroup for itself.
 //
 // Every wait ends: the launch is cooperative (all its workgroups are resident), and a poll that has not seen its word after
-// `polls` rounds gives up: its workgroup ends without publishing, so that every other one's polls end the same way, and the
-// state says so (checks = -1, done); the host then runs the loop again in launches.
+// `polls` rounds gives up: its workgroup ends without publishing, so that every other one's polls end the same way, and says
+// so in a word that nothing else writes. A launch of one workgroup behind it (repair_kernel, which returns at once
+// otherwise: 2 us) then runs the same iterations by itself from where the launch began, so that whoever reads the potentials
+// next, the caller or a kernel, finds them done.
 //
 // Where CUs would be idle, `ranks` workgroups share a row block: each takes every ranks-th segment, and rank 0 merges them all,
 // one exchange more and a ranks-th of the tiles (2,048 x 2,048 d 64, us an iteration: one rank 27.1, two 22.6, four 19.3).
 //
 // A potential's word is overwritten only after every reader has it: the next iteration's value is published by a
 // workgroup that has read all of the other cloud's values, each published by a workgroup that had read all of this one's.
+
+#include <stddef.h>
 
 #include "sk_common.h"
 #include "sk_epilogue.h"
@@ -249,12 +253,13 @@ __device__ __forceinline__ void update(const PartialArgs& a, const u64* ex, unsi
 }
 
 // The control of one iteration (every workgroup for itself, from the same measures): advances ctl, true when the loop is
-// done. ny: row blocks of y; msr their published measures {max change}, {low}, {high half of the error sum}.
+// done. ny: row blocks of y; msr their published measures {max change}, {low}, {high half of the error sum} (null: they are in
+// lds_mx and lds_sm already).
 template <int NT>
 __device__ inline bool control(const PartialArgs& g, const u64* msr, unsigned tag, int ny, bool measured, Ctl& ctl, float* lds_mx,
                                double* lds_sm) {
     const int tid = tid_x();
-    if (measured) {
+    if (measured && msr != nullptr) {
         for (int b = tid; b < ny; b += NT) {
             u64 w[3];
             bool all = false;
@@ -324,13 +329,82 @@ __device__ inline bool control(const PartialArgs& g, const u64* msr, unsigned ta
     return ctl.st.done != 0;
 }
 
+// Where a launch began, for repair_kernel to begin there again: saved by the launch's workgroups before they do anything
+// else (one that starts after another has given up as well: nothing of its rows has changed by then).
+struct Saved {
+    sk_state st;
+    CopyTag tag;
+    char apart[168];      // (a cache line away from what another XCD's workgroup stores plainly)
+    int gave_up;          // a workgroup of the launch has
+    int repairs;          // launches run again since the loop's init
+};
+static_assert(sizeof(Saved) <= 8 * kLoopSavedWords, "the exchange has kLoopSavedWords words for it");
+
 struct LoopArgs {
     PartialArgs f, g;
     u64 *ex, *ey, *msr;      // the potentials of x and y and (two turns of) the measures of y's row blocks, tagged words
     u64 *sx, *sy;            // the segments' (M, S) of the ranks above 0 (Rank)
+    float2* rows;            // y's potentials where the launch began: gh and its log2-unit potential
+    Saved* saved;
     int iters, polls, ranks;
     int slots_x, slots_y;    // segments of a row block, at most
 };
+
+// One row of an update from its merged maximum and sum: the new potential, and R in its log2-unit potential (R + Ll).
+template <int ROLE>
+__device__ __forceinline__ float row_of(const PartialArgs& a, const Ctl& ctl, float M, float S, float p2, float off, float l2lo,
+                                        float& u2, bool& l2) {
+    const float* sc = ROLE == 0 ? ctl.st.sc_x : ctl.st.sc_y;
+    const float chs = sc[0] * kLog2e;
+    l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(ROLE == 0 ? a.yc : a.xr);
+    const Log2Split ls = lse_log2(S);
+    double R = 0.0;
+    const float h = row_value({sc[2], sc[3], chs, p2, off}, l2, true, (double)M + (l2 ? (double)loop_weight_offset(a.yc) : 0.0),
+                              (double)ls.e + (double)ls.lm, R);
+    u2 = (float)(R + (double)l2lo);
+    return h;
+}
+
+// The measures of a block of y's rows, one row per lane of the first half wave: the largest change and the error sum.
+__device__ __forceinline__ void row_measures(const Ctl& ctl, float old, float now, bool real, float w, float& dmax, double& derr) {
+    dmax = real ? fabsf(now - old) : 0.0f;
+    const float delta = fminf((old - now) * ctl.st.sc_y[1], kDeltaCap);
+    derr = (double)fabsf(w * (expf(delta) - 1.0f));
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {
+        dmax = fmaxf(dmax, __shfl_xor(dmax, o));
+        derr += __shfl_xor(derr, o);
+    }
+}
+
+// Whether the control of the iteration that ends looks at its measures.
+__device__ __forceinline__ bool takes_measures(const LoopCfg& cfg, int it) {
+    return cfg.n_stages > 0 || (cfg.fixed_iters == 0 && it > cfg.n_sched);
+}
+
+// This iteration's f update has made a pending copy if it was for its eps. (Another eps: the copy of another loop on the same
+// clouds, still pending.)
+__device__ __forceinline__ bool made_copy(const PartialArgs& f, const Ctl& ctl) {
+    return ctl.pending != 0 && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(f.yc);
+}
+
+// y's log2-unit potential at a new eps, from gh as the control derives it.
+__device__ __forceinline__ float at_new_eps(const Ctl& ctl, float gh, float l2lo) {
+    return (float)((double)gh * (0.5 * (double)(ctl.st.sc_x[0] * kLog2e)) + (double)l2lo);
+}
+
+// The state and the copy's header, by one thread.
+__device__ __forceinline__ void write_back(const LoopArgs& a, const Ctl& ctl) {
+    *a.g.state = ctl.st;
+    float* h = reinterpret_cast<float*>(a.f.rebake);
+    const bool p = ctl.pending != 0;
+    h[2] = p ? 0.0f : ctl.c;
+    h[3] = ctl.s2;
+    if (!p) h[4] = ctl.t;
+    h[7] = ctl.c;
+    h[8] = ctl.t;
+    reinterpret_cast<int*>(h)[6] = p ? 1 : 0;
+}
 
 template <int NC>
 __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
@@ -350,29 +424,34 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     const int nsx = segments(a.f), nsy = segments(a.g);
     const bool has_x = rank < nsx, has_y = rank < nsy;
     if (!has_x && !has_y) return;
-    sk_state* gst = a.g.state;
+    const int i = w * kRowsOfBlock + tid;
+    const bool rx = has_x && rank == 0 && tid < kRowsOfBlock, ry = has_y && rank == 0 && tid < kRowsOfBlock;
+    float fh = rx ? a.f.out[i] : 0.0f, fr = rx ? a.f.out2[i] : 0.0f, gh = ry ? a.g.out[i] : 0.0f, gr = ry ? a.g.out2[i] : 0.0f;
+    if (ry) a.rows[i] = make_float2(gh, gr);
+    const sk_state* gst = a.g.state;
+    const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
+    if (w == 0 && rank == 0 && tid == 0) {
+        a.saved->st = *gst;
+        a.saved->tag = tag;
+    }
     if (tid == 0) {
-        ctl.st = *gst;                     // by one thread: a workgroup that gives up may be setting done
-        const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
+        ctl.st = *gst;
         ctl.c = tag.c;
         ctl.t = tag.t;
         ctl.s2 = tag.s2;
         ctl.pending = tag.pending;
         ctl.unseen = 0;
         ctl.polls = a.polls;
-        ctl.abort = 0;
+        ctl.abort = coh_load(&a.saved->gave_up);      // by one thread: another workgroup may be setting it
     }
-    const int i = w * kRowsOfBlock + tid;
-    const bool rx = has_x && rank == 0 && tid < kRowsOfBlock, ry = has_y && rank == 0 && tid < kRowsOfBlock;
     u64* const sx = a.sx + (size_t)w * a.slots_x * kRowsOfBlock * 2;
     u64* const sy = a.sy + (size_t)w * a.slots_y * kRowsOfBlock * 2;
     const LoopCfg& cfg = a.g.cfg;
     const float x2 = rx ? a.f.xsq[i] : 0.0f, xo = rx && a.f.off != nullptr ? a.f.off[i] : 0.0f, xl = rx ? a.f.rows_l2lo[i] : 0.0f;
     const float y2 = ry ? a.g.xsq[i] : 0.0f, yo = ry && a.g.off != nullptr ? a.g.off[i] : 0.0f, yl = ry ? a.g.rows_l2lo[i] : 0.0f;
     const float yw = ry ? a.g.w[i] : 0.0f;
-    float fh = rx ? a.f.out[i] : 0.0f, fr = rx ? a.f.out2[i] : 0.0f, gh = ry ? a.g.out[i] : 0.0f, gr = ry ? a.g.out2[i] : 0.0f;
     __syncthreads();
-    const bool idle = ctl.st.done != 0;
+    const bool idle = ctl.st.done != 0 || ctl.abort != 0;
     __syncthreads();                       // every wave has the same answer before one may set abort
     if (idle) return;
     unsigned ytag = 0u;                    // the tag of y's latest potentials (0: in memory)
@@ -384,13 +463,8 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         if (has_x) {
             update<NC, 0>(a.f, a.ey, ytag, w, {rank, a.ranks, sx, tag}, ctl, cols, slots, M, S);
             if (rx && ctl.abort == 0) {
-                const float chs = ctl.st.sc_x[0] * kLog2e;
-                const bool l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.f.yc);
-                const Log2Split ls = lse_log2(S);
-                double R = 0.0;
-                fh = row_value({ctl.st.sc_x[2], ctl.st.sc_x[3], chs, x2, xo}, l2, true,
-                               (double)M + (l2 ? (double)loop_weight_offset(a.f.yc) : 0.0), (double)ls.e + (double)ls.lm, R);
-                fr = (float)(R + (double)xl);
+                bool l2;
+                fh = row_of<0>(a.f, ctl, M, S, x2, xo, xl, fr, l2);
                 publish(a.ex + i, __float_as_uint(l2 ? fr : fh), tag);
             }
         }
@@ -404,28 +478,17 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         // the g update
         const bool need = needs_control(ctl.st.it, ctl.st.stage, ctl.st.stage_it, cfg);
         u64* const msr = a.msr + 3 * (size_t)a.g.nrb * (ctl.st.it & 1);
-        const bool measured = need && (cfg.n_stages > 0 || (cfg.fixed_iters == 0 && ctl.st.it > cfg.n_sched));
-        float R32 = 0.0f;
+        const bool measured = need && takes_measures(cfg, ctl.st.it);
         if (has_y) {
             update<NC, 1>(a.g, a.ex, tag, w, {rank, a.ranks, sy, tag}, ctl, cols, slots, M, S);
             if (ry && ctl.abort == 0) {
-                const float chs = ctl.st.sc_y[0] * kLog2e;
-                const bool l2 = ctl.c != 0.0f && ctl.c == chs && ctl.s2 == packed_scale(a.g.xr);
-                const Log2Split ls = lse_log2(S);
-                double R = 0.0;
+                bool l2;
                 const float old = gh;
-                gh = row_value({ctl.st.sc_y[2], ctl.st.sc_y[3], chs, y2, yo}, l2, true,
-                               (double)M + (l2 ? (double)loop_weight_offset(a.g.yc) : 0.0), (double)ls.e + (double)ls.lm, R);
-                R32 = (float)(R + (double)yl);
+                gh = row_of<1>(a.g, ctl, M, S, y2, yo, yl, gr, l2);
                 if (measured) {
-                    float dmax = i < a.g.n_real ? fabsf(gh - old) : 0.0f;
-                    const float delta = fminf((old - gh) * ctl.st.sc_y[1], kDeltaCap);
-                    double derr = (double)fabsf(yw * (expf(delta) - 1.0f));
-#pragma unroll
-                    for (int o = 16; o > 0; o >>= 1) {
-                        dmax = fmaxf(dmax, __shfl_xor(dmax, o));
-                        derr += __shfl_xor(derr, o);
-                    }
+                    float dmax;
+                    double derr;
+                    row_measures(ctl, old, gh, i < a.g.n_real, yw, dmax, derr);
                     if (tid == 0) {
                         const u64 e = (u64)__double_as_longlong(derr);
                         publish(msr + 3 * w, __float_as_uint(dmax), tag + 1u);
@@ -438,9 +501,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         __syncthreads();
         if (ctl.abort != 0) break;
         if (tid == 0) {
-            // This iteration's f update has made a pending copy for its eps: rank 0 its block's tiles itself, and a g update
-            // waits for all of them. (Another eps: the copy of another loop on the same clouds, still pending.)
-            if (ctl.pending != 0 && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(a.f.yc)) {
+            if (made_copy(a.f, ctl)) {       // rank 0 its block's tiles itself, and a g update waits for all of them
                 if (rank != 0 && !has_y) ctl.unseen = 1;
                 ctl.pending = 0;
             }
@@ -452,11 +513,8 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
             if (ctl.abort != 0) break;
         }
         if (ry) {
-            // y's potentials in the units of the next f update: at a new eps derived from gh, as the control does
-            if (!done && ctl.st.sc_x[0] != ran)
-                gr = (float)((double)gh * (0.5 * (double)(ctl.st.sc_x[0] * kLog2e)) + (double)yl);
-            else
-                gr = R32;
+            // y's potentials in the units of the next f update
+            if (!done && ctl.st.sc_x[0] != ran) gr = at_new_eps(ctl, gh, yl);
             const bool next_l2 = ctl.c != 0.0f && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(a.g.xr);
             publish(a.ey + i, __float_as_uint(next_l2 ? gr : gh), tag + 1u);
         }
@@ -484,23 +542,103 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     }
     __syncthreads();
     if (ctl.abort != 0) {
-        if (tid == 0) {
-            gst->checks = -1;
-            gst->converged = 0;
-            gst->done = 1;
-        }
+        if (tid == 0) coh_store(&a.saved->gave_up, 1);
         return;
     }
-    if (w == 0 && rank == 0 && tid == 0) {
-        *gst = ctl.st;
-        float* h = reinterpret_cast<float*>(a.f.rebake);
-        const bool p = ctl.pending != 0;
-        h[2] = p ? 0.0f : ctl.c;
-        h[3] = ctl.s2;
-        if (!p) h[4] = ctl.t;
-        h[7] = ctl.c;
-        h[8] = ctl.t;
-        reinterpret_cast<int*>(h)[6] = p ? 1 : 0;
+    if (w == 0 && rank == 0 && tid == 0) write_back(a, ctl);
+}
+
+// The iterations of a launch that gave up, by one workgroup: every row block in turn, with the same instructions in the same
+// order, the potentials through memory (fences: the workgroup reads its own stores). 100 iterations at 2,048 x 2,048 d 64
+// take 0.4 s, which nobody is meant to see.
+template <int NC>
+__global__ __launch_bounds__(64 * loop_waves(NC)) void repair_kernel(LoopArgs a) {
+    constexpr int NT = 64 * loop_waves(NC);
+    __shared__ __attribute__((aligned(16))) bf16x8 cols[kLoopMaxTiles * 32];
+    __shared__ float2 slots[kLoopMaxTiles * kRowsOfBlock];
+    __shared__ float lds_mx[kLoopMaxBlocks];
+    __shared__ double lds_sm[kLoopMaxBlocks];
+    __shared__ Ctl ctl;
+    if (a.saved->gave_up == 0) return;
+    const int tid = tid_x();
+    const Rank alone = {0, 1, nullptr, 0u};
+    const LoopCfg& cfg = a.g.cfg;
+    if (tid == 0) {
+        const CopyTag tag = a.saved->tag;
+        ctl.st = a.saved->st;
+        ctl.c = tag.c;
+        ctl.t = tag.t;
+        ctl.s2 = tag.s2;
+        ctl.pending = tag.pending;
+        ctl.unseen = 0;
+        ctl.polls = 0;
+        ctl.abort = 0;
+        // (this loop's copy may be overwritten by a later eps's, whose f updates the launch has reached: made anew)
+        if (ctl.c != 0.0f && ctl.c == ctl.st.sc_x[0] * kLog2e && ctl.s2 == packed_scale(a.f.yc)) ctl.pending = 1;
+    }
+    for (int i = tid; i < a.g.nrb * kRowsOfBlock; i += NT) {
+        const float2 v = a.rows[i];
+        a.g.out[i] = v.x;
+        a.g.out2[i] = v.y;
+    }
+    __threadfence();
+    __syncthreads();
+    bool done = false;
+    for (int k = 0; k < a.iters && !done; ++k) {
+        for (int b = 0; b < a.f.nrb; ++b) {
+            float M = 0.0f, S = 1.0f;
+            update<NC, 0>(a.f, nullptr, 0u, b, alone, ctl, cols, slots, M, S);
+            if (tid < kRowsOfBlock) {
+                const int i = b * kRowsOfBlock + tid;
+                float u2;
+                bool l2;
+                a.f.out[i] = row_of<0>(a.f, ctl, M, S, a.f.xsq[i], a.f.off != nullptr ? a.f.off[i] : 0.0f, a.f.rows_l2lo[i], u2, l2);
+                a.f.out2[i] = u2;
+            }
+            __syncthreads();
+        }
+        __threadfence();
+        if (tid == 0) {
+            ctl.st.it += 1;
+            ctl.st.stage_it += 1;
+        }
+        __syncthreads();
+        const bool need = needs_control(ctl.st.it, ctl.st.stage, ctl.st.stage_it, cfg);
+        const bool measured = need && takes_measures(cfg, ctl.st.it);
+        for (int b = 0; b < a.g.nrb; ++b) {
+            float M = 0.0f, S = 1.0f;
+            update<NC, 1>(a.g, nullptr, 0u, b, alone, ctl, cols, slots, M, S);
+            if (tid < kRowsOfBlock) {
+                const int i = b * kRowsOfBlock + tid;
+                float u2;
+                bool l2;
+                const float old = a.g.out[i];
+                const float gh = row_of<1>(a.g, ctl, M, S, a.g.xsq[i], a.g.off != nullptr ? a.g.off[i] : 0.0f, a.g.rows_l2lo[i], u2, l2);
+                a.g.out[i] = gh;
+                a.g.out2[i] = u2;
+                float dmax;
+                double derr;
+                row_measures(ctl, old, gh, i < a.g.n_real, a.g.w[i], dmax, derr);
+                if (tid == 0) {
+                    lds_mx[b] = dmax;
+                    lds_sm[b] = derr;
+                }
+            }
+            __syncthreads();
+        }
+        const float ran = ctl.st.sc_x[0];
+        if (tid == 0 && made_copy(a.f, ctl)) ctl.pending = 0;
+        __syncthreads();
+        if (need) done = control<NT>(a.g, nullptr, 0u, a.g.nrb, measured, ctl, lds_mx, lds_sm);
+        if (!done && ctl.st.sc_x[0] != ran)
+            for (int i = tid; i < a.g.nrb * kRowsOfBlock; i += NT) a.g.out2[i] = at_new_eps(ctl, a.g.out[i], a.g.rows_l2lo[i]);
+        __threadfence();
+        __syncthreads();
+    }
+    if (tid == 0) {
+        write_back(a, ctl);
+        a.saved->gave_up = 0;
+        a.saved->repairs += 1;
     }
 }
 
@@ -508,10 +646,18 @@ template <int NC>
 hipError_t launch_nc(const LoopArgs& a, int workgroups, hipStream_t st) {
     LoopArgs args = a;
     void* params[] = {&args};
-    return hipLaunchCooperativeKernel(loop_kernel<NC>, dim3(workgroups), dim3(64 * loop_waves(NC)), params, 0, st);
+    const dim3 threads(64 * loop_waves(NC));
+    const hipError_t e = hipLaunchCooperativeKernel(loop_kernel<NC>, dim3(workgroups), threads, params, 0, st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(repair_kernel<NC>, dim3(1), threads, 0, st, a);
+    return hipGetLastError();
 }
 
 }  // namespace
+
+size_t loop_repairs_at(int nx_pad, int ny_pad, int slots_x, int slots_y) {
+    return 8 * (loop_exchange_words(nx_pad, ny_pad, slots_x, slots_y) - kLoopSavedWords) + offsetof(Saved, repairs);
+}
 
 hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int ranks, int slots_x,
                        int slots_y, int polls, hipStream_t st) {
@@ -523,6 +669,8 @@ hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchang
     a.msr = a.ey + g.rows_pad;
     a.sx = a.msr + 6 * (size_t)g.nrb;
     a.sy = a.sx + (size_t)f.nrb * slots_x * kRowsOfBlock * 2;
+    a.rows = (float2*)(a.sy + (size_t)g.nrb * slots_y * kRowsOfBlock * 2);
+    a.saved = (Saved*)(a.rows + g.rows_pad);
     a.slots_x = slots_x;
     a.slots_y = slots_y;
     a.ranks = ranks;

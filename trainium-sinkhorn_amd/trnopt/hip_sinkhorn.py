@@ -98,6 +98,7 @@ _SIGS = {
     "sk_loop_init_f32": (ctypes.c_int, [ctypes.POINTER(SkLoop), ctypes.c_void_p]),
     "sk_loop_run_f32": (ctypes.c_int, [ctypes.POINTER(SkLoop), ctypes.c_int, ctypes.c_void_p]),
     "sk_loop_resident": (ctypes.c_int, [ctypes.POINTER(SkLoop)]),
+    "sk_loop_repairs_offset": (ctypes.c_size_t, [ctypes.POINTER(SkLoop)]),
     "sk_loop_run_resident_f32": (ctypes.c_int, [ctypes.POINTER(SkLoop), ctypes.c_int, ctypes.c_void_p]),
     "sk_loop_batch_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int]),
     "sk_loop_batch_plan": (ctypes.c_int, [ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int), ctypes.c_int,
@@ -445,8 +446,8 @@ class DeviceLoop:
     next batch already queued behind it (no per-iteration synchronisation).
 
     On the default stream a small loop (sk_loop_resident) runs each call's iterations as one resident launch instead, bit
-    for bit the same; on any other stream the caller may have more loops in flight, which resident launches would run one
-    after another.
+    for bit the same (should it give up, they are run again on the GPU: repairs); on any other stream the caller may have
+    more loops in flight, which resident launches would run one after another.
 
     With TRNOPT_HIP_GRAPH=1, whole batches of GRAPH_BATCH iterations are replayed from one captured HIP graph
     (20 to 40 kernels, no memset nodes): fewer host calls, for callers whose host enqueue is the bottleneck. Graph
@@ -489,17 +490,10 @@ class DeviceLoop:
         L.fixed_iters, L.balanced = int(bool(fixed_iters)), int(bool(balanced))
         L.ws, L.ws_bytes = self.ws.data_ptr(), self.ws.numel()
         self._L = L
-        self._queued, self._g0 = 0, None      # iterations enqueued since init; gh at init where launches are resident
         self._pinned = None                   # two pinned state buffers, made by the first run (a batch has its own)
         self._graph = None
 
     def init(self) -> None:
-        self._queued, self._g0 = 0, None
-        if _stream() == 0 and lib().sk_loop_resident(ctypes.byref(self._L)):
-            self._g0 = self.gh.clone()        # to start again from, should a resident launch give up
-        self._start()
-
-    def _start(self) -> None:
         _check(lib().sk_loop_init_f32(ctypes.byref(self._L), _stream()), "sk_loop_init_f32")
 
     @staticmethod
@@ -534,32 +528,25 @@ class DeviceLoop:
 
     def enqueue(self, iters: int) -> None:
         iters = int(iters)
-        self._queued += iters
         if iters >= self.GRAPH_BATCH and self.graphs_enabled():
             self.capture()
             for _ in range(iters // self.GRAPH_BATCH):
                 self._graph.replay()
             iters %= self.GRAPH_BATCH
         if iters > 0:
-            run = lib().sk_loop_run_f32 if self._g0 is None else lib().sk_loop_run_resident_f32
+            run = lib().sk_loop_run_resident_f32 if _stream() == 0 else lib().sk_loop_run_f32
             _check(run(ctypes.byref(self._L), iters, _stream()), "sk_loop_run_f32")
 
     def read_state(self) -> SkState:
         """Synchronous read of the current state (waits for everything enqueued)."""
         host = self.state.to("cpu")
-        return self._checked(SkState.from_buffer_copy(host.numpy().tobytes()))
+        return SkState.from_buffer_copy(host.numpy().tobytes())
 
-    def _checked(self, st: SkState) -> SkState:
-        """The state; where a resident launch gave up because its workgroups were not all running (sk_loop.hip), that
-        of everything enqueued, run again as launches."""
-        if st.checks >= 0:
-            return st
-        if self._g0 is not None:
-            self.gh.copy_(self._g0)
-            self._g0 = None
-            self._start()
-            _check(lib().sk_loop_run_f32(ctypes.byref(self._L), self._queued, _stream()), "sk_loop_run_f32")
-        return self.read_state()
+    def repairs(self) -> int:
+        """Resident launches since init that gave up, because their workgroups were not all running, and whose iterations
+        one workgroup then ran again (sk_loop.hip). Synchronises."""
+        at = lib().sk_loop_repairs_offset(ctypes.byref(self._L))
+        return int(self.ws[at:at + 4].cpu().view(torch.int32)) if at else 0
 
     def run(self, batch: int | None = None) -> SkState:
         """Run to `done` (converged or max_iters). Returns the final state."""
@@ -588,7 +575,7 @@ class DeviceLoop:
                     continue                  # keep a second batch queued behind the one we wait on
             buf, ev = inflight.pop(0)
             ev.synchronize()
-            st = self._checked(SkState.from_buffer_copy(buf.numpy().tobytes()))
+            st = SkState.from_buffer_copy(buf.numpy().tobytes())
             if st.done:
                 return st                     # final: the launches still queued return at once, changing nothing
             if not inflight and queued >= self.max_iters:  # pragma: no cover - done must be set by then
@@ -630,7 +617,7 @@ class DeviceLoopBatch:
 
     def init(self) -> None:
         for l in self.loops:
-            l._start()
+            l.init()
         _check(lib().sk_loop_batch_init_f32(self._ptrs, len(self.loops), self.ws.data_ptr(), self.ws.numel(),
                                             self._launch, _stream()), "sk_loop_batch_init_f32")
 
