@@ -333,8 +333,11 @@ __device__ inline bool merge_group(const PartialArgs& a, int g) {
         }
     }
     if (a.meas != nullptr) {
+        // Each half wave first, then the two: a 32-row block of the one-launch loop (sk_loop.hip) has the sum of a half
+        // wave, and adds the same numbers in the same order.
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
+        for (int k = 0; k < 6; ++k) {
+            const int o = k < 5 ? 16 >> k : 32;
             dmax = fmaxf(dmax, __shfl_xor(dmax, o));
             derr += __shfl_xor(derr, o);
         }
