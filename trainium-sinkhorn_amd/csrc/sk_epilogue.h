@@ -436,8 +436,7 @@ __device__ inline void control_step(sk_state* st, const float2* meas, int nmeas,
 // The loop's state counters as a g update sees them on entry (before any workgroup can reach the control).
 struct LoopCounters {
     int it, stage, stage_it;
-    int pending;               // this iteration's f update has made the pending copy's tiles: it was for this eps. (A copy
-                               // that another loop on the same clouds has still to make stays that loop's.)
+    int pending;               // the copy was pending in this iteration
 };
 __device__ inline LoopCounters loop_counters(const PartialArgs& a) {
     LoopCounters k = {0, 0, 0, 0};
@@ -445,10 +444,7 @@ __device__ inline LoopCounters loop_counters(const PartialArgs& a) {
         k.it = a.state->it;
         k.stage = a.state->stage;
         k.stage_it = a.state->stage_it;
-        if (a.rebake != nullptr) {
-            const CopyTag t = copy_tag(reinterpret_cast<const float*>(a.rebake), true);
-            k.pending = t.pending != 0 && t.c == a.sc[0] * kLog2e && t.s2 == packed_scale(a.xr) ? 1 : 0;
-        }
+        if (a.rebake != nullptr) k.pending = reinterpret_cast<const int*>(a.rebake)[6];
     }
     return k;
 }
@@ -467,7 +463,11 @@ __device__ inline void loop_step(const PartialArgs& a, int g, const LoopCounters
         }
         return;
     }
-    if (a.state == nullptr || !(lc.pending != 0 || needs_control(lc.it, lc.stage, lc.stage_it, a.cfg))) return;
+    // This iteration's f update has made a pending copy if it was for its eps. (Else the copy is another loop's, on the same
+    // clouds, and stays that loop's to make.) The header's words change only in the control, after every group's arrival.
+    const float* h1 = reinterpret_cast<const float*>(a.rebake);
+    const bool made = lc.pending != 0 && h1[7] == a.sc[0] * kLog2e && h1[3] == packed_scale(a.xr);
+    if (a.state == nullptr || !(made || needs_control(lc.it, lc.stage, lc.stage_it, a.cfg))) return;
     __shared__ int s_last;
     if constexpr (!COH) __threadfence();   // release: this group's outputs and meas[g]
     __syncthreads();                       // (COH: every wave's stores have completed)
@@ -490,7 +490,7 @@ __device__ inline void loop_step(const PartialArgs& a, int g, const LoopCounters
     if (a.rebake == nullptr) return;
     __syncthreads();
     float* h = reinterpret_cast<float*>(a.rebake);
-    if (tid_x() == 0 && lc.pending != 0) {                // this iteration's f update made the copy's tiles
+    if (tid_x() == 0 && made) {
         h[2] = h[7];
         h[4] = h[8];
         reinterpret_cast<int*>(h)[6] = 0;
