@@ -4,11 +4,14 @@ the launch-by-launch loop: potentials, iteration counts, errors and convergence 
 256-row groups and its largest (192 tiles), every width of kernel, one to four workgroups per row block, calls of several lengths, and clouds without a
 log2-unit copy; and from several streams and threads."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from trnopt import Backend
+from trnopt import hip_sinkhorn as hk
 from trnopt.sinkhorn import SinkhornOptions, sinkhorn
 
 pytestmark = pytest.mark.gpu
@@ -35,9 +38,16 @@ def _both(monkeypatch, n, m, d, o, x=None):
     x0, y, a, b = _clouds(n, m, d)
     kw = dict(a_target=a[::-1].copy(), b_target=b) if "rho" in o else {}
     out = []
+    lib = hk.lib()
+    run = lib.sk_loop_run_resident_f32
     for v in ("0", "1"):
+        resident = []                        # the form that each call of the loop's iterations takes
         monkeypatch.setenv("TRNOPT_HIP_LOOP", v)
+        monkeypatch.setattr(lib, "sk_loop_run_resident_f32",
+                            lambda L, k, stream: (resident.append(lib.sk_loop_resident(L)), run(L, k, stream))[1])
         out.append(sinkhorn(x0 if x is None else x, y, a, b, SinkhornOptions(kernel="hip", backend=ROCM, **o), **kw))
+        assert resident and set(resident) == {int(v)}
+    monkeypatch.setattr(lib, "sk_loop_run_resident_f32", run)
     return out
 
 
@@ -61,6 +71,17 @@ def test_every_form_bit_for_bit(hip, monkeypatch, form, n, m, d):
 def test_sizes_bit_for_bit(hip, monkeypatch, n, m, d):
     print(f"resident {n} x {m} d {d}", flush=True)
     _same(*_both(monkeypatch, n, m, d, dict(eps=0.3, max_iters=5, fixed_iters=True)))
+
+
+@pytest.mark.parametrize("n,m,fits", [(6144, 6144, 1), (6145, 40, 0), (40, 6145, 0)])
+def test_the_largest_loop_that_fits(hip, monkeypatch, n, m, fits):
+    monkeypatch.setenv("TRNOPT_HIP_LOOP", "1")
+    x, y, a, b = _clouds(n, m, 3)
+    loop = hip.DeviceLoop(hip.HipCloud(x, np.log(a), "cuda"), hip.HipCloud(y, np.log(b), "cuda", role=1), eps=1.0, rho_x=None,
+                          rho_y=None, sched=[], stages=[], tol=0.0, stage_tol=0.0, max_iters=1, check_every=1,
+                          stage_max_iters=1, fixed_iters=True, balanced=True)
+    assert hip.lib().sk_loop_resident(ctypes.byref(loop._L)) == fits
+    assert (hip.lib().sk_loop_repairs_offset(ctypes.byref(loop._L)) > 0) == bool(fits)
 
 
 def test_clouds_without_a_log2_copy(hip, monkeypatch):
