@@ -1,0 +1,105 @@
+"""The exact median where the approximate costs cannot narrow it down: a few points far outside the others (the bracket's
+width follows the largest norm), many of them, tight clusters far apart, ties. Integer coordinates, whose costs are exact in
+float64 whatever the order of the sums: the GPU's median equals numpy's."""
+
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_median import dense_median
+
+pytestmark = pytest.mark.gpu
+
+
+def _clouds(n, m, d, seed=0):
+    rng = np.random.default_rng(seed + n + 3 * m + 7 * d)
+    return np.round(rng.normal(size=(n, d)) * 300.0), np.round(rng.normal(size=(m, d)) * 250.0 + 100.0), rng
+
+
+def _far(p, rows, times, rng):
+    """Those rows moved out to `times` the others' typical norm, in random directions."""
+    v = rng.normal(size=(len(rows), p.shape[1]))
+    v *= times * np.sqrt((p * p).sum(1).mean()) / np.linalg.norm(v, axis=1)[:, None]
+    p[rows] = np.round(v)
+
+
+@pytest.mark.parametrize("times", [6, 30, 200, 5000])
+@pytest.mark.parametrize("n,m,d", [(257, 300, 3), (300, 2500, 17), (2200, 2100, 30), (1500, 700, 70), (600, 600, 128)])
+@pytest.mark.parametrize("where", ["x", "y", "both"])
+def test_a_few_points_far_out(hip, n, m, d, times, where):
+    print(f"median, far points {where} {times}: {n} x {m}, d {d}", flush=True)
+    x, y, rng = _clouds(n, m, d)
+    if where != "y":
+        _far(x, np.array([n // 3, n - 1]), times, rng)
+    if where != "x":
+        _far(y, np.array([0, m // 2, m - 1]), times, rng)
+    assert hip.cost_median(x, y, "cuda") == dense_median(x, y)
+
+
+@pytest.mark.parametrize("share", [0.02, 0.1, 0.3, 0.6])
+@pytest.mark.parametrize("clumped", [False, True])
+def test_many_points_far_out(hip, share, clumped):
+    n, m, d = 1900, 2300, 12
+    x, y, rng = _clouds(n, m, d)
+    k, l = int(share * n), int(share * m)
+    _far(x, np.arange(k) if clumped else rng.choice(n, k, replace=False), 60, rng)
+    _far(y, np.arange(l) if clumped else rng.choice(m, l, replace=False), 900, rng)
+    assert hip.cost_median(x, y, "cuda") == dense_median(x, y)
+
+
+@pytest.mark.parametrize("k", [1, 20, 90])
+def test_far_points_that_are_close_to_each_other(hip, k):
+    """Both clouds have a group at the same far place: pairs within it cost less than the typical pair."""
+    n, m, d = 1000, 1200, 8
+    x, y, rng = _clouds(n, m, d)
+    place = np.full(d, 400_000.0)
+    x[:k] = place + np.round(rng.normal(size=(k, d)) * 20)
+    y[-k:] = place + np.round(rng.normal(size=(k, d)) * 20)
+    assert hip.cost_median(x, y, "cuda") == dense_median(x, y)
+
+
+@pytest.mark.parametrize("share", [0.5, 0.52, 0.7])
+@pytest.mark.parametrize("n,m", [(900, 800), (2300, 2200)])
+def test_tight_clusters_far_apart(hip, n, m, share):
+    """Two clusters each, a thousand times their spread apart: costs within a cluster are a millionth of the others."""
+    d = 5
+    x, y, rng = _clouds(n, m, d)
+    x, y = np.round(x / 10), np.round(y / 10)
+    for p in (x, y):
+        p[: int(share * len(p))] += 15_000.0
+        p[int(share * len(p)):] -= 15_000.0
+    assert hip.cost_median(x, y, "cuda") == dense_median(x, y)
+
+
+@pytest.mark.parametrize("n", [2000, 2500])
+def test_ties_with_a_point_far_out(hip, n):
+    rng = np.random.default_rng(n)
+    x, y = rng.integers(0, 2, size=(n, 4)).astype(float), rng.integers(0, 2, size=(n, 4)).astype(float)
+    assert hip.cost_median(x, y, "cuda") == dense_median(x, y)
+    x[5] = 70_000.0
+    assert hip.cost_median(x, y, "cuda") == dense_median(x, y)
+
+
+@pytest.mark.parametrize("times", [40, 1000])
+def test_a_far_point_does_not_cost_many_times_the_call(hip, times):
+    """At 7,355 x 8,962 d 30 the call takes 0.2 ms and three passes over every float64 cost 0.7; one far point made it 2 to
+    13 ms (every pair's collection its own global atomic, then six such passes). Eight times leaves room for noise."""
+    x, y, rng = _clouds(7355, 8962, 30)
+
+    def time(x, y):
+        X, Y = torch.as_tensor(x).cuda(), torch.as_tensor(y).cuda()
+        out = torch.empty(1, dtype=torch.float64, device="cuda")
+        ts = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                hip.cost_median_device(X, Y, out)
+            b.record()
+            b.synchronize()
+            ts.append(a.elapsed_time(b))
+        return min(ts)
+
+    plain = time(x, y)
+    _far(x, np.array([3000]), times, rng)
+    assert time(x, y) <= 8 * plain

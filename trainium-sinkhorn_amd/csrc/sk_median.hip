@@ -16,8 +16,10 @@
 //   2. the pairs below that bracket counted, the pairs inside collected (0.1-0.3 % of them);
 //   3. the float64 costs of the collected pairs, and their order statistics k0 - below and k1 - below by a radix
 //      select (non-negative doubles order like their bit patterns), 11 bits at a time.
-// When the bracket holds more pairs than the workspace (massive ties), six radix-select passes over every float64
-// cost take over (select_pass_kernel). Every launch goes on the caller's stream with no host round trip.
+// When the bracket holds more pairs than the workspace (massive ties), radix-select passes over every float64 cost take
+// over (select_pass_kernel): three digits, the third also keeping the keys that still match, and the other three over
+// those keys (or over every cost again, if those are too many as well). Every launch goes on the caller's stream with no
+// host round trip.
 //
 // From the norms to the answer, all launches back to back: 7,355 x 8,962 d 30 192 us (the histogram pass 37 of them,
 // the collecting pass 50); 10,000 x 10,000 d 64 457 us; 7,000 x 7,000 d 128 276 us; 300 x 257 d 30 96 us. With three
@@ -44,6 +46,7 @@ constexpr int kColTile = 32;                // column points per LDS tile
 constexpr int kTargetBlocks = 1024;         // blocks a full pass aims for: columns per block follow
 constexpr int kChunk = 8;                   // coordinates per register chunk of the row
 constexpr int kPasses = 6;
+constexpr int kKeepPass = 2;                // the full pass that keeps the keys matching its prefix
 constexpr unsigned long long kCandMax = 1ull << 22;   // collected pairs, at most
 constexpr int kShift[kPasses] = {53, 42, 31, 20, 9, 0};
 constexpr int kWidth[kPasses] = {11, 11, 11, 11, 11, 9};
@@ -64,6 +67,7 @@ struct MedianState {
     unsigned long long base;        // key of the bracket's lower end less E: subtracted from the collected keys
     int bits;                       // bits of the largest difference to base
     int fallback;                   // 1: the bracket held more pairs than the workspace, or not the ranks
+    unsigned long long kept;        // keys that the third full pass kept
     int arrived;
     float lo, hi;                   // the bracket, in scaled units
     double scale;                   // power of two: (max |x| + max |y|) scale in [8, 16)
@@ -204,6 +208,7 @@ __global__ __launch_bounds__(kApproxThreads) void approx_pass_kernel(
     __shared__ unsigned fill;
     __shared__ unsigned long long base;
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+    if (COLLECT && st->fallback != 0) return;        // more pairs than cap in the bracket (written by the launch before)
     if (tid == 0) fill = 0u;
     if constexpr (!COLLECT)
         for (int b = tid; b < kHistBins; b += kApproxThreads) bins[b] = 0u;
@@ -219,6 +224,7 @@ __global__ __launch_bounds__(kApproxThreads) void approx_pass_kernel(
     const int rbs = (ntx + RB - 1) / RB;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     unsigned long long below = 0;
+    bool full = false;                               // COLLECT: more pairs than cap, no use collecting any more
     const unsigned long long units = (unsigned long long)rbs * (unsigned)nty, waves = (unsigned long long)gridDim.x * kApproxWaves;
     const unsigned long long w = (unsigned long long)blockIdx.x * kApproxWaves + wave;
     const unsigned u1 = (unsigned)(units * (w + 1) / waves);
@@ -273,9 +279,13 @@ __global__ __launch_bounds__(kApproxThreads) void approx_pass_kernel(
                     }
                 }
                 if constexpr (COLLECT) {
-                    if (in != 0u) {
+                    if (in != 0u && !full) {
                         // (padding points cost 1e38, above every bracket)
-                        unsigned p = atomicAdd(&fill, (unsigned)__popc(in));
+                        const unsigned k = (unsigned)__popc(in);
+                        unsigned p = atomicAdd(&fill, k);
+                        const unsigned staged = p >= kStage ? 0u : p + k <= kStage ? k : kStage - p;
+                        unsigned long long g = staged < k ? atomicAdd(&st->count, (unsigned long long)(k - staged)) : 0ull;
+                        full = g >= cap;
                         do {
                             const int r = __ffs((int)in) - 1;
                             in &= in - 1u;
@@ -284,8 +294,8 @@ __global__ __launch_bounds__(kApproxThreads) void approx_pass_kernel(
                             if (p < kStage) {
                                 bins[p] = idx;
                             } else {
-                                const unsigned long long g = atomicAdd(&st->count, 1ull);
                                 if (g < cap) pairs[g] = idx;
+                                ++g;
                             }
                             ++p;
                         } while (in != 0u);
@@ -336,7 +346,7 @@ __device__ inline bool last_to_arrive(int* counter, int blocks) {
 constexpr int kSumBlocks = kHistBins / 64;
 static_assert(kSumBlocks == 256, "one workgroup sum per thread of the last workgroup");
 __global__ __launch_bounds__(256) void bracket_kernel(const unsigned* __restrict__ slabs, int nslabs, MedianState* st,
-                                                      unsigned long long* __restrict__ total) {
+                                                      unsigned long long* __restrict__ total, unsigned long long cap) {
     __shared__ unsigned long long part[256];
     __shared__ int pick[2];
     const int tid = threadIdx.x, bin = (int)blockIdx.x * 64 + (tid & 63);
@@ -406,6 +416,12 @@ __global__ __launch_bounds__(256) void bracket_kernel(const unsigned* __restrict
         const unsigned long long k1 = (unsigned long long)__double_as_longlong(c1 < 1.7e308 ? c1 : 1.7e308);
         st->base = k0;
         st->bits = k1 > k0 ? 64 - __clzll((long long)(k1 - k0)) : 1;
+        // More pairs than the workspace holds in whole groups of 64 bins inside the bracket: not even tried. (The last
+        // group, with the padding points', is never inside.)
+        const unsigned l0 = __float_as_uint(st->lo) >> kHistShift, h0 = __float_as_uint(st->hi) >> kHistShift;
+        const int first = (int)(l0 < kHistBase ? 0u : l0 - kHistBase) / 64 + 1;
+        const int last = (int)(h0 < kHistBase ? 0u : h0 - kHistBase < kHistBins ? h0 - kHistBase : kHistBins - 1u) / 64 - 1;
+        if (last >= first && part[last] - part[first - 1] > cap) st->fallback = 1;
     }
 }
 
@@ -548,11 +564,19 @@ __global__ __launch_bounds__(256) void select_cand_kernel(const unsigned long lo
 // this keeps them on scalar loads whatever else the kernel stores.
 typedef __attribute__((address_space(4))) const double ConstDouble;
 
+// KEEP: the pass also keeps the matching keys, if no workgroup has more than kKeepStage of them and all together no more
+// than cap; the later passes then read those (`kept_keys`) instead of recomputing every cost. 7,355 x 8,962 d 30 with one
+// point 60 times the others' norm: 703 us by this way, 1,145 with six full passes.
+constexpr unsigned kKeepStage = 2048;
+template <bool KEEP>
 __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
     const double* __restrict__ xp, const double* __restrict__ yp, const double* __restrict__ xx,
     const double* __restrict__ yy, int n, int m, int dp, int cols, MedianState* ms, unsigned* __restrict__ hist, int shift,
-    int width, double* __restrict__ out) {
+    int width, double* __restrict__ out, unsigned long long* __restrict__ keys, unsigned long long cap, int kept_keys) {
     __shared__ unsigned h[2][kBins];
+    __shared__ unsigned long long stage[KEEP ? kKeepStage : 1];
+    __shared__ unsigned fill;
+    __shared__ unsigned long long base;
     const int tid = threadIdx.x;
     SelectState* st = &ms->full;
     if (ms->fallback == 0) {                              // the collected pairs hold the answer
@@ -568,10 +592,23 @@ __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
     const unsigned long long p0 = st->prefix[0] & high, p1 = st->prefix[1] & high;
     const unsigned dmask = (1u << width) - 1u;
     for (int b = tid; b < 2 * kBins; b += kRowsPerBlock) (&h[0][0])[b] = 0u;
+    if (tid == 0) fill = 0u;
+    bool full = false;
     __syncthreads();
+    const bool on_keys = kept_keys != 0 && ms->kept <= cap;
+    if (on_keys) {
+        const unsigned long long c = ms->kept;
+        for (unsigned long long e = (unsigned long long)blockIdx.x * kRowsPerBlock + tid; e < c;
+             e += (unsigned long long)gridDim.x * kRowsPerBlock) {
+            const unsigned long long key = keys[e];
+            const unsigned digit = (unsigned)(key >> shift) & dmask;
+            if ((key & high) == p0) atomicAdd(&h[0][digit], 1u);
+            if (!same && (key & high) == p1) atomicAdd(&h[1][digit], 1u);
+        }
+    }
 
     const int rbs = (n + kRowsPerBlock - 1) / kRowsPerBlock, cbs = (m + cols - 1) / cols;
-    for (int blk = blockIdx.x; blk < rbs * cbs; blk += gridDim.x) {
+    for (int blk = on_keys ? rbs * cbs : (int)blockIdx.x; blk < rbs * cbs; blk += gridDim.x) {
         const int i = blk % rbs * kRowsPerBlock + tid;
         const bool row_ok = i < n;
         const double xi2 = row_ok ? xx[i] : 0.0;
@@ -609,10 +646,25 @@ __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
                 const bool m1 = ok && !same && (key & high) == p1;
                 if (m0) atomicAdd(&h[0][digit], 1u);
                 if (m1) atomicAdd(&h[1][digit], 1u);
+                if constexpr (KEEP) {
+                    if ((m0 || m1) && !full) {
+                        const unsigned p = atomicAdd(&fill, 1u);
+                        if (p < kKeepStage) stage[p] = key;
+                        full = p >= kKeepStage;
+                    }
+                }
             }
         }
     }
     __syncthreads();
+    if constexpr (KEEP) {
+        const unsigned nf = fill;                          // past the stage: too many, cap and more
+        if (tid == 0 && nf != 0u) base = atomicAdd(&ms->kept, nf <= kKeepStage ? (unsigned long long)nf : cap + 1ull);
+        __syncthreads();
+        if (nf <= kKeepStage)
+            for (unsigned e = tid; e < nf; e += kRowsPerBlock)
+                if (base + e < cap) keys[base + e] = stage[e];
+    }
     if (add_counts(st, h, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0) {
         const double a = __longlong_as_double((long long)st->prefix[0]);
         const double b = __longlong_as_double((long long)st->prefix[1]);
@@ -682,7 +734,7 @@ void launch_approx(const MedianLayout& o, char* w, int n, int m, hipStream_t s) 
     hipLaunchKernelGGL((approx_pass_kernel<NC, false>), dim3(o.blocks), dim3(kApproxThreads), 0, s, xt, yt, xf, yf, n, m, o.ntx,
                        o.nty, st, slabs, slabs, o.cap);
     hipLaunchKernelGGL(bracket_kernel, dim3(kSumBlocks), dim3(256), 0, s, slabs, o.blocks, st,
-                       (unsigned long long*)(w + o.total));
+                       (unsigned long long*)(w + o.total), o.cap);
     hipLaunchKernelGGL((approx_pass_kernel<NC, true>), dim3(o.blocks), dim3(kApproxThreads), 0, s, xt, yt, xf, yf, n, m, o.ntx,
                        o.nty, st, slabs, slabs, o.cap);
 }
@@ -745,8 +797,8 @@ int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, 
     const long long blocks = (long long)rb * ((m + cols - 1) / cols);
     const dim3 grid((unsigned)std::min<long long>(blocks, kTargetBlocks));
     for (int q = 0; q < kPasses; ++q)
-        hipLaunchKernelGGL(select_pass_kernel, grid, dim3(kRowsPerBlock), 0, s, xp, yp, xx, yy, n, m, o.dp, cols, st, hist,
-                           kShift[q], kWidth[q], out);
+        hipLaunchKernelGGL(q == kKeepPass ? select_pass_kernel<true> : select_pass_kernel<false>, grid, dim3(kRowsPerBlock), 0, s,
+                           xp, yp, xx, yy, n, m, o.dp, cols, st, hist, kShift[q], kWidth[q], out, keys, o.cap, q > kKeepPass ? 1 : 0);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? SK_OK : hip_fail(e, "sk_cost_median_f64");
 }
