@@ -282,8 +282,10 @@ int sk_prepare_cloud_f64(const double* pts, int n, int d, const double* stat, fl
  * np.median's definition (mean of the two middle values when n m is even). xc (n, d), yc (m, d): row-major
  * float64 device arrays, already centred; out: one device double. Two passes over approximate costs (fp16 matrix
  * cores) bracket the middle ranks and collect the pairs that can hold the answer (up to 2^22 of them, 12 bytes each, in
- * ws), whose float64 costs are then selected by radix; with more of them (massive ties, a point very far out), three
- * radix-select passes over every float64 cost and three over the keys that are left. ws (sk_cost_median_workspace_bytes) also holds zero-padded copies and fp16 tiles of xc and yc.
+ * ws), whose float64 costs are then selected by radix; with more of them (massive ties), three radix-select passes
+ * over every float64 cost and three over the keys that are left. The pairs of a few points far outside the others are
+ * told apart by their float64 costs. ws (sk_cost_median_workspace_bytes) also holds zero-padded copies and fp16 tiles of
+ * xc and yc.
  * n m < 2^32, d <= SK_MEDIAN_D_MAX; ws 256-byte aligned.
  */
 #define SK_MEDIAN_D_MAX 128

@@ -82,8 +82,8 @@ def test_ties_with_a_point_far_out(hip, n):
 
 @pytest.mark.parametrize("times", [40, 1000])
 def test_a_far_point_does_not_cost_many_times_the_call(hip, times):
-    """At 7,355 x 8,962 d 30 the call takes 0.2 ms and three passes over every float64 cost 0.7; one far point made it 2 to
-    13 ms (every pair's collection its own global atomic, then six such passes). Eight times leaves room for noise."""
+    """At 7,355 x 8,962 d 30 the call takes 0.2 ms, with three passes over every float64 cost 0.7 to 1; one far point made it
+    2 to 13 ms once (a global atomic for every pair collected, then six such passes). Three times leaves room for noise."""
     x, y, rng = _clouds(7355, 8962, 30)
 
     def time(x, y):
@@ -102,4 +102,4 @@ def test_a_far_point_does_not_cost_many_times_the_call(hip, times):
 
     plain = time(x, y)
     _far(x, np.array([3000]), times, rng)
-    assert time(x, y) <= 8 * plain
+    assert time(x, y) <= 3 * plain

@@ -16,6 +16,11 @@
 //   2. the pairs below that bracket counted, the pairs inside collected (0.1-0.3 % of them);
 //   3. the float64 costs of the collected pairs, and their order statistics k0 - below and k1 - below by a radix
 //      select (non-negative doubles order like their bit patterns), 11 bits at a time.
+// E follows the largest norms, so the few points far outside the others are set aside first (near_limit): they take no part
+// in 1 and 2, their pairs' float64 costs are sorted into below, inside and above the bracket one by one (far_kernel), and the
+// answer is checked to lie inside it. Without that, one point 40 times the others' norm widened the bracket past the
+// workspace: 7,355 x 8,962 d 30 with one point at 20 / 30 / 40 / 1,000 times 290 / 437 / 918 / 1,000 us, and 208 at all of
+// them with it.
 // When the bracket holds more pairs than the workspace (massive ties), radix-select passes over every float64 cost take
 // over (select_pass_kernel): three digits, the third also keeping the keys that still match, and the other three over
 // those keys (or over every cost again, if those are too many as well). Every launch goes on the caller's stream with no
@@ -68,6 +73,8 @@ struct MedianState {
     int bits;                       // bits of the largest difference to base
     int fallback;                   // 1: the bracket held more pairs than the workspace, or not the ranks
     unsigned long long kept;        // keys that the third full pass kept
+    unsigned far[2];                // points of x and of y set aside
+    double vlo, vhi;                // an answer in here is right with points set aside
     int arrived;
     float lo, hi;                   // the bracket, in scaled units
     double scale;                   // power of two: (max |x| + max |y|) scale in [8, 16)
@@ -131,26 +138,52 @@ constexpr unsigned kHistBase = (0x43800000u >> kHistShift) - (unsigned)kHistBins
 // Twice the dot product's error is below 2^-16 R^2.
 constexpr double kCostErr = 0x1p-16;
 
-typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+constexpr float kOutside = 1.0e38f;          // the scaled |p|^2 of a point that takes no part
 
-__device__ __forceinline__ double max_of(const double* __restrict__ v, int n) {
+// The squared norm above which a cloud's points are set aside, from the largest of every 32 points (v, n of them): none
+// unless the largest norm is more than 8 times the typical one (the geometric mean of the n, to a power of two of the
+// square); then from 4 times, if that concerns at most an eighth of the n. By one wave, alike in every wave.
+__device__ inline double near_limit(const double* __restrict__ v, int n) {
     double mx = 0.0;
-    for (int e = (int)(threadIdx.x & 63); e < n; e += 64) mx = fmax(mx, v[e]);
-    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
-    return mx;
+    int exps = 0, cnt = 0;
+    const int lane = (int)(threadIdx.x & 63);
+    for (int e = lane; e < n; e += 64) {
+        const double t = v[e];
+        mx = fmax(mx, t);
+        if (t > 0.0 && t < 1.0e300) {
+            int x;
+            frexp(t, &x);
+            exps += x;
+            ++cnt;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        mx = fmax(mx, __shfl_xor(mx, o));
+        exps += __shfl_xor(exps, o);
+        cnt += __shfl_xor(cnt, o);
+    }
+    const double typical = cnt > 0 ? ldexp(1.0, exps / cnt) : mx;
+    if (!(mx > 64.0 * typical)) return mx;
+    int far = 0;
+    for (int e = lane; e < n; e += 64) far += v[e] > 16.0 * typical ? 1 : 0;
+    for (int o = 32; o > 0; o >>= 1) far += __shfl_xor(far, o);
+    return 8 * far <= n ? 16.0 * typical : mx;
 }
 
 // Both clouds laid out for the passes: a float64 copy with rows of dp coordinates (zeros after d; the columns' also to
 // whole tiles), the fp16 pieces of the scaled coordinates in the order of the matrix cores (as sk_pack_cloud_f32's
-// tiles: one thread per tile, K chunk and lane), the scaled |p|^2 in float32 (padding points: 1e38, above every cost).
+// tiles: one thread per tile, K chunk and lane), the scaled |p|^2 in float32 (padding points and those set aside, which
+// are listed: 1e38, above every cost).
 __global__ __launch_bounds__(256) void layout_kernel(const double* __restrict__ x, int n, const double* __restrict__ y, int m,
                                                      int d, int dp, int mp, int nc, const double* __restrict__ xx,
                                                      const double* __restrict__ yy, const double* __restrict__ block_max,
                                                      int xblocks, int yblocks, double* __restrict__ xp,
                                                      double* __restrict__ yp, f16x8* __restrict__ xt,
                                                      f16x8* __restrict__ yt, float* __restrict__ xf, float* __restrict__ yf,
-                                                     int ntx, int nty, MedianState* st) {
-    const double R = sqrt(max_of(block_max, xblocks)) + sqrt(max_of(block_max + xblocks, yblocks));
+                                                     int ntx, int nty, MedianState* st, unsigned* __restrict__ far_x,
+                                                     unsigned* __restrict__ far_y) {
+    const double lim_x = near_limit(block_max, xblocks), lim_y = near_limit(block_max + xblocks, yblocks);
+    const double R = sqrt(lim_x) + sqrt(lim_y);
     int e = 0;
     if (R > 0.0 && R < 1.0e300) frexp(R, &e);            // R in [2^(e - 1), 2^e)
     const double s = R > 0.0 && R < 1.0e300 ? ldexp(1.0, 4 - e) : 1.0;
@@ -171,12 +204,14 @@ __global__ __launch_bounds__(256) void layout_kernel(const double* __restrict__ 
             for (int k = lane; k < dp; k += 64) out[(size_t)i * dp + k] = i < np && k < d ? p[(size_t)i * d + k] : 0.0;
         for (int T = wave; T < nt; T += waves) {
             const int row = T * SK_TILE + (lane & 31);
+            const double nn = row < np ? (side == 0 ? xx : yy)[row] : 0.0;
+            const bool far = nn > (side == 0 ? lim_x : lim_y), near = row < np && !far;
             for (int cc = 0; cc < nc; ++cc) {
                 f16x8 p0, p1;
 #pragma unroll
                 for (int c = 0; c < 8; ++c) {
                     const int k = 16 * cc + 8 * (lane >> 5) + c;
-                    const float v = row < np && k < d ? (float)(p[(size_t)row * d + k] * s) : 0.0f;
+                    const float v = near && k < d ? (float)(p[(size_t)row * d + k] * s) : 0.0f;
                     const _Float16 a = (_Float16)v;
                     p0[c] = a;
                     p1[c] = (_Float16)(v - (float)a);
@@ -185,7 +220,10 @@ __global__ __launch_bounds__(256) void layout_kernel(const double* __restrict__ 
                 o[0] = p0;
                 o[64] = p1;
             }
-            if (lane < 32) f[row] = row < np ? (float)((side == 0 ? xx : yy)[row] * s * s) : 1.0e38f;
+            if (lane < 32) {
+                f[row] = near ? (float)(nn * s * s) : kOutside;
+                if (far) (side == 0 ? far_x : far_y)[atomicAdd(&st->far[side], 1u)] = (unsigned)row;
+            }
         }
     }
 }
@@ -240,7 +278,7 @@ __global__ __launch_bounds__(kApproxThreads) void approx_pass_kernel(
             const int blk = RB * rb + b < ntx ? RB * rb + b : ntx - 1;
             const bool twice = RB * rb + b >= ntx;           // a missing block repeats the last one: kept out by its |x|^2
             row[b] = blk * SK_TILE + (lane & 31);
-            xr[b] = twice ? 1.0e38f : xf[row[b]];
+            xr[b] = twice ? kOutside : xf[row[b]];
 #pragma unroll
             for (int c = 0; c < 2 * NC; ++c) xv[b][c / 2][c % 2] = xt[(size_t)blk * (NC * 128) + c * 64 + lane];
         }
@@ -414,6 +452,8 @@ __global__ __launch_bounds__(256) void bracket_kernel(const unsigned* __restrict
         const double c0 = (lb - 2.0 * err) / s2, c1 = (ub + 2.0 * err) / s2;
         const unsigned long long k0 = c0 > 0.0 ? (unsigned long long)__double_as_longlong(c0) : 0ull;
         const unsigned long long k1 = (unsigned long long)__double_as_longlong(c1 < 1.7e308 ? c1 : 1.7e308);
+        st->vlo = st->lo > 0.0f ? ((double)st->lo + err) / s2 : 0.0;      // what is below costs less than this
+        st->vhi = ((double)st->hi - err) / s2;                            // and what is above more than this
         st->base = k0;
         st->bits = k1 > k0 ? 64 - __clzll((long long)(k1 - k0)) : 1;
         // More pairs than the workspace holds in whole groups of 64 bins inside the bracket: not even tried. (The last
@@ -423,6 +463,59 @@ __global__ __launch_bounds__(256) void bracket_kernel(const unsigned* __restrict
         const int last = (int)(h0 < kHistBase ? 0u : h0 - kHistBase < kHistBins ? h0 - kHistBase : kHistBins - 1u) / 64 - 1;
         if (last >= first && part[last] - part[first - 1] > cap) st->fallback = 1;
     }
+}
+
+__device__ __forceinline__ unsigned long long exact_key(const double* __restrict__ xp, const double* __restrict__ yp,
+                                                        const double* __restrict__ xx, const double* __restrict__ yy, unsigned i,
+                                                        unsigned j, int dp) {
+    const double2* xr = reinterpret_cast<const double2*>(xp + (size_t)i * dp);
+    const double2* yr = reinterpret_cast<const double2*>(yp + (size_t)j * dp);
+    double acc = 0.0;
+    for (int k = 0; k < dp / 2; k += 4) {
+        double2 a[4], b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            a[q] = xr[k + q];
+            b[q] = yr[k + q];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = fma(a[q].y, b[q].y, fma(a[q].x, b[q].x, acc));
+    }
+    return cost_key((xx[i] + yy[j]) - 2.0 * acc);
+}
+
+// The pairs of the points set aside, by their float64 costs: below the bracket, inside it, or above. Every x with the far y,
+// every near y with the far x. With more of them than kFarPairs (a quarter of a millisecond at d 30) the full passes are
+// as good.
+constexpr unsigned long long kFarPairs = 1ull << 21;
+__global__ __launch_bounds__(256) void far_kernel(const unsigned* __restrict__ far_x, const unsigned* __restrict__ far_y,
+                                                  const float* __restrict__ yf, const double* __restrict__ xp,
+                                                  const double* __restrict__ yp, const double* __restrict__ xx,
+                                                  const double* __restrict__ yy, int n, int m, int dp, MedianState* st,
+                                                  unsigned* __restrict__ pairs, unsigned long long cap) {
+    const unsigned long long px = (unsigned long long)st->far[0] * (unsigned)m, py = (unsigned long long)st->far[1] * (unsigned)n;
+    if (px + py == 0 || px + py > kFarPairs) {
+        if (px + py != 0 && blockIdx.x == 0 && threadIdx.x == 0) st->fallback = 1;
+        return;
+    }
+    const unsigned long long base = st->base;
+    const int bits = st->bits;
+    unsigned long long below = 0;
+    for (unsigned long long e = (unsigned long long)blockIdx.x * 256 + threadIdx.x; e < px + py; e += (unsigned long long)gridDim.x * 256) {
+        const bool of_x = e < px;
+        const unsigned q = (unsigned)(of_x ? e : e - px), len = (unsigned)(of_x ? m : n), p = q / len, o = q - p * len;
+        const unsigned i = of_x ? far_x[p] : o, j = of_x ? o : far_y[p];
+        if (of_x && yf[j] == kOutside) continue;
+        const unsigned long long key = exact_key(xp, yp, xx, yy, i, j, dp), v = key - base;
+        if (key < base) {
+            ++below;
+        } else if (bits >= 64 || (v >> bits) == 0ull) {
+            const unsigned long long g = atomicAdd(&st->count, 1ull);
+            if (g < cap) pairs[g] = i * (unsigned)m + j;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o);
+    if ((threadIdx.x & 63) == 0 && below != 0) atomicAdd(&st->below, below);
 }
 
 // The float64 keys of the collected pairs, less the bracket's base; a key outside the bracket's bits (a cost further
@@ -448,20 +541,7 @@ __global__ __launch_bounds__(256) void exact_kernel(const unsigned* __restrict__
     for (unsigned long long e = (unsigned long long)blockIdx.x * 256 + threadIdx.x; e < count; e += (unsigned long long)gridDim.x * 256) {
         const unsigned idx = pairs[e];
         const unsigned i = idx / (unsigned)m, j = idx - i * (unsigned)m;
-        const double2* xr = reinterpret_cast<const double2*>(xp + (size_t)i * dp);
-        const double2* yr = reinterpret_cast<const double2*>(yp + (size_t)j * dp);
-        double acc = 0.0;
-        for (int k = 0; k < dp / 2; k += 4) {
-            double2 a[4], b[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                a[q] = xr[k + q];
-                b[q] = yr[k + q];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc = fma(a[q].y, b[q].y, fma(a[q].x, b[q].x, acc));
-        }
-        const unsigned long long key = cost_key((xx[i] + yy[j]) - 2.0 * acc);
+        const unsigned long long key = exact_key(xp, yp, xx, yy, i, j, dp);
         const unsigned long long v = key - base;
         if (key < base || (bits < 64 && (v >> bits) != 0ull)) st->fallback = 1;
         keys[e] = v;
@@ -551,7 +631,11 @@ __global__ __launch_bounds__(256) void select_cand_kernel(const unsigned long lo
         if (!same && (key & high) == p1) atomicAdd(&h[1][digit], 1u);
     }
     __syncthreads();
-    add_counts(&st->cand, h, hist, shift, width, (int)gridDim.x);
+    if (add_counts(&st->cand, h, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0 && (st->far[0] | st->far[1]) != 0u) {
+        const double a = __longlong_as_double((long long)(st->cand.prefix[0] + st->base));
+        const double b = __longlong_as_double((long long)(st->cand.prefix[1] + st->base));
+        if (!(a >= st->vlo && b <= st->vhi)) st->fallback = 1;
+    }
 }
 
 // One digit pass over the workgroup's block of 256 rows x `cols` columns, on the zero-padded copies (rows of
@@ -565,8 +649,8 @@ __global__ __launch_bounds__(256) void select_cand_kernel(const unsigned long lo
 typedef __attribute__((address_space(4))) const double ConstDouble;
 
 // KEEP: the pass also keeps the matching keys, if no workgroup has more than kKeepStage of them and all together no more
-// than cap; the later passes then read those (`kept_keys`) instead of recomputing every cost. 7,355 x 8,962 d 30 with one
-// point 60 times the others' norm: 703 us by this way, 1,145 with six full passes.
+// than cap; the later passes then read those (`kept_keys`) instead of recomputing every cost. A call at 7,355 x 8,962 d 30
+// that ends here takes 703 us by this way, 1,145 with six full passes.
 constexpr unsigned kKeepStage = 2048;
 template <bool KEEP>
 __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
@@ -684,7 +768,7 @@ unsigned long long cand_cap(int n, int m) {
 struct MedianLayout {
     int dp, mp, nc, ntx, nty, xblocks, yblocks, blocks;
     unsigned long long cap;
-    size_t state, hist, xx, yy, bmax, xp, yp, xt, yt, xf, yf, total, slabs, keys, bytes;
+    size_t state, hist, xx, yy, bmax, xp, yp, xt, yt, xf, yf, farx, fary, total, slabs, keys, bytes;
 };
 
 MedianLayout median_layout(int n, int m, int d) {
@@ -717,6 +801,8 @@ MedianLayout median_layout(int n, int m, int d) {
     o.yt = take((size_t)o.nty * o.nc * 2048);
     o.xf = take((size_t)o.ntx * SK_TILE * 4);
     o.yf = take((size_t)o.nty * SK_TILE * 4);
+    o.farx = take((size_t)n * 4);
+    o.fary = take((size_t)m * 4);
     o.total = take((size_t)(kHistBins + kSumBlocks) * 8);
     // the histogram slabs, then (they are done with by then) the collected pairs
     o.slabs = take(std::max((size_t)o.blocks * kHistBins * 4, (size_t)o.cap * 4));
@@ -771,7 +857,7 @@ int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, 
                        m, d, xx, yy, bmax, o.xblocks, st, hist);
     hipLaunchKernelGGL(layout_kernel, dim3(1024), dim3(256), 0, s, xc, n, yc, m, d, o.dp, o.mp, o.nc, xx, yy, bmax, o.xblocks,
                        o.yblocks, xp, yp, (f16x8*)(w + o.xt), (f16x8*)(w + o.yt), (float*)(w + o.xf), (float*)(w + o.yf),
-                       o.ntx, o.nty, st);
+                       o.ntx, o.nty, st, (unsigned*)(w + o.farx), (unsigned*)(w + o.fary));
     switch (o.nc) {
         case 1: launch_approx<1>(o, w, n, m, s); break;
         case 2: launch_approx<2>(o, w, n, m, s); break;
@@ -782,6 +868,9 @@ int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, 
         case 7: launch_approx<7>(o, w, n, m, s); break;
         default: launch_approx<8>(o, w, n, m, s); break;
     }
+    if (std::max(o.xblocks, o.yblocks) >= 8)          // else near_limit sets none aside
+        hipLaunchKernelGGL(far_kernel, dim3(256), dim3(256), 0, s, (const unsigned*)(w + o.farx), (const unsigned*)(w + o.fary),
+                           (const float*)(w + o.yf), xp, yp, xx, yy, n, m, o.dp, st, (unsigned*)(w + o.slabs), o.cap);
     hipLaunchKernelGGL(exact_kernel, dim3(1024), dim3(256), 0, s, (const unsigned*)(w + o.slabs), xp, yp, xx, yy, m, o.dp, st,
                        keys, o.cap);
     // Six digits at most; a typical bracket's keys differ in their low 43 bits (four digits, the other launches return).
