@@ -220,11 +220,11 @@ int sk_loop_init_f32(const sk_loop_f32* L, void* stream);
  * below that);
  * iterations after `done` do nothing. ws (sk_loop_workspace_bytes) must be 256-byte aligned. */
 int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream);
-/* The same iterations, bit for bit; where the problem is small (sk_loop_resident returns 1; else 0) as one cooperative
- * launch whose workgroups stay for all of them and pass the potentials to one another directly, else (and while the stream
- * captures, and for a single iteration) as sk_loop_run_f32. Cooperative launches of one device run one after another: for
- * a caller whose loops share the GPU on several streams sk_loop_run_f32 is the better form. If the workgroups should not
- * all get to run, the launch gives up after about a second, and a launch of one workgroup queued behind it runs the same
+/* The same iterations, bit for bit; where the problem is small (sk_loop_resident returns 1; else 0) as one launch whose
+ * workgroups stay for all of them and pass the potentials to one another directly, else (and while the stream captures, and
+ * for a single iteration) as sk_loop_run_f32. Keep the calls of one device on one stream: at the same time they hold CUs that
+ * the other waits for (a caller whose loops share the GPU on several streams takes sk_loop_run_f32). If the workgroups do
+ * not all get to run, the launch gives up after about a second, and a launch of one workgroup queued behind it runs the same
  * iterations again; how often that was since sk_loop_init_f32 is an int at byte sk_loop_repairs_offset of L->ws (0: the
  * problem has no such form). */
 int sk_loop_resident(const sk_loop_f32* L);

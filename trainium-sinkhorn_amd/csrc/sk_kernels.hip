@@ -1001,6 +1001,28 @@ int check_loop(const sk_loop_f32* L, const char* where) {
     return SK_OK;
 }
 
+bool resident(const LoopLayout& lo) { return lo.exchange != nullptr && log2_enabled() && loop_persists(lo.pf, lo.pg); }
+
+// The iterations of a checked call: as launches, or as one (may_stay) where the problem and the stream allow it.
+int run_loop(const sk_loop_f32* L, int iters, bool may_stay, hipStream_t hs, const char* where) {
+    const LoopLayout lo = loop_layout(L);
+    Pass f, g;
+    loop_passes(L, lo, f, g);
+    hipError_t e = hipSuccess;
+    if (may_stay && iters > 1 && resident(lo) && !capturing(hs)) {
+        const int ranks = loop_ranks(lo.pf, lo.pg);
+        e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc, ranks, ranks > 1 ? lo.pf.slots : 0,
+                        ranks > 1 ? lo.pg.slots : 0, env_int("TRNOPT_HIP_LOOP_POLLS", 0), hs);
+        return e == hipSuccess ? SK_OK : hip_fail(e, where);
+    }
+    for (int k = 0; k < iters; ++k) {
+        e = run_pass(f, lo.pf, hs);
+        if (e == hipSuccess) e = run_pass(g, lo.pg, hs);
+        if (e != hipSuccess) return hip_fail(e, where);
+    }
+    return SK_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1008,22 +1030,11 @@ extern "C" {
 int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream) {
     if (int r = check_loop(L, "sk_loop_run_f32")) return r;
     if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_f32: iters %d < 0", iters);
-    const LoopLayout lo = loop_layout(L);
-    Pass f, g;
-    loop_passes(L, lo, f, g);
-    hipStream_t hs = (hipStream_t)stream;
-    for (int k = 0; k < iters; ++k) {
-        hipError_t e = run_pass(f, lo.pf, hs);
-        if (e == hipSuccess) e = run_pass(g, lo.pg, hs);
-        if (e != hipSuccess) return hip_fail(e, "sk_loop_run_f32");
-    }
-    return SK_OK;
+    return run_loop(L, iters, false, (hipStream_t)stream, "sk_loop_run_f32");
 }
 
 int sk_loop_resident(const sk_loop_f32* L) {
-    if (check_loop(L, "sk_loop_resident") != SK_OK || !log2_enabled()) return 0;
-    const LoopLayout lo = loop_layout(L);
-    return lo.exchange != nullptr && loop_persists(lo.pf, lo.pg) ? 1 : 0;
+    return check_loop(L, "sk_loop_resident") == SK_OK && resident(loop_layout(L)) ? 1 : 0;
 }
 
 size_t sk_loop_repairs_offset(const sk_loop_f32* L) {
@@ -1038,14 +1049,7 @@ size_t sk_loop_repairs_offset(const sk_loop_f32* L) {
 int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream) {
     if (int r = check_loop(L, "sk_loop_run_resident_f32")) return r;
     if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_resident_f32: iters %d < 0", iters);
-    if (iters < 2 || sk_loop_resident(L) == 0 || capturing((hipStream_t)stream)) return sk_loop_run_f32(L, iters, stream);
-    const LoopLayout lo = loop_layout(L);
-    const int ranks = loop_ranks(lo.pf, lo.pg);
-    Pass f, g;
-    loop_passes(L, lo, f, g);
-    const hipError_t e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc, ranks, ranks > 1 ? lo.pf.slots : 0,
-                                    ranks > 1 ? lo.pg.slots : 0, env_int("TRNOPT_HIP_LOOP_POLLS", 0), (hipStream_t)stream);
-    return e == hipSuccess ? SK_OK : hip_fail(e, "sk_loop_run_resident_f32");
+    return run_loop(L, iters, true, (hipStream_t)stream, "sk_loop_run_resident_f32");
 }
 
 }  // extern "C"

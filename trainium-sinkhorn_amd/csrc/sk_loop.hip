@@ -14,11 +14,16 @@
 // row's segments are merged in the same order (merge_group); the control takes the same decisions from the same measures
 // (control_decide), each workgroup for itself.
 //
-// Every wait ends: the launch is cooperative (all its workgroups are resident), and a poll that has not seen its word after
-// `polls` rounds gives up: its workgroup ends without publishing, so that every other one's polls end the same way, and says
-// so in a word that nothing else writes. A launch of one workgroup behind it (repair_kernel, which returns at once
-// otherwise: 2 us) then runs the same iterations by itself from where the launch began, so that whoever reads the potentials
-// next, the caller or a kernel, finds them done.
+// Every wait ends. The launch has at most one workgroup per CU, which all run at once where the GPU is free or as soon as
+// other streams' workgroups leave their CUs; a poll that has not seen its word after `polls` rounds gives up: its workgroup
+// ends without publishing, so that every other one's polls end the same way, and says so in a word that nothing else writes.
+// A launch of one workgroup behind it (repair_kernel, 3 us where there is nothing to do) then runs the same iterations by
+// itself from where the launch began, so that whoever reads the potentials next, the caller or a kernel, finds them done.
+//
+// An ordinary launch, not a cooperative one: the first cooperative launch of a process makes the runtime open one more
+// hardware queue, and from then on everything that uses several streams runs slower (four single-cell pairs on streams of
+// their own 17 -> 54 ms). What it would add is that two such launches never share the GPU; they must not (each would hold CUs
+// that the other waits for, until both give up), so a caller keeps them on one stream.
 //
 // Where CUs would be idle, `ranks` workgroups share a row block: each takes every ranks-th segment, and rank 0 merges them all,
 // one exchange more and a ranks-th of the tiles (2,048 x 2,048 d 64, us an iteration: one rank 27.1, two 22.6, four 19.3).
@@ -644,11 +649,8 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void repair_kernel(LoopArgs a)
 
 template <int NC>
 hipError_t launch_nc(const LoopArgs& a, int workgroups, hipStream_t st) {
-    LoopArgs args = a;
-    void* params[] = {&args};
     const dim3 threads(64 * loop_waves(NC));
-    const hipError_t e = hipLaunchCooperativeKernel(loop_kernel<NC>, dim3(workgroups), threads, params, 0, st);
-    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(loop_kernel<NC>, dim3(workgroups), threads, 0, st, a);
     hipLaunchKernelGGL(repair_kernel<NC>, dim3(1), threads, 0, st, a);
     return hipGetLastError();
 }
