@@ -556,19 +556,22 @@ __device__ inline void select_digit(SelectState* st, unsigned* hist, int shift, 
     __shared__ unsigned long long below[2];
     const int tid = threadIdx.x;
     const int bins = 1 << width, per = (bins + 255) / 256;
-    const int same = st->same;
-    for (int s = 0; s < 2; ++s) {
-        const unsigned* hs = hist + (same ? 0 : s) * kBins;
-        unsigned c[kBins / 256];
+    const int same = st->same, hists = same ? 1 : 2;      // one histogram, scanned once, while the ranks share a prefix
+    for (int s = 0; s < hists; ++s) {
+        const unsigned* hs = hist + s * kBins;
+        unsigned c[kBins / 256];                 // all requested at once: the loads come from beyond this XCD's L2
         unsigned long long mine = 0;
-        for (int b = 0; b < per; ++b) {
-            c[b] = tid * per + b < bins ? __hip_atomic_load(hs + tid * per + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-            mine += c[b];
+#pragma unroll
+        for (int b = 0; b < kBins / 256; ++b) {
+            const bool in = b < per && tid * per + b < bins;
+            c[b] = in ? __hip_atomic_load(hs + tid * per + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
         }
+#pragma unroll
+        for (int b = 0; b < kBins / 256; ++b) mine += c[b];
         part[tid] = mine;
-        if (tid == 0) {
-            pick[s] = 0;
-            below[s] = 0ull;
+        if (tid < 2 && (same || tid == s)) {
+            pick[tid] = 0;
+            below[tid] = 0ull;
         }
         __syncthreads();
         for (int off = 1; off < 256; off <<= 1) {
@@ -577,13 +580,20 @@ __device__ inline void select_digit(SelectState* st, unsigned* hist, int shift, 
             part[tid] += v;
             __syncthreads();
         }
-        const unsigned long long k = st->k[s];
-        unsigned long long before = part[tid] - mine;
-        if (k >= before && k < before + mine) {
-            int b = 0;
-            while (k >= before + c[b]) before += c[b++];
-            pick[s] = tid * per + b;
-            below[s] = before;
+        for (int r = s; r < (same ? 2 : s + 1); ++r) {
+            const unsigned long long k = st->k[r];
+            unsigned long long before = part[tid] - mine;
+            if (k >= before && k < before + mine) {
+                int at = -1;
+#pragma unroll
+                for (int b = 0; b < kBins / 256; ++b)
+                    if (at < 0) {
+                        if (k < before + c[b]) at = b;
+                        else before += c[b];
+                    }
+                pick[r] = tid * per + at;
+                below[r] = before;
+            }
         }
         __syncthreads();
     }
@@ -595,12 +605,14 @@ __device__ inline void select_digit(SelectState* st, unsigned* hist, int shift, 
         st->same = (same && pick[0] == pick[1]) ? 1 : 0;
         st->arrived = 0;
     }
-    for (int b = tid; b < 2 * kBins; b += 256) hist[b] = 0u;
+    for (int b = tid; b < hists * kBins; b += 256) hist[b] = 0u;
 }
 
 // A workgroup's digit counts into the launch's, and the digit picked by the last workgroup to add its own (true there).
-__device__ inline bool add_counts(SelectState* st, const unsigned (&h)[2][kBins], unsigned* hist, int shift, int width, int blocks) {
-    for (int b = threadIdx.x; b < 2 * kBins; b += 256) {
+// same: as select_digit reads it.
+__device__ inline bool add_counts(SelectState* st, const unsigned (&h)[2][kBins], int same, unsigned* hist, int shift, int width,
+                                  int blocks) {
+    for (int b = threadIdx.x; b < (same ? 1 : 2) * kBins; b += 256) {
         const unsigned v = (&h[0][0])[b];
         if (v != 0u) atomicAdd(&hist[b], v);
     }
@@ -622,7 +634,7 @@ __global__ __launch_bounds__(256) void select_cand_kernel(const unsigned long lo
     const unsigned long long high = top >= 64 ? 0ull : ~((1ull << top) - 1ull);
     const unsigned long long p0 = st->cand.prefix[0] & high, p1 = st->cand.prefix[1] & high;
     const unsigned dmask = (1u << width) - 1u;
-    for (int b = tid; b < 2 * kBins; b += 256) (&h[0][0])[b] = 0u;
+    for (int b = tid; b < (same ? 1 : 2) * kBins; b += 256) (&h[0][0])[b] = 0u;
     __syncthreads();
     for (unsigned long long e = (unsigned long long)blockIdx.x * 256 + tid; e < c; e += (unsigned long long)gridDim.x * 256) {
         const unsigned long long key = keys[e];
@@ -631,7 +643,7 @@ __global__ __launch_bounds__(256) void select_cand_kernel(const unsigned long lo
         if (!same && (key & high) == p1) atomicAdd(&h[1][digit], 1u);
     }
     __syncthreads();
-    if (add_counts(&st->cand, h, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0 && (st->far[0] | st->far[1]) != 0u) {
+    if (add_counts(&st->cand, h, same, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0 && (st->far[0] | st->far[1]) != 0u) {
         const double a = __longlong_as_double((long long)(st->cand.prefix[0] + st->base));
         const double b = __longlong_as_double((long long)(st->cand.prefix[1] + st->base));
         if (!(a >= st->vlo && b <= st->vhi)) st->fallback = 1;
@@ -749,7 +761,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void select_pass_kernel(
             for (unsigned e = tid; e < nf; e += kRowsPerBlock)
                 if (base + e < cap) keys[base + e] = stage[e];
     }
-    if (add_counts(st, h, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0) {
+    if (add_counts(st, h, same, hist, shift, width, (int)gridDim.x) && shift == 0 && tid == 0) {
         const double a = __longlong_as_double((long long)st->prefix[0]);
         const double b = __longlong_as_double((long long)st->prefix[1]);
         *out = (a + b) * 0.5;
@@ -869,7 +881,7 @@ int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, 
         default: launch_approx<8>(o, w, n, m, s); break;
     }
     if (std::max(o.xblocks, o.yblocks) >= 8)          // else near_limit sets none aside
-        hipLaunchKernelGGL(far_kernel, dim3(256), dim3(256), 0, s, (const unsigned*)(w + o.farx), (const unsigned*)(w + o.fary),
+        hipLaunchKernelGGL(far_kernel, dim3(64), dim3(256), 0, s, (const unsigned*)(w + o.farx), (const unsigned*)(w + o.fary),
                            (const float*)(w + o.yf), xp, yp, xx, yy, n, m, o.dp, st, (unsigned*)(w + o.slabs), o.cap);
     hipLaunchKernelGGL(exact_kernel, dim3(1024), dim3(256), 0, s, (const unsigned*)(w + o.slabs), xp, yp, xx, yy, m, o.dp, st,
                        keys, o.cap);
