@@ -68,7 +68,6 @@ class _HipPlan:
         with torch.cuda.device(self.dev):
             self.X = hk.HipCloud(xs, log_a, self.dev, role=0)
             self.Y = hk.HipCloud(ys, log_b, self.dev, role=1)
-            self.X.sq, self.Y.sq = torch.zeros_like(self.X.sq), torch.zeros_like(self.Y.sq)
             self.sc = hk.scalars(eps, 1.0, self.dev)
 
     def lse(self, role: int, h_cols) -> torch.Tensor:
@@ -77,12 +76,13 @@ class _HipPlan:
         with torch.cuda.device(self.dev):
             h = np.zeros(C.npad, dtype=np.float32)
             h[:C.n] = h_cols
+            R.sq = torch.zeros_like(R.sq)
             out = self.hk.half_step(R, C, torch.from_numpy(h).to(self.dev), self.sc, use_off=False, log2=not self.baked)
         self.baked = True
         return out[:R.n]
 
     def read(self, *outs) -> list:
-        host = torch.cat(outs).to("cpu", torch.float64).numpy()
+        host = (outs[0] if len(outs) == 1 else torch.cat(outs)).to("cpu", torch.float64).numpy()
         return [-v / self.eps for v in np.split(host, np.cumsum([len(o) for o in outs])[:-1])]
 
 
