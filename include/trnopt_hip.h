@@ -265,7 +265,7 @@ int sk_loop_run_batch_f32(const void* ws, size_t ws_bytes, int count, const int*
  * sk_centre_f64: out = pts - centre, what sk_cost_median_f64 takes.
  * sk_prepare_cloud_f64: the packed cloud pk (as sk_pack_cloud_f32 makes it from the points cast to fp32), |p|^2 (float64
  * sums, cast; sk_pad_points(n) floats, 0 past n) and range, the largest |coordinate| in float64 (infinity if any is
- * * not finite): a caller refuses values above 7e13, as for sk_pack_cloud_f32.
+ * not finite): a caller refuses values above 7e13, as for sk_pack_cloud_f32.
  */
 size_t sk_cloud_stats_workspace_bytes(int d);
 int sk_cloud_stats_f64(const double* x, int n, const double* y, int m, int d, const int* pairs_x, const int* pairs_y,

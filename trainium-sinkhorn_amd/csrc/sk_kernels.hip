@@ -548,8 +548,8 @@ bool loop_fits(const Plan& pf, const Plan& pg) {
 }
 
 // Its workgroups per row block: up to 4 where they have CUs; one for up to kLoopLoneTiles tiles, which the waves of one take
-// at once. us an iteration by ranks 1 / 2 / 4 / 8: 100 x 90 d 30 11.5 / 12.7 / 12.5 / 12.3, 300 x 280 13.0 / 13.3 / 12.7 / 12.6,
-// 700 x 500 14.6 / 14.0 / 13.6 / 13.4, 1,000 x 1,000 d 64 19.7 / 18.1 / 17.4 / 17.4, 2,048 x 2,048 d 64 27.1 / 22.6 / 19.3.
+// at once. us an iteration by ranks 1 / 2 / 4 / 8: 100 x 90 d 30 9.6 / 10.6 / 10.4 / 10.3, 300 x 280 10.8 / 11.2 / 10.6 / 10.6,
+// 700 x 500 12.4 / 11.9 / 11.4 / 11.1, 1,000 x 1,000 d 64 17.9 / 16.1 / 15.5 / 15.7, 2,048 x 2,048 d 64 25.6 / 20.6 / 16.9.
 constexpr int kLoopMaxRanks = 4, kLoopLoneTiles = 8;
 int loop_ranks(const Plan& pf, const Plan& pg) {
     if (std::max(pf.nt, pg.nt) <= kLoopLoneTiles) return 1;
@@ -561,12 +561,12 @@ size_t loop_words(const Plan& pf, const Plan& pg) {
     return loop_exchange_words(pf.nrb * SK_TILE, pg.nrb * SK_TILE, shared ? pf.slots : 0, shared ? pg.slots : 0);
 }
 
-// And whether it is the faster one: an update costs it 5 to 7 us plus the tiles of a row block on `ranks` CUs, the launches
+// And whether it is the faster one: an update costs it 4 to 6 us plus the tiles of a row block on `ranks` CUs, the launches
 // 7-8 us plus the tiles spread over every CU. The line is tiles x 16-wide chunks per wave of a row block's workgroups. Measured
-// (us an iteration, launches against one launch of 10 iterations): 100 x 90 d 5 13.6 / 9.8, 700 x 500 d 16 17.0 / 11.7, d 64
-// 18.9 / 15.6, d 128 21.2 / 18.5, 2,048 x 2,048 d 16 18.3 / 13.9, d 30 19.0 / 16.0, d 64 21.1 / 19.1, 4,096 x 4,096 d 30 23.4 /
-// 21.1, 300 x 4,096 24.1 / 21.7; at the line 2,300 x 2,300 d 64 21.4 / 21.4; past it 3,000 x 3,000 d 64 24.0 / 25.5,
-// 4,300 x 4,300 d 30 24.2 / 26.7, 1,300 x 1,300 d 128 25.0 / 25.3. TRNOPT_HIP_LOOP=0 turns it off, =1 takes it wherever it fits.
+// (us an iteration, launches against one launch of 10 iterations): 100 x 90 d 5 13.0 / 8.0, 700 x 500 d 16 16.3 / 9.7, d 64
+// 18.1 / 13.5, d 128 20.4 / 16.6, 2,048 x 2,048 d 16 17.5 / 12.0, d 30 18.2 / 14.0, d 64 20.3 / 17.4, 4,096 x 4,096 d 30 21.9 /
+// 18.0, 300 x 4,096 23.7 / 20.3; at the line 2,300 x 2,300 d 64 21.0 / 19.2; past it 1,300 x 1,300 d 128 23.8 / 23.0,
+// 3,000 x 3,000 d 64 23.1 / 23.4, 4,300 x 4,300 d 30 22.9 / 24.7. TRNOPT_HIP_LOOP=0 turns it off, =1 takes it wherever it fits.
 constexpr int kLoopMaxWaveChunks = 8;
 bool loop_persists(const Plan& pf, const Plan& pg) {
     const int v = env_int("TRNOPT_HIP_LOOP", -1);

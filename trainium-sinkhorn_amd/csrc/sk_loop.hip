@@ -6,8 +6,8 @@
 // potentials and the arguments pass between them through memory. Here one workgroup per 32-row block of x and of y
 // stays for all the iterations; all that passes between workgroups is the new potentials, each as one 8-byte word
 // {value, iteration tag} that its readers poll: the data is its own flag, so an exchange costs one store and one load
-// across the XCDs and no barrier, fence or counter. 700 x 500 d 5: 16.9 -> 11.6 us an iteration, 100 x 90 14.5 -> 10.0,
-// 2,048 x 2,048 d 64 21.0 -> 19.3 (launches of 10 iterations; loop_persists has more sizes and both sides of its line).
+// across the XCDs and no barrier, fence or counter. 700 x 500 d 5: 16.2 -> 9.7 us an iteration, 100 x 90 13.0 -> 8.0,
+// 2,048 x 2,048 d 64 20.3 -> 17.4 (launches of 10 iterations; loop_persists has more sizes and both sides of its line).
 //
 // Bit for bit the launch-by-launch loop: a row block's columns are summed in the same segments as the split of the
 // partial kernel gives its row group (Split), each segment by one wave with the same instructions (sk_tile.h), and a
@@ -26,7 +26,7 @@
 // that the other waits for, until both give up), so a caller keeps them on one stream.
 //
 // Where CUs would be idle, `ranks` workgroups share a row block: each takes every ranks-th segment, and rank 0 merges them all,
-// one exchange more and a ranks-th of the tiles (2,048 x 2,048 d 64, us an iteration: one rank 27.1, two 22.6, four 19.3).
+// one exchange more and a ranks-th of the tiles (2,048 x 2,048 d 64, us an iteration: one rank 25.6, two 20.6, four 16.9).
 //
 // A potential's word is overwritten only after every reader has it: the next iteration's value is published by a
 // workgroup that has read all of the other cloud's values, each published by a workgroup that had read all of this one's.
