@@ -182,7 +182,8 @@ typedef struct sk_state {
     int it;               /* iterations done */
     int stage;            /* index into stages (n_stages = the final eps) */
     int stage_it;         /* iterations in the current stage */
-    int done;             /* 1: converged or max_iters reached; later loop kernels do nothing */
+    int done;             /* 1: converged or max_iters reached; later loop kernels do nothing. 2: as 1, after a launch of
+                           * sk_loop_try_resident_f32 gave up */
     int converged;
     int checks;           /* convergence checks run */
     float sc_x[4];        /* {2/eps, 1/eps, eps, kappa_x} of the next iteration (f update) */
@@ -226,10 +227,16 @@ int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream);
  * the other waits for (a caller whose loops share the GPU on several streams takes sk_loop_run_f32). If the workgroups do
  * not all get to run, the launch gives up after about a second, and a launch of one workgroup queued behind it runs the same
  * iterations again; how often that was since sk_loop_init_f32 is an int at byte sk_loop_repairs_offset of L->ws (0: the
- * problem has no such form). */
+ * problem has no such form).
+ * sk_loop_try_resident_f32 leaves that second launch out, and gives up after a few ms if not all workgroups get to run by the
+ * first iteration: the state is then the one the launch began with but for done = 2, and launches already queued behind it do
+ * nothing. For a caller that reads the state: sk_loop_recover_f32 takes the loop back to where that launch began and runs
+ * `iters` iterations (all those queued that the state does not count) as launches. */
 int sk_loop_resident(const sk_loop_f32* L);
 size_t sk_loop_repairs_offset(const sk_loop_f32* L);
 int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream);
+int sk_loop_try_resident_f32(const sk_loop_f32* L, int iters, void* stream);
+int sk_loop_recover_f32(const sk_loop_f32* L, int iters, void* stream);
 
 /*
  * Several loops at once: `count` independent solves of the same d (each set up and initialised as above, on its

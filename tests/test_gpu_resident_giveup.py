@@ -1,5 +1,6 @@
-"""A resident launch whose waits run out (TRNOPT_HIP_LOOP_POLLS=1: a single poll each) is made good on the device: whoever
-enqueued the iterations finds them done, without having looked at the state, bit for bit as launches do them."""
+"""A resident launch whose waits run out (TRNOPT_HIP_LOOP_POLLS: a few polls each) is made good on the device: whoever
+enqueued the iterations finds them done, without having looked at the state, bit for bit as launches do them. A whole run,
+which reads the state, goes on as launches from where that launch began, with the same results."""
 
 import ctypes
 
@@ -54,6 +55,28 @@ def test_enqueued_iterations_are_done(hip, monkeypatch, n, m, d, form):
         assert torch.equal(p, q)
     np.testing.assert_array_equal(got[0][1], got[1][1])
     assert torch.equal(got[0][2][:28], got[1][2][:28])
+
+
+@pytest.mark.parametrize("polls", [2, 4, 6, 9, 14])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_a_give_up_on_the_way_changes_nothing(hip, monkeypatch, form, polls):
+    """With a few polls a wait runs out in some iteration or in none: enqueued calls and whole runs alike."""
+    n, m, d = 700, 500, 30
+    print(f"give-up on the way {form} {polls} polls", flush=True)
+    monkeypatch.setenv("TRNOPT_HIP_LOOP", "0")
+    want = _loop(hip, n, m, d, form)
+    end = _state(want.run())
+    monkeypatch.setenv("TRNOPT_HIP_LOOP", "1")
+    monkeypatch.setenv("TRNOPT_HIP_LOOP_POLLS", str(polls))
+    runs, calls = _loop(hip, n, m, d, form), _loop(hip, n, m, d, form)
+    np.testing.assert_array_equal(_state(runs.run()), end)
+    calls.init()
+    for _ in range(9):
+        calls.enqueue(10)
+    np.testing.assert_array_equal(_state(calls.read_state()), end)
+    for l in (runs, calls):
+        assert torch.equal(l.fh, want.fh) and torch.equal(l.gh, want.gh)
+    print("runs made good:", runs.repairs(), calls.repairs(), flush=True)
 
 
 def test_no_launch_gives_up_by_itself(hip, monkeypatch):

@@ -39,15 +39,15 @@ def _both(monkeypatch, n, m, d, o, x=None):
     kw = dict(a_target=a[::-1].copy(), b_target=b) if "rho" in o else {}
     out = []
     lib = hk.lib()
-    run = lib.sk_loop_run_resident_f32
+    run = lib.sk_loop_try_resident_f32
     for v in ("0", "1"):
         resident = []                        # the form that each call of the loop's iterations takes
         monkeypatch.setenv("TRNOPT_HIP_LOOP", v)
-        monkeypatch.setattr(lib, "sk_loop_run_resident_f32",
+        monkeypatch.setattr(lib, "sk_loop_try_resident_f32",
                             lambda L, k, stream: (resident.append(lib.sk_loop_resident(L)), run(L, k, stream))[1])
         out.append(sinkhorn(x0 if x is None else x, y, a, b, SinkhornOptions(kernel="hip", backend=ROCM, **o), **kw))
         assert resident and set(resident) == {int(v)}
-    monkeypatch.setattr(lib, "sk_loop_run_resident_f32", run)
+    monkeypatch.setattr(lib, "sk_loop_try_resident_f32", run)
     return out
 
 
@@ -111,7 +111,7 @@ def test_mixed_calls_continue_one_loop(hip, monkeypatch):
 
 @pytest.mark.parametrize("form", ["fixed", "converged", "stages"])
 def test_a_launch_that_gives_up_is_run_again_as_launches(hip, monkeypatch, form):
-    """With a single poll allowed, any wait gives up: the iterations are run again with the result of launches."""
+    """With a single poll allowed, any wait gives up: the solve goes on in launches from there with the same result."""
     monkeypatch.setenv("TRNOPT_HIP_LOOP_POLLS", "1")
     loops, init = [], hip.DeviceLoop.init
     monkeypatch.setattr(hip.DeviceLoop, "init", lambda loop: (loops.append(loop), init(loop))[1])

@@ -1,6 +1,11 @@
-"""A small solve leaves the rest of the process as fast as it was: pairs on streams of their own take as long in a process
+"""Several streams and several processes on one GPU beside the one-launch loop.
+
+A small solve leaves the rest of the process as fast as it was: pairs on streams of their own take as long in a process
 whose first solve ran as one launch as in one whose first solve ran as launches. (One launched cooperatively makes the
-runtime open a hardware queue more: four pairs in flight took 54 ms after it, 17 without.)"""
+runtime open a hardware queue more: four pairs in flight took 54 ms after it, 17 without.)
+
+Processes that share the GPU all get their results. (A cooperative launch was refused where another process had made one.
+Ordinary ones may share the CUs so that each waits for the rest of its own: they give up and go on as launches.)"""
 
 import os
 import re
@@ -48,3 +53,50 @@ def test_pairs_on_streams_are_as_fast_after_a_one_launch_solve(hip):
         seconds.append(float(r.stdout.split("median")[1]))
         print("first solve", "as one launch" if v == "1" else "as launches", seconds[-1], flush=True)
     assert seconds[1] <= 2.0 * seconds[0]
+
+
+SOLVES = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+from trnopt import Backend, SinkhornOptions, hip_sinkhorn, sinkhorn
+rng = np.random.default_rng(5)
+x, y = rng.normal(size=(2000, 30)), rng.normal(size=(2040, 30))
+rocm = Backend.preset("rocm")
+fixed = SinkhornOptions(kernel="hip", backend=rocm, eps=0.1, max_iters=60, fixed_iters=True)
+checked = SinkhornOptions(kernel="hip", backend=rocm, eps=0.2, tol=1e-6, max_iters=80)
+loops, init = [], hip_sinkhorn.DeviceLoop.init
+hip_sinkhorn.DeviceLoop.init = lambda l: (loops.append(l), init(l))[1]
+first = [sinkhorn(x, y, opts=o) for o in (fixed, checked)]
+print("ready", flush=True)
+sys.stdin.readline()
+for _ in range(25):
+    for o, want in zip((fixed, checked), first):
+        r = sinkhorn(x, y, opts=o)
+        assert r.iterations == want.iterations
+        np.testing.assert_array_equal(r.f, want.f)
+        np.testing.assert_array_equal(r.g, want.g)
+print("done", len(loops), sum(l.repairs() for l in loops[-20:]), flush=True)
+"""
+
+
+@pytest.mark.gpu
+def test_processes_that_share_the_gpu(hip):
+    """Four processes of solves whose loops would each take most of the CUs."""
+    ps = [subprocess.Popen([sys.executable, "-c", SOLVES, str(ROOT / "trainium-sinkhorn_amd")], stdin=subprocess.PIPE,
+                           stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True) for _ in range(4)]
+    try:
+        for p in ps:
+            assert p.stdout.readline().startswith("ready"), p.stderr.read()[-2000:]
+        for p in ps:
+            p.stdin.write("go\n")
+            p.stdin.flush()
+        for p in ps:
+            out, err = p.communicate(timeout=60)
+            assert p.returncode == 0 and "done" in out, err[-2000:]
+            print(out.strip(), flush=True)
+    finally:
+        for p in ps:
+            if p.poll() is None:
+                p.kill()
+                p.wait()

@@ -218,19 +218,23 @@ int hip_fail(hipError_t e, const char* where);
 // Several iterations of the loop with passes f and g in one launch (sk_loop.hip): both clouds of at most kLoopMaxBlocks
 // row blocks (one workgroup each and CU) and kLoopMaxTiles tiles. exchange: loop_exchange_words 8-byte words, zero at
 // loop init.
-constexpr int kLoopMaxTiles = 192, kLoopMaxBlocks = 256, kLoopSavedWords = 34;
+constexpr int kLoopMaxTiles = 192, kLoopMaxBlocks = 256, kLoopNoteWords = 32;
 inline size_t loop_exchange_words(int nx_pad, int ny_pad, int slots_x, int slots_y) {
-    return (size_t)nx_pad * (1 + 2 * slots_x) + (size_t)ny_pad * (2 + 2 * slots_y) + 6 * (size_t)(ny_pad / 32) + kLoopSavedWords;
+    return (size_t)nx_pad * (1 + 2 * slots_x) + (size_t)ny_pad * (2 + 2 * slots_y) + 6 * (size_t)(ny_pad / 32) + kLoopNoteWords;
 }
 // Byte offset in the exchange of the 4-byte count of launches that gave up and were run again.
-size_t loop_repairs_at(int nx_pad, int ny_pad, int slots_x, int slots_y);
+size_t loop_repairs_at();
 // Waves of a workgroup: as many as hide each other's latencies with the tile loop's operands in registers (128, 168, 256 a
-// lane). Around the tile loop the compiler spills: 4, 26, 16, 48, 0, 25, 56, 87 registers a lane at kp 16, 32, ... 128 and
-// 102 to 117 scalars at each; the tile loops themselves have no scratch access.
+// lane). Around the tile loop the compiler spills: 4, 25, 17, 45, 0, 26, 54, 87 registers a lane at kp 16, 32, ... 128 and
+// 104 to 111 scalars at each; the tile loops themselves have no scratch access.
 constexpr int loop_waves(int nc) { return nc <= 2 ? 16 : nc <= 4 ? 12 : 8; }
-// ranks: workgroups that share a row block; slots_x, slots_y: the most segments of one, for ranks > 1 (else 0).
+// ranks: workgroups that share a row block; slots_x, slots_y: the most segments of one, for ranks > 1 (else 0). repair: a
+// launch that gives up is run again on the device, else it leaves the state's done at 2 and launch_recover takes the loop
+// back to where it began.
 hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int ranks, int slots_x,
-                       int slots_y, int polls, hipStream_t stream);
+                       int slots_y, int polls, bool repair, hipStream_t stream);
+hipError_t launch_recover(const PartialArgs& f, const PartialArgs& g, void* exchange, int ranks, int slots_x, int slots_y,
+                          hipStream_t stream);
 hipError_t launch_partial_small(const PartialArgs& a, int nc, hipStream_t stream);
 hipError_t launch_partial_large(const PartialArgs& a, int nc, hipStream_t stream);
 inline hipError_t launch_partial(const PartialArgs& a, int nc, hipStream_t stream) {

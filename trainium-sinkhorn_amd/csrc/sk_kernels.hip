@@ -1003,18 +1003,24 @@ int check_loop(const sk_loop_f32* L, const char* where) {
 
 bool resident(const LoopLayout& lo) { return lo.exchange != nullptr && log2_enabled() && loop_persists(lo.pf, lo.pg); }
 
-// The iterations of a checked call: as launches, or as one (may_stay) where the problem and the stream allow it.
-int run_loop(const sk_loop_f32* L, int iters, bool may_stay, hipStream_t hs, const char* where) {
+// The iterations of a checked call: as launches, or as one where the problem and the stream allow it (with the launch that
+// makes a give-up good, or without), or as launches from where a launch that gave up began.
+enum LoopForm { kLaunches, kStay, kTryStay, kRecover };
+int run_loop(const sk_loop_f32* L, int iters, LoopForm form, hipStream_t hs, const char* where) {
     const LoopLayout lo = loop_layout(L);
     Pass f, g;
     loop_passes(L, lo, f, g);
     hipError_t e = hipSuccess;
-    if (may_stay && iters > 1 && resident(lo) && !capturing(hs)) {
-        const int ranks = loop_ranks(lo.pf, lo.pg);
-        e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc, ranks, ranks > 1 ? lo.pf.slots : 0,
-                        ranks > 1 ? lo.pg.slots : 0, env_int("TRNOPT_HIP_LOOP_POLLS", 0), hs);
+    const int ranks = lo.exchange != nullptr ? loop_ranks(lo.pf, lo.pg) : 1;
+    const int slots_x = ranks > 1 ? lo.pf.slots : 0, slots_y = ranks > 1 ? lo.pg.slots : 0;
+    if ((form == kStay || form == kTryStay) && iters > 1 && resident(lo) && !capturing(hs)) {
+        e = launch_loop(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, iters, lo.pf.nc, ranks, slots_x, slots_y,
+                        env_int("TRNOPT_HIP_LOOP_POLLS", 0), form == kStay, hs);
         return e == hipSuccess ? SK_OK : hip_fail(e, where);
     }
+    if (form == kRecover && lo.exchange != nullptr && f.rebake != nullptr)
+        e = launch_recover(pass_args(f, lo.pf), pass_args(g, lo.pg), lo.exchange, ranks, slots_x, slots_y, hs);
+    if (e != hipSuccess) return hip_fail(e, where);
     for (int k = 0; k < iters; ++k) {
         e = run_pass(f, lo.pf, hs);
         if (e == hipSuccess) e = run_pass(g, lo.pg, hs);
@@ -1030,7 +1036,7 @@ extern "C" {
 int sk_loop_run_f32(const sk_loop_f32* L, int iters, void* stream) {
     if (int r = check_loop(L, "sk_loop_run_f32")) return r;
     if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_f32: iters %d < 0", iters);
-    return run_loop(L, iters, false, (hipStream_t)stream, "sk_loop_run_f32");
+    return run_loop(L, iters, kLaunches, (hipStream_t)stream, "sk_loop_run_f32");
 }
 
 int sk_loop_resident(const sk_loop_f32* L) {
@@ -1040,16 +1046,25 @@ int sk_loop_resident(const sk_loop_f32* L) {
 size_t sk_loop_repairs_offset(const sk_loop_f32* L) {
     if (check_loop(L, "sk_loop_repairs_offset") != SK_OK) return 0;
     const LoopLayout lo = loop_layout(L);
-    if (lo.exchange == nullptr) return 0;
-    const bool shared = loop_ranks(lo.pf, lo.pg) > 1;
-    return (size_t)((char*)lo.exchange - (char*)L->ws) +
-           loop_repairs_at(lo.pf.nrb * SK_TILE, lo.pg.nrb * SK_TILE, shared ? lo.pf.slots : 0, shared ? lo.pg.slots : 0);
+    return lo.exchange == nullptr ? 0 : (size_t)((char*)lo.exchange - (char*)L->ws) + loop_repairs_at();
 }
 
 int sk_loop_run_resident_f32(const sk_loop_f32* L, int iters, void* stream) {
     if (int r = check_loop(L, "sk_loop_run_resident_f32")) return r;
     if (iters < 0) return fail(SK_E_ARG, "sk_loop_run_resident_f32: iters %d < 0", iters);
-    return run_loop(L, iters, true, (hipStream_t)stream, "sk_loop_run_resident_f32");
+    return run_loop(L, iters, kStay, (hipStream_t)stream, "sk_loop_run_resident_f32");
+}
+
+int sk_loop_try_resident_f32(const sk_loop_f32* L, int iters, void* stream) {
+    if (int r = check_loop(L, "sk_loop_try_resident_f32")) return r;
+    if (iters < 0) return fail(SK_E_ARG, "sk_loop_try_resident_f32: iters %d < 0", iters);
+    return run_loop(L, iters, kTryStay, (hipStream_t)stream, "sk_loop_try_resident_f32");
+}
+
+int sk_loop_recover_f32(const sk_loop_f32* L, int iters, void* stream) {
+    if (int r = check_loop(L, "sk_loop_recover_f32")) return r;
+    if (iters < 0) return fail(SK_E_ARG, "sk_loop_recover_f32: iters %d < 0", iters);
+    return run_loop(L, iters, kRecover, (hipStream_t)stream, "sk_loop_recover_f32");
 }
 
 }  // extern "C"

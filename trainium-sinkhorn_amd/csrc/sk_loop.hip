@@ -16,9 +16,15 @@
 //
 // Every wait ends. The launch has at most one workgroup per CU, which all run at once where the GPU is free or as soon as
 // other streams' workgroups leave their CUs; a poll that has not seen its word after `polls` rounds gives up: its workgroup
-// ends without publishing, so that every other one's polls end the same way, and says so in a word that nothing else writes.
-// A launch of one workgroup behind it (repair_kernel, 3 us where there is nothing to do) then runs the same iterations by
-// itself from where the launch began, so that whoever reads the potentials next, the caller or a kernel, finds them done.
+// ends without publishing, so that every other one's polls end the same way. The first workgroup, which waits for all the
+// others' last words before it writes the state, then writes done = 2 instead and nothing else: the state and the copy's header
+// are those the launch began with, y's potentials are saved (`rows`), and launches queued behind do nothing. From there the
+// iterations are run again: by one workgroup in a launch queued behind (repair_kernel, 3 us where there is nothing to do), so
+// that whoever reads the potentials next, the caller or a kernel, finds them done; or, for a host that looks at the state
+// anyway, as ordinary launches (launch_recover), at their speed. When workgroups of several processes share the GPU's CUs,
+// each waiting for the rest of its own, that is what ends it, so the first iteration, after which all are known to run, has
+// fewer polls in that second form. Four processes side by side, each in 2,048 x 2,048 d 64 solves: 5.4-6.9 ms a solve (launches
+// 12.5-12.8), one in 25 with a give-up and then 17-69 ms; with a second's polls and the repair on the device up to 1.1 s.
 //
 // An ordinary launch, not a cooperative one: the first cooperative launch of a process makes the runtime open one more
 // hardware queue, and from then on everything that uses several streams runs slower (four single-cell pairs on streams of
@@ -33,6 +39,8 @@
 
 #include <stddef.h>
 
+#include <atomic>
+
 #include "sk_common.h"
 #include "sk_epilogue.h"
 #include "sk_tile.h"
@@ -41,6 +49,7 @@ namespace sk {
 namespace {
 
 constexpr int kMaxPolls = 1 << 20;                  // of a word before a workgroup gives up: about a second
+constexpr int kFirstPolls = 1 << 11;                // in the first iteration, where giving up is cheap: a few ms
 constexpr int kRowsOfBlock = 32;
 
 typedef unsigned long long u64;
@@ -334,24 +343,21 @@ __device__ inline bool control(const PartialArgs& g, const u64* msr, unsigned ta
     return ctl.st.done != 0;
 }
 
-// Where a launch began, for repair_kernel to begin there again: saved by the launch's workgroups before they do anything
-// else (one that starts after another has given up as well: nothing of its rows has changed by then).
-struct Saved {
-    sk_state st;
-    CopyTag tag;
-    char apart[168];      // (a cache line away from what another XCD's workgroup stores plainly)
-    int gave_up;          // a workgroup of the launch has
+// The head of the exchange (zero at loop init).
+struct Notes {
+    int gave_up;          // the launch (LoopArgs::id) of which a workgroup has given up last
     int repairs;          // launches run again since the loop's init
 };
-static_assert(sizeof(Saved) <= 8 * kLoopSavedWords, "the exchange has kLoopSavedWords words for it");
+static_assert(sizeof(Notes) <= 8 * kLoopNoteWords, "the exchange begins with kLoopNoteWords words for it");
 
 struct LoopArgs {
     PartialArgs f, g;
     u64 *ex, *ey, *msr;      // the potentials of x and y and (two turns of) the measures of y's row blocks, tagged words
     u64 *sx, *sy;            // the segments' (M, S) of the ranks above 0 (Rank)
     float2* rows;            // y's potentials where the launch began: gh and its log2-unit potential
-    Saved* saved;
-    int iters, polls, ranks;
+    Notes* notes;
+    int id;                  // of this launch, not 0: another one's for every launch of the process
+    int iters, polls, first_polls, ranks;
     int slots_x, slots_y;    // segments of a row block, at most
 };
 
@@ -432,22 +438,21 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     const int i = w * kRowsOfBlock + tid;
     const bool rx = has_x && rank == 0 && tid < kRowsOfBlock, ry = has_y && rank == 0 && tid < kRowsOfBlock;
     float fh = rx ? a.f.out[i] : 0.0f, fr = rx ? a.f.out2[i] : 0.0f, gh = ry ? a.g.out[i] : 0.0f, gr = ry ? a.g.out2[i] : 0.0f;
-    if (ry) a.rows[i] = make_float2(gh, gr);
-    const sk_state* gst = a.g.state;
-    const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
-    if (w == 0 && rank == 0 && tid == 0) {
-        a.saved->st = *gst;
-        a.saved->tag = tag;
-    }
+    sk_state* const gst = a.g.state;
     if (tid == 0) {
+        // by one thread: workgroups that have given up already may be writing both
+        const int was_done = coh_load(&gst->done);
+        __threadfence();
+        ctl.abort = coh_load(&a.notes->gave_up) == a.id ? 1 : 0;
         ctl.st = *gst;
+        ctl.st.done = ctl.abort != 0 ? 0 : was_done;
+        const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
         ctl.c = tag.c;
         ctl.t = tag.t;
         ctl.s2 = tag.s2;
         ctl.pending = tag.pending;
         ctl.unseen = 0;
-        ctl.polls = a.polls;
-        ctl.abort = coh_load(&a.saved->gave_up);      // by one thread: another workgroup may be setting it
+        ctl.polls = a.first_polls;
     }
     u64* const sx = a.sx + (size_t)w * a.slots_x * kRowsOfBlock * 2;
     u64* const sy = a.sy + (size_t)w * a.slots_y * kRowsOfBlock * 2;
@@ -456,9 +461,14 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     const float y2 = ry ? a.g.xsq[i] : 0.0f, yo = ry && a.g.off != nullptr ? a.g.off[i] : 0.0f, yl = ry ? a.g.rows_l2lo[i] : 0.0f;
     const float yw = ry ? a.g.w[i] : 0.0f;
     __syncthreads();
-    const bool idle = ctl.st.done != 0 || ctl.abort != 0;
+    const bool done_before = ctl.st.done != 0, late = ctl.abort != 0;
     __syncthreads();                       // every wave has the same answer before one may set abort
-    if (idle) return;
+    if (done_before) return;
+    if (ry) a.rows[i] = make_float2(gh, gr);       // (a late workgroup's rows too: nothing has changed them)
+    if (late) {
+        if (w == 0 && rank == 0 && tid == 0) coh_store(&gst->done, 2);
+        return;
+    }
     unsigned ytag = 0u;                    // the tag of y's latest potentials (0: in memory)
     bool done = false;
     for (int k = 0; k < a.iters && !done; ++k) {
@@ -524,6 +534,7 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
             publish(a.ey + i, __float_as_uint(next_l2 ? gr : gh), tag + 1u);
         }
         ytag = tag + 1u;
+        if (k == 0 && tid == 0) ctl.polls = a.polls;
         __syncthreads();
     }
     if (rx) {
@@ -535,7 +546,8 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
         a.g.out2[i] = gr;
     }
     // The state and the copy's header, once every workgroup has read them (they all have published y's last values, or
-    // x's that those rest on).
+    // x's that those rest on). A workgroup that gives up after that, in its last control, has stored its rows above and owes
+    // nobody anything.
     if (w == 0 && rank == 0 && ctl.abort == 0) {
         bool all = true;
         for (int j = tid; j < a.g.nrb; j += NT) {
@@ -547,7 +559,11 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void loop_kernel(LoopArgs a) {
     }
     __syncthreads();
     if (ctl.abort != 0) {
-        if (tid == 0) coh_store(&a.saved->gave_up, 1);
+        if (tid == 0) {
+            coh_store(&a.notes->gave_up, a.id);
+            __threadfence();
+            if (w == 0 && rank == 0) coh_store(&gst->done, 2);
+        }
         return;
     }
     if (w == 0 && rank == 0 && tid == 0) write_back(a, ctl);
@@ -564,13 +580,14 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void repair_kernel(LoopArgs a)
     __shared__ float lds_mx[kLoopMaxBlocks];
     __shared__ double lds_sm[kLoopMaxBlocks];
     __shared__ Ctl ctl;
-    if (a.saved->gave_up == 0) return;
+    if (a.g.state->done != 2) return;
     const int tid = tid_x();
     const Rank alone = {0, 1, nullptr, 0u};
     const LoopCfg& cfg = a.g.cfg;
     if (tid == 0) {
-        const CopyTag tag = a.saved->tag;
-        ctl.st = a.saved->st;
+        const CopyTag tag = copy_tag(reinterpret_cast<const float*>(a.f.xr), true);
+        ctl.st = *a.g.state;
+        ctl.st.done = 0;
         ctl.c = tag.c;
         ctl.t = tag.t;
         ctl.s2 = tag.s2;
@@ -642,52 +659,90 @@ __global__ __launch_bounds__(64 * loop_waves(NC)) void repair_kernel(LoopArgs a)
     }
     if (tid == 0) {
         write_back(a, ctl);
-        a.saved->gave_up = 0;
-        a.saved->repairs += 1;
+        a.notes->repairs += 1;
+    }
+}
+
+// Back to where a launch that gave up began, for launches to go on from. The copy's tiles may be those of an eps that the
+// launch had reached: this loop's copy is made anew by the next f update, another's is dropped.
+__global__ __launch_bounds__(256) void recover_kernel(LoopArgs a) {
+    __shared__ int failed;
+    const int tid = tid_x();
+    if (tid == 0) failed = a.g.state->done == 2 ? 1 : 0;
+    __syncthreads();
+    if (failed == 0) return;
+    for (int i = tid; i < a.g.nrb * kRowsOfBlock; i += 256) {
+        const float2 v = a.rows[i];
+        a.g.out[i] = v.x;
+        a.g.out2[i] = v.y;
+    }
+    if (tid != 0) return;
+    a.g.state->done = 0;
+    a.notes->repairs += 1;
+    float* h = reinterpret_cast<float*>(a.f.rebake);
+    const CopyTag tag = copy_tag(h, true);
+    h[2] = 0.0f;
+    if (tag.c != 0.0f && tag.c == a.g.state->sc_x[0] * kLog2e && tag.s2 == packed_scale(a.f.yc)) {
+        h[7] = tag.c;
+        h[8] = tag.t;
+        reinterpret_cast<int*>(h)[6] = 1;
     }
 }
 
 template <int NC>
-hipError_t launch_nc(const LoopArgs& a, int workgroups, hipStream_t st) {
+hipError_t launch_nc(const LoopArgs& a, int workgroups, bool repair, hipStream_t st) {
     const dim3 threads(64 * loop_waves(NC));
     hipLaunchKernelGGL(loop_kernel<NC>, dim3(workgroups), threads, 0, st, a);
-    hipLaunchKernelGGL(repair_kernel<NC>, dim3(1), threads, 0, st, a);
+    if (repair) hipLaunchKernelGGL(repair_kernel<NC>, dim3(1), threads, 0, st, a);
     return hipGetLastError();
 }
 
-}  // namespace
-
-size_t loop_repairs_at(int nx_pad, int ny_pad, int slots_x, int slots_y) {
-    return 8 * (loop_exchange_words(nx_pad, ny_pad, slots_x, slots_y) - kLoopSavedWords) + offsetof(Saved, repairs);
-}
-
-hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int ranks, int slots_x,
-                       int slots_y, int polls, hipStream_t st) {
+LoopArgs loop_args(const PartialArgs& f, const PartialArgs& g, void* exchange, int ranks, int slots_x, int slots_y) {
     LoopArgs a;
     a.f = f;
     a.g = g;
-    a.ex = (u64*)exchange;
+    a.notes = (Notes*)exchange;
+    a.ex = (u64*)exchange + kLoopNoteWords;
     a.ey = a.ex + f.rows_pad;
     a.msr = a.ey + g.rows_pad;
     a.sx = a.msr + 6 * (size_t)g.nrb;
     a.sy = a.sx + (size_t)f.nrb * slots_x * kRowsOfBlock * 2;
     a.rows = (float2*)(a.sy + (size_t)g.nrb * slots_y * kRowsOfBlock * 2);
-    a.saved = (Saved*)(a.rows + g.rows_pad);
     a.slots_x = slots_x;
     a.slots_y = slots_y;
     a.ranks = ranks;
+    a.id = a.iters = a.polls = a.first_polls = 0;
+    return a;
+}
+
+}  // namespace
+
+size_t loop_repairs_at() { return offsetof(Notes, repairs); }
+
+hipError_t launch_recover(const PartialArgs& f, const PartialArgs& g, void* exchange, int ranks, int slots_x, int slots_y,
+                          hipStream_t st) {
+    hipLaunchKernelGGL(recover_kernel, dim3(1), dim3(256), 0, st, loop_args(f, g, exchange, ranks, slots_x, slots_y));
+    return hipGetLastError();
+}
+
+hipError_t launch_loop(const PartialArgs& f, const PartialArgs& g, void* exchange, int iters, int nc, int ranks, int slots_x,
+                       int slots_y, int polls, bool repair, hipStream_t st) {
+    static std::atomic<unsigned> launches{0};
+    LoopArgs a = loop_args(f, g, exchange, ranks, slots_x, slots_y);
+    a.id = (int)(launches.fetch_add(1, std::memory_order_relaxed) << 1 | 1u);
     a.iters = iters;
     a.polls = polls > 0 ? polls : kMaxPolls;
+    a.first_polls = repair || polls > 0 ? a.polls : kFirstPolls;
     const int wgs = (f.nrb > g.nrb ? f.nrb : g.nrb) * ranks;
     switch (nc) {
-        case 1: return launch_nc<1>(a, wgs, st);
-        case 2: return launch_nc<2>(a, wgs, st);
-        case 3: return launch_nc<3>(a, wgs, st);
-        case 4: return launch_nc<4>(a, wgs, st);
-        case 5: return launch_nc<5>(a, wgs, st);
-        case 6: return launch_nc<6>(a, wgs, st);
-        case 7: return launch_nc<7>(a, wgs, st);
-        case 8: return launch_nc<8>(a, wgs, st);
+        case 1: return launch_nc<1>(a, wgs, repair, st);
+        case 2: return launch_nc<2>(a, wgs, repair, st);
+        case 3: return launch_nc<3>(a, wgs, repair, st);
+        case 4: return launch_nc<4>(a, wgs, repair, st);
+        case 5: return launch_nc<5>(a, wgs, repair, st);
+        case 6: return launch_nc<6>(a, wgs, repair, st);
+        case 7: return launch_nc<7>(a, wgs, repair, st);
+        case 8: return launch_nc<8>(a, wgs, repair, st);
         default: return hipErrorInvalidValue;
     }
 }

@@ -100,6 +100,8 @@ _SIGS = {
     "sk_loop_resident": (ctypes.c_int, [ctypes.POINTER(SkLoop)]),
     "sk_loop_repairs_offset": (ctypes.c_size_t, [ctypes.POINTER(SkLoop)]),
     "sk_loop_run_resident_f32": (ctypes.c_int, [ctypes.POINTER(SkLoop), ctypes.c_int, ctypes.c_void_p]),
+    "sk_loop_try_resident_f32": (ctypes.c_int, [ctypes.POINTER(SkLoop), ctypes.c_int, ctypes.c_void_p]),
+    "sk_loop_recover_f32": (ctypes.c_int, [ctypes.POINTER(SkLoop), ctypes.c_int, ctypes.c_void_p]),
     "sk_loop_batch_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int]),
     "sk_loop_batch_plan": (ctypes.c_int, [ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int), ctypes.c_int,
                                           ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
@@ -446,7 +448,7 @@ class DeviceLoop:
     next batch already queued behind it (no per-iteration synchronisation).
 
     On the default stream a small loop (sk_loop_resident) runs each call's iterations as one resident launch instead, bit
-    for bit the same (should it give up, they are run again on the GPU: repairs); on any other stream the caller may have
+    for bit the same (should it give up, they are run again, for enqueue on the GPU: repairs); on any other stream the caller may have
     more loops in flight, which resident launches would run one after another.
 
     With TRNOPT_HIP_GRAPH=1, whole batches of GRAPH_BATCH iterations are replayed from one captured HIP graph
@@ -527,6 +529,10 @@ class DeviceLoop:
         self._graph = g
 
     def enqueue(self, iters: int) -> None:
+        lb = lib()
+        self._enqueue(iters, lb.sk_loop_run_resident_f32 if _stream() == 0 else lb.sk_loop_run_f32)
+
+    def _enqueue(self, iters: int, run) -> None:
         iters = int(iters)
         if iters >= self.GRAPH_BATCH and self.graphs_enabled():
             self.capture()
@@ -534,7 +540,6 @@ class DeviceLoop:
                 self._graph.replay()
             iters %= self.GRAPH_BATCH
         if iters > 0:
-            run = lib().sk_loop_run_resident_f32 if _stream() == 0 else lib().sk_loop_run_f32
             _check(run(ctypes.byref(self._L), iters, _stream()), "sk_loop_run_f32")
 
     def read_state(self) -> SkState:
@@ -542,18 +547,28 @@ class DeviceLoop:
         host = self.state.to("cpu")
         return SkState.from_buffer_copy(host.numpy().tobytes())
 
+    def _recovered(self, st: SkState, queued: int) -> SkState:
+        """The state after the `queued` iterations since init, a resident launch having given up after st.it of them: the
+        rest as launches."""
+        _check(lib().sk_loop_recover_f32(ctypes.byref(self._L), queued - st.it, _stream()), "sk_loop_recover_f32")
+        return self.read_state()
+
     def repairs(self) -> int:
         """Resident launches since init that gave up, because their workgroups were not all running, and whose iterations
-        one workgroup then ran again (sk_loop.hip). Synchronises."""
+        were run again (sk_loop.hip). Synchronises."""
         at = lib().sk_loop_repairs_offset(ctypes.byref(self._L))
         return int(self.ws[at:at + 4].cpu().view(torch.int32)) if at else 0
 
     def run(self, batch: int | None = None) -> SkState:
         """Run to `done` (converged or max_iters). Returns the final state."""
         self.init()
+        lb = lib()
+        # (the state is read anyway, so a resident launch that gives up need not be made good on the GPU)
+        launch = lb.sk_loop_try_resident_f32 if _stream() == 0 else lb.sk_loop_run_f32
         if self.fixed_iters:
-            self.enqueue(self.max_iters)
-            return self.read_state()
+            self._enqueue(self.max_iters, launch)
+            st = self.read_state()
+            return self._recovered(st, self.max_iters) if st.done == 2 else st
         batch = max(1, int(batch or max(self.check_every, 10)))
         if self._pinned is None:
             self._pinned = [torch.empty(ctypes.sizeof(SkState), dtype=torch.uint8, pin_memory=True) for _ in range(2)]
@@ -563,7 +578,7 @@ class DeviceLoop:
         while True:
             if queued < self.max_iters:
                 k = min(batch, self.max_iters - queued)
-                self.enqueue(k)
+                self._enqueue(k, launch)
                 queued += k
                 buf = self._pinned[slot % 2]
                 slot += 1
@@ -576,6 +591,9 @@ class DeviceLoop:
             buf, ev = inflight.pop(0)
             ev.synchronize()
             st = SkState.from_buffer_copy(buf.numpy().tobytes())
+            if st.done == 2:
+                st, launch = self._recovered(st, queued), lb.sk_loop_run_f32
+                inflight.clear()
             if st.done:
                 return st                     # final: the launches still queued return at once, changing nothing
             if not inflight and queued >= self.max_iters:  # pragma: no cover - done must be set by then
