@@ -378,7 +378,8 @@ def check_range(max_abs: float) -> None:
 
 
 def to_device_f64(pts: np.ndarray, device) -> torch.Tensor:
-    return torch.as_tensor(np.ascontiguousarray(pts, dtype=np.float64)).to(device)
+    p = np.ascontiguousarray(pts, dtype=np.float64)
+    return torch.as_tensor(p if p.flags.writeable else p.copy()).to(device)      # (torch warns about read-only memory)
 
 
 def cloud_stats(x: torch.Tensor, y: torch.Tensor, stat: torch.Tensor, pairs=None) -> None:
