@@ -19,15 +19,15 @@
 // E follows the largest norms, so the few points far outside the others are set aside first (near_limit): they take no part
 // in 1 and 2, their pairs' float64 costs are sorted into below, inside and above the bracket one by one (far_kernel), and the
 // answer is checked to lie inside it. Without that, one point 40 times the others' norm widened the bracket past the
-// workspace: 7,355 x 8,962 d 30 with one point at 20 / 30 / 40 / 1,000 times 290 / 437 / 918 / 1,000 us, and 208 at all of
+// workspace: 7,355 x 8,962 d 30 with one point at 20 / 30 / 40 / 1,000 times 290 / 437 / 918 / 1,000 us, and 204 at all of
 // them with it.
 // When the bracket holds more pairs than the workspace (massive ties), radix-select passes over every float64 cost take
 // over (select_pass_kernel): three digits, the third also keeping the keys that still match, and the other three over
 // those keys (or over every cost again, if those are too many as well). Every launch goes on the caller's stream with no
 // host round trip.
 //
-// From the norms to the answer, all launches back to back: 7,355 x 8,962 d 30 192 us (the histogram pass 37 of them,
-// the collecting pass 50); 10,000 x 10,000 d 64 457 us; 7,000 x 7,000 d 128 276 us; 300 x 257 d 30 96 us. With three
+// From the norms to the answer, all launches back to back: 7,355 x 8,962 d 30 188 us (the histogram pass 37 of them,
+// the collecting pass 52); 10,000 x 10,000 d 64 455 us; 7,000 x 7,000 d 128 271 us; 300 x 257 d 30 94 us. With three
 // radix passes over every float64 cost (254 to 187 us each at 7,355 x 8,962, where their fma floor is 54) it was 704,
 // 1,633, 1,529 and 121 us.
 
@@ -485,9 +485,10 @@ __device__ __forceinline__ unsigned long long exact_key(const double* __restrict
 }
 
 // The pairs of the points set aside, by their float64 costs: below the bracket, inside it, or above. Every x with the far y,
-// every near y with the far x. With more of them than kFarPairs (a quarter of a millisecond at d 30) the full passes are
-// as good.
-constexpr unsigned long long kFarPairs = 1ull << 21;
+// every near y with the far x. Bound by gathering the other cloud's rows: the whole call with 2.0 / 3.3 / 7.4 / 8.2 million
+// such pairs at 7,355 x 8,962 d 30 494 / 557 / 709 / 739 us, d 128 883 / 1,077 / 1,646 / 1,761; the full passes, taken above
+// kFarPairs, 970 and 2,180.
+constexpr unsigned long long kFarPairs = 1ull << 23;
 __global__ __launch_bounds__(256) void far_kernel(const unsigned* __restrict__ far_x, const unsigned* __restrict__ far_y,
                                                   const float* __restrict__ yf, const double* __restrict__ xp,
                                                   const double* __restrict__ yp, const double* __restrict__ xx,
@@ -881,7 +882,7 @@ int sk_cost_median_f64(const double* xc, const double* yc, int n, int m, int d, 
         default: launch_approx<8>(o, w, n, m, s); break;
     }
     if (std::max(o.xblocks, o.yblocks) >= 8)          // else near_limit sets none aside
-        hipLaunchKernelGGL(far_kernel, dim3(64), dim3(256), 0, s, (const unsigned*)(w + o.farx), (const unsigned*)(w + o.fary),
+        hipLaunchKernelGGL(far_kernel, dim3(256), dim3(256), 0, s, (const unsigned*)(w + o.farx), (const unsigned*)(w + o.fary),
                            (const float*)(w + o.yf), xp, yp, xx, yy, n, m, o.dp, st, (unsigned*)(w + o.slabs), o.cap);
     hipLaunchKernelGGL(exact_kernel, dim3(1024), dim3(256), 0, s, (const unsigned*)(w + o.slabs), xp, yp, xx, yy, m, o.dp, st,
                        keys, o.cap);
