@@ -449,8 +449,9 @@ class DeviceLoop:
     next batch already queued behind it (no per-iteration synchronisation).
 
     On the default stream a small loop (sk_loop_resident) runs each call's iterations as one resident launch instead, bit
-    for bit the same (should it give up, they are run again, for enqueue on the GPU: repairs); on any other stream the caller may have
-    more loops in flight, which resident launches would run one after another.
+    for bit the same (should it give up because something else holds the CUs, they are run again: on the GPU after enqueue,
+    as launches in run; repairs counts them). On any other stream the caller may have more loops in flight, and two resident
+    launches at once would each hold CUs that the other waits for.
 
     With TRNOPT_HIP_GRAPH=1, whole batches of GRAPH_BATCH iterations are replayed from one captured HIP graph
     (20 to 40 kernels, no memset nodes): fewer host calls, for callers whose host enqueue is the bottleneck. Graph
